@@ -52,8 +52,7 @@ struct Error : std::runtime_error {
 enum Slot {
   S_PTS, S_X, S_XS, S_KEYS, S_KEYS_TMP, S_IDS, S_IDS_TMP, S_CELLKEYS, S_CELLSTART, S_FLAGS, S_POS,
   S_ACT, S_NTILES, S_TILEOFF, S_TILES, S_FAILED, S_ROWSUM, S_OUTIDS, S_OUTDISTS, S_SCRATCH,
-  S_HEAP, S_SMALL, S_PART, S_CTR, S_CSUM, S_HOSTFLAGS, S_OVERFLOW, S_STAGE, S_DENSE, S_BFLAGS,
-  S_BPOS, S_BSTART, S_CELLOF, S_CELLMAX, S_FCNT, S_RADIUS, S_RHIST, S_MODEL, S_TRAIN, S_OCC, S_ACTQ, S_BRUTE_PK, S_BRUTE_PI, S_BLIST, S_TILEMETA, S_HCPU, S_HGPU, S_HLIST, S_HROWI, S_HROWD, S_XS2, S_SIDS, S_SIDS2, S_BKEY, S_PARTNER, S_ABITS, S_NSLOTS
+  S_HEAP, S_SMALL, S_PART, S_CTR, S_CSUM, S_HOSTFLAGS, S_OVERFLOW, S_STAGE, S_DENSE, S_CELLOF, S_CELLMAX, S_FCNT, S_RADIUS, S_RHIST, S_MODEL, S_TRAIN, S_OCC, S_ACTQ, S_BRUTE_PK, S_BRUTE_PI, S_BLIST, S_TILEMETA, S_HCPU, S_HGPU, S_HLIST, S_HROWI, S_HROWD, S_XS2, S_SIDS, S_SIDS2, S_ABITS, S_NSLOTS
 };
 
 // Slots of one no-allocation call: regions of the static device scratch array handed out in
@@ -457,14 +456,6 @@ struct Pipeline {
   // 1 GiB of cell starts at most: filled and scanned once per build (~0.6 ms at 2^28 cells),
   // against a binary search of the cell table for every row of every block without it
   static constexpr uint64_t kDenseMaxCells = 1ull << 28;
-  // tiles a pass should have before the cost model widens its blocks (2816 persistent waves;
-  // KNN_MIN_TILES overrides it for tuning: 2816, 4096, 8192 and 16384 are within 1 % of each
-  // other on the 10M mixed 2-D joins, K = 16 to 128)
-  static double min_tiles() {
-    const char *v = std::getenv("KNN_MIN_TILES");
-    const double t = v ? std::atof(v) : 8192.0;
-    return t >= 1.0 ? t : 8192.0;
-  }
   const uint32_t *denseStart = nullptr;
   uint32_t *cellOf = nullptr;  // compacted cell index of each sorted position
 
@@ -477,30 +468,20 @@ struct Pipeline {
                   T *dDists, unsigned long long *ctr, Timer &tK, Timer &tPass,
                   const std::function<void()> &beforeWait = {}, const std::function<void()> &afterHeap = {});
   T uniform_radius() const { return radiusAll > (T)0 ? radiusAll : (T)g.eps; }
-  // tiles of the active queries, every count kept on the device; the tile count ends in
-  // *ntilesDev (the range kernels read it there)
-  void make_tiles(const uint8_t *activeFailed, uint32_t *&act, uint4 *&tiles, const uint32_t *&ntilesDev,
-                  uint8_t *failed, unsigned long long *cellAcc);
+  // the active queries in cell order (all, those with activeFailed[q] != 0), less the ones the
+  // own-block pre-check fails (with `failed`); their count stays on the device (activeDev)
+  void make_active(const uint8_t *activeFailed, uint32_t *&act, uint8_t *failed, unsigned long long *cellAcc);
+  // tiles of at most 64 of them per cell for the heap kernel, which scans the union of a tile's
+  // blocks; the tile count ends in *ntilesDev
+  void make_tiles(uint4 *&tiles, const uint32_t *&ntilesDev);
   unsigned long long accBytes = 0;  // accumulated pre-check accounting bytes
   const T *radius = nullptr;  // per-query radii (learned schedule), null = radiusAll
   T radiusAll = (T)0;         // one radius for every query (plain schedule); 0 = the grid's eps
-  uint32_t lastSpan = 1;
-  uint32_t lastRows = 1;
-  uint32_t selBuckets = (uint32_t)SEL_NB_OTHER;  // the select kernel's bucket count for the passes
-  uint32_t lastActive = 0;   // queries left in tiles after the pre-check
-  double avgReach = 1.0;     // typical search radius in cells (tile-span cost model)
-  // persistent range-kernel workgroups: 11 per CU on 256 CUs (the select kernel's LDS,
-  // about 14 KB per one-wave workgroup, admits 11 per CU).  The kernel is latency-bound, so
-  // residency pays: 10M mixed 2-D points, K = 64, learned / plain schedule: 2048 -> 34.7 /
-  // 60.6 ms per join, 2560 -> 31.1 / 54.9 ms, 2816 -> 30.5 / 53.6 ms; 32 buckets with up to
-  // 16 waves per CU: 30.0 / 57.5 ms (coarser buckets stage and rank more in the plain schedule).
-#ifndef KNN_PASS_GRID
-#define KNN_PASS_GRID 2816
-#endif
-  static constexpr uint32_t kPassGrid = KNN_PASS_GRID;
+  uint32_t lastRows = 1;     // rows per lookup step of the last pass
+  uint32_t lastActive = 0;   // queries left to the range kernel after the pre-check
+  static constexpr uint32_t kCollectGrid = 2816;  // persistent collect-kernel workgroups
   static constexpr uint32_t kHeapGrid = 512;   // persistent heap-kernel workgroups
-  const uint32_t *activeDev = nullptr;         // active count of the last tile build (device)
-  const uint32_t *spanDev = nullptr;           // its tile-block span (device)
+  const uint32_t *activeDev = nullptr;         // active count of the last make_active (device)
 };
 
 template <typename T>
@@ -616,23 +597,18 @@ static EpsResult estimate_eps(const T *x, uint32_t n, uint32_t d, uint32_t k, do
 }
 
 
-// Range kernel of a pass: the collect kernel (one pass over each query's own block) with 5 or
-// more indexed dims, else the two-pass select kernel, whose first pass reads each candidate
-// once for all queries of a tile.  Measured on MI355X, 5M points, K = 32 (learned / plain
-// schedule, ms): 6 indexed dims, uniform 225 / 264 against 317 / 302, skewed 339 / 409
-// against 567 / 582; 4 indexed dims, uniform 63 / 98 against 59 / 66; 2 of 4 dims indexed
-// 2475 against 1504 (learned): queries share most of their candidates with the rest of their
-// tile there.  KNN_RANGE_KERNEL=select|collect overrides the choice for tuning.
-static bool use_collect(uint32_t nd, uint32_t k1) {
+// Range kernel of a pass: the direct kernel up to K+1 = DR_MAX_K1, above it the collect kernel
+// (LDS top-(K+1) collector, up to BRUTE_MAX_K1), then the heap kernel.
+// KNN_RANGE_KERNEL=collect takes the collect kernel for the small K+1 too, for the tests.
+enum RangeKernel { RK_DIRECT, RK_COLLECT, RK_HEAP };
+static RangeKernel range_kernel(uint32_t k1) {
   const char *v = std::getenv("KNN_RANGE_KERNEL");  // read per pass: tests switch it in-process
-  const int env = !v ? -1 : (std::strcmp(v, "collect") == 0 ? 1 : (std::strcmp(v, "select") == 0 ? 0 : -1));
-  if (k1 > BRUTE_MAX_K1) return false;
-  return env >= 0 ? env == 1 : nd >= 5;
+  if (k1 > BRUTE_MAX_K1) return RK_HEAP;
+  return k1 > DR_MAX_K1 || (v && std::strcmp(v, "collect") == 0) ? RK_COLLECT : RK_DIRECT;
 }
 
-// Kernel for the queries the select kernel cannot stage (staging overflow, or K+1 beyond its
-// LDS slots): the collect kernel (wave = query, LDS collector) up to K+1 = BRUTE_MAX_K1, the
-// per-lane heap kernel above.  KNN_OVERFLOW_KERNEL=heap|collect overrides it for tuning.
+// Kernel for the queries the direct kernel cannot list (thousands of equal keys): the collect
+// kernel; KNN_OVERFLOW_KERNEL=heap takes the heap kernel, for the tests.
 static bool overflow_by_collect(uint32_t k1) {
   const char *v = std::getenv("KNN_OVERFLOW_KERNEL");
   if (k1 > BRUTE_MAX_K1) return false;
@@ -659,27 +635,11 @@ static uint64_t reuse_tail_div() {
   return c >= 1 ? (uint64_t)c : 64u;
 }
 
-// Rows of a tile block with 2 indexed dims: up to 2 (k_choose_span picks 1 or 2 per pass from
-// the active density); KNN_TILE_ROWS=1 keeps single-row blocks, for tuning.  Measured on one
-// MI355X (ms per join, single rows against row pairs, same rows out): 10M mixed 2-D points,
-// K=64, plain 34.90 / 32.45, learned 20.00 / 20.01 (K=16 16.69 / 16.59, K=128 30.10 / 30.28);
-// with 4 indexed dims (5M uniform 4-D, K=32, plain) 25.8 / 26.2 with 15 % more candidates, as
-// the rows' chords narrow less for a union of two rows: above 2 indexed dims blocks keep one.
-static uint32_t tile_rows_max() {
-  const char *v = std::getenv("KNN_TILE_ROWS");  // read per pass: tuning runs switch it in-process
-  return (v && std::atoi(v) == 1) ? 1u : 2u;
-}
-
-// Density basis of the tile-block cost model: active queries per cell holding any (default),
-// or KNN_SPAN_DENSITY=cells for active queries per non-empty cell, for tuning.  Clustered
-// active queries fill a block's 64 query slots over fewer cells than the average over all
-// non-empty cells says, and further tiles of the block rescan the same union.  Measured on one
-// MI355X with row pairs (ms per join, per non-empty cell against per active cell, same rows
-// out): 10M mixed 2-D points, learned K=16 16.90 / 15.55, K=64 20.22 / 19.92, K=128 30.50 /
-// 29.89, plain K=64 32.54 / 32.07; 5M points, K=32, 3 and 4 indexed dims: equal candidates.
-static bool span_by_active_cells() {
-  const char *v = std::getenv("KNN_SPAN_DENSITY");  // read per pass: tuning runs switch it in-process
-  return !(v && std::strcmp(v, "cells") == 0);
+// Rows of a query's block looked up per step of the direct kernel's chunk set-up with 2 indexed
+// dims: 2 (their table reads are in flight together); KNN_TILE_ROWS=1 looks up one, for tuning.
+static uint32_t lookup_rows(uint32_t nd) {
+  const char *v = std::getenv("KNN_TILE_ROWS");  // read per pass: tests switch it in-process
+  return nd == 2 && !(v && std::atoi(v) == 1) ? 2u : 1u;
 }
 
 // Replica grids of the learned features' point counts: up to 16, within 2^24 counters in all
@@ -709,14 +669,9 @@ static uint32_t tile_ranges(uint32_t d, bool batched) {
   return (d >= 3 && !batched) ? TILE_QUEUES : 1u;
 }
 
-// Builds tiles of <= 64 active queries per tile block: activeFailed[q] != 0 selects q (all
-// when null); act/tiles point into the cache, the tile count is left in device memory.
-// Tile blocks are windows of `span` cells along dim 0 within one row; the span is chosen on the
-// device from the active count (k_choose_span: wide windows pay only when active queries are
-// dense, and a pass with few tiles ends with its slowest ones).
 template <typename T>
-void Pipeline<T>::make_tiles(const uint8_t *activeFailed, uint32_t *&act, uint4 *&tiles,
-                             const uint32_t *&ntilesDev, uint8_t *failed, unsigned long long *cellAcc) {
+void Pipeline<T>::make_active(const uint8_t *activeFailed, uint32_t *&act, uint8_t *failed,
+                              unsigned long long *cellAcc) {
   uint32_t *flags = buf<uint32_t>(S_FLAGS, n + 1);
   uint32_t *pos = buf<uint32_t>(S_POS, n + 1);
   bool all = !activeFailed;
@@ -744,26 +699,18 @@ void Pipeline<T>::make_tiles(const uint8_t *activeFailed, uint32_t *&act, uint4 
     compact_active(sortedIds, flags, pos, n, act, s);
   }
   activeDev = pos + n;
-  uint32_t *meta = buf<uint32_t>(S_TILEMETA, 16);
-  const uint32_t spanMax = nd == 1 ? 4096u : (nd == 2 ? 256u : 8u);
-  // the pre-check's count of cells holding active queries (cellAcc[1]) as the density basis
-  const unsigned long long *activeCells = (cellAcc && span_by_active_cells()) ? cellAcc + 1 : nullptr;
-  choose_span(activeDev, activeCells, ncell, avgReach, spanMax, nd == 2 ? tile_rows_max() : 1u, min_tiles(), meta, s);
-  spanDev = meta;
-  uint32_t *bflags = buf<uint32_t>(S_BFLAGS, (size_t)ncell + 1);
-  uint32_t *bpos = buf<uint32_t>(S_BPOS, (size_t)ncell + 1);
-  uint32_t *bstart = buf<uint32_t>(S_BSTART, (size_t)ncell + 1);
-  uint64_t *bkey = buf<uint64_t>(S_BKEY, (size_t)ncell + 1);
-  uint32_t *partner = buf<uint32_t>(S_PARTNER, (size_t)ncell + 1);
-  block_flags_dev(cellKeys, ncell, g.nCells[0], meta, bflags, s);
-  scan_exclusive_u32(bflags, bpos, ncell, scratch, s);
-  compact_blocks_keyed(cellKeys, cellStart, bflags, bpos, ncell, g.nCells[0], meta, n, bstart, bkey, s);
-  uint32_t *ntiles = buf<uint32_t>(S_NTILES, (size_t)ncell + 1);
-  uint32_t *tileOff = buf<uint32_t>(S_TILEOFF, (size_t)ncell + 1);
+}
+
+template <typename T>
+void Pipeline<T>::make_tiles(uint4 *&tiles, const uint32_t *&ntilesDev) {
+  const uint32_t *pos = buf<uint32_t>(S_POS, n + 1);
+  uint32_t *ntiles = buf<uint32_t>(S_NTILES, (size_t)n + 2);
+  uint32_t *tileOff = buf<uint32_t>(S_TILEOFF, (size_t)n + 3);
   tiles = buf<uint4>(S_TILES, n);
-  pair_tiles_dev(bstart, bkey, pos, bpos + ncell, ncell, g.nCells[0], nd >= 2 ? g.nCells[1] : 1u, meta, partner,
-                 ntiles, tileOff, scratch, tiles, s);
-  ntilesDev = tileOff + ncell;
+  uint32_t *nc = buf<uint32_t>(S_TILEMETA, 16);  // (the build's own device count is overwritten by now)
+  fill_u32(nc, ncell, 1, s);
+  batch_tiles(cellStart, pos, nc, n, 64u, ntiles, tileOff, scratch, tiles, s);
+  ntilesDev = tileOff + n + 1;
 }
 
 template <typename T>
@@ -777,11 +724,9 @@ PassResult Pipeline<T>::pass(const uint8_t *activeFailed, uint32_t nq, uint8_t *
   uint32_t *overflowCount = counters + 1;
   uint32_t *tileCounter = reinterpret_cast<uint32_t *>(ctr + 16);
   uint32_t *act;
-  uint4 *tiles;
-  const uint32_t *ntDev;
   tPass.start();
   fill_u32(reinterpret_cast<uint32_t *>(ctr + 4), 0u, 4, s);
-  make_tiles(activeFailed, act, tiles, ntDev, failed, ctr + 4);
+  make_active(activeFailed, act, failed, ctr + 4);
   uint8_t *overflow = buf<uint8_t>(S_OVERFLOW, n);
   fill_u8(overflow, 0, n, s);
   fill_u32(counters, 0u, 4, s);
@@ -796,9 +741,7 @@ PassResult Pipeline<T>::pass(const uint8_t *activeFailed, uint32_t nq, uint8_t *
   a.ncell = ncell;
   a.denseStart = denseStart;
   a.act = act;
-  a.tiles = tiles;
-  a.ntiles = kPassGrid;  // persistent grid; the tile count is read from ntilesDev
-  a.ntilesDev = ntDev;
+  a.activeCount = activeDev;
   a.n = n;
   a.d = d;
   a.k1 = K1;
@@ -812,32 +755,28 @@ PassResult Pipeline<T>::pass(const uint8_t *activeFailed, uint32_t nq, uint8_t *
   a.tileCounter = tileCounter;
   a.tileRanges = tile_ranges(d, false);
   a.segCapLog2 = seg_cap_log2();
-  // LDS staging slots per query: K+1 and 64 more (the items of the K+1-th neighbour's
-  // bucket beyond K+1), at most 512, within the 64 KB a workgroup may allocate
-  a.selBuckets = selBuckets;
-  a.smax = std::min<uint32_t>(K1 + 64, 512u);
-  while (a.smax > K1 && range_select_lds_bytes<T>(a.smax, selBuckets) > 65536) a.smax -= 16;
+  a.lookupRows = lastRows = lookup_rows(nd);
   a.overflow = overflow;
   a.overflowCount = overflowCount;
   PassResult r{};
-  bool selectK = false;
+  auto heap = [&]() {
+    uint4 *tiles;
+    make_tiles(tiles, a.ntilesDev);
+    a.tiles = tiles;
+    a.ntiles = kHeapGrid;
+    const size_t hs = range_heap_scratch_bytes<T>(kHeapGrid, K1);
+    a.heapScratch = hs ? g_cache.get(S_HEAP, hs) : nullptr;
+    range_topk<T>(a, g, s);
+  };
+  const RangeKernel rk = range_kernel(K1);
   tK.start();
-  if (use_collect(nd, K1)) {
+  if (rk == RK_DIRECT) {
+    range_direct<T>(a, g, s);
+  } else if (rk == RK_COLLECT) {
+    a.ntiles = kCollectGrid;
     range_collect<T>(a, g, s);
-  } else if (!(a.smax > K1 && range_select_lds_bytes<T>(a.smax, selBuckets) <= 65536)) {
-    // K+1 too large for LDS staging: the collect (or heap) kernel takes every query of the pass
-    if (overflow_by_collect(K1)) {
-      range_collect<T>(a, g, s);
-    } else {
-      a.ntiles = kHeapGrid;
-      size_t hs = range_heap_scratch_bytes<T>(kHeapGrid, K1);
-      a.heapScratch = hs ? g_cache.get(S_HEAP, hs) : nullptr;
-      range_topk<T>(a, g, s);
-    }
   } else {
-    a.ntiles = sel_pass_grid(selBuckets);  // persistent grid: the workgroups its LDS admits
-    range_select<T>(a, g, s);
-    selectK = true;
+    heap();
   }
   LAUNCH_CHECK();
   tK.stop_async();
@@ -846,7 +785,6 @@ PassResult Pipeline<T>::pass(const uint8_t *activeFailed, uint32_t nq, uint8_t *
   auto readback = [&]() {
     HIP_CHECK(hipMemcpyAsync(pin + PW_KFAIL, counters, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipMemcpyAsync(pin + PW_ACTIVE, activeDev, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(pin + PW_SPAN, spanDev, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipMemcpyAsync(pin + PW_CTR, ctr, 6 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
   };
   if (beforeWait) beforeWait();
@@ -855,32 +793,22 @@ PassResult Pipeline<T>::pass(const uint8_t *activeFailed, uint32_t nq, uint8_t *
   sync();
   r.kernel_ms = tK.elapsed();
   lastActive = pin[PW_ACTIVE];
-  lastSpan = pin[PW_SPAN];
-  lastRows = pin[PW_SPAN + 1];
-  r.noverflow = selectK ? pin[PW_OVF] : 0u;
+  r.noverflow = rk == RK_DIRECT ? pin[PW_OVF] : 0u;
   if (r.noverflow) {
-    // queries whose candidates overflow the staging slots: the collect (or heap) kernel
-    uint32_t *act2;
-    uint4 *tiles2;
-    const uint32_t *nt2;
+    // queries whose candidates overflow the direct kernel's lists: the collect (or heap) kernel
     const uint32_t A1 = lastActive;
-    make_tiles(overflow, act2, tiles2, nt2, nullptr, nullptr);
+    make_active(overflow, act, nullptr, nullptr);
     fill_u32(tileCounter, 0u, TILE_QUEUES, s);
-    a.act = act2;
-    a.tiles = tiles2;
-    a.ntilesDev = nt2;
-    const bool byCollect = overflow_by_collect(K1);
-    a.ntiles = byCollect ? kPassGrid : kHeapGrid;
-    if (!byCollect) {
-      size_t hs = range_heap_scratch_bytes<T>(kHeapGrid, K1);
-      a.heapScratch = hs ? g_cache.get(S_HEAP, hs) : nullptr;
-    }
+    a.act = act;
+    a.activeCount = activeDev;
     Timer tH(s, 5);
     tH.start();
-    if (byCollect)
+    if (overflow_by_collect(K1)) {
+      a.ntiles = kCollectGrid;
       range_collect<T>(a, g, s);
-    else
-      range_topk<T>(a, g, s);
+    } else {
+      heap();
+    }
     LAUNCH_CHECK();
     tH.stop_async();
     if (afterHeap) afterHeap();
@@ -1154,16 +1082,25 @@ static double env_knob(const char *name, double lo, double hi) {
   const double x = v ? std::atof(v) : 0.0;
   return (x >= lo && x <= hi) ? x : 0.0;
 }
-// Measured on MI355X (plain schedule, 2 indexed dims): cells of width eps kept until eps
-// doubles, against a re-index at every growth: 10M mixed points 85.4 / 98.1 ms at K = 64 and
-// 83.0 / 97.7 ms at K = 16, 10M uniform 47.2 / 48.1 ms, 1M mixed K = 8 17.8 / 18.7 ms.
-static double plain_grid_div(uint32_t) {
+// Measured on MI355X (plain schedule, direct kernel, ms per join).  Up to 2 indexed dims, every
+// dim indexed, cells of eps kept until eps doubles against cells of eps / 2.5: a query's rows fit
+// its ball closer, which pays from about K+1 = 12 on (10M mixed K=64 28.1 / 20.8, 10M uniform
+// K=16 8.60 / 7.81, 3M mixed K=128 16.2 / 13.3) and costs more index than it saves below (100k
+// uniform K=8 0.89 / 0.98, 1M mixed K=8 5.4 / 5.9).  Above 2 indexed dims cells of eps until eps
+// has grown by half, against a re-index at every growth: 3M skewed 4-D K=16 27.8 / 24.3, 500k
+// skewed 6-D K=32 31.0 / 26.1, finer cells multiply the rows (500k 6-D at eps / 1.5: 28.7).
+// Projected grids of up to 2 indexed dims, eps / 1.5: 500k skewed 4-D K=16 22.7 / 18.7.
+static double plain_grid_div(uint32_t d, uint32_t nd, uint32_t k1) {
   const double e = env_knob("KNN_PLAIN_GRID_DIV", 1.0, 8.0);
-  return e > 0.0 ? e : 1.0;
+  if (e > 0.0) return e;
+  if (nd > 2) return 1.0;
+  return nd < d ? 1.5 : (k1 >= 12 ? 2.5 : 1.0);
 }
-static double plain_max_reach(uint32_t nd) {
+static double plain_max_reach(uint32_t d, uint32_t nd, uint32_t k1) {
   const double e = env_knob("KNN_PLAIN_MAX_REACH", 1.0, 8.0);
-  return e > 0.0 ? e : (nd <= 2 ? 2.0 : 1.0);
+  if (e > 0.0) return e;
+  if (nd > 2) return 1.5;
+  return nd < d ? 2.0 : (k1 >= 12 ? 5.0 : 2.0);
 }
 
 // ------------------------------------------------------------------ hybrid split
@@ -1348,11 +1285,11 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
   stats.eps0 = (float)eps0;
 
   // ---- the join loop (main.cu:305-430)
-  const double pdiv = plain_grid_div(nd), preach = plain_max_reach(nd);
+  const double pdiv = plain_grid_div(d, nd, K1), preach = plain_max_reach(d, nd, K1);
   T curW = (T)0;
   auto build = [&](T e) -> double {
     T w = (T)((double)e / pdiv);
-    if (pdiv > 1.0) {  // a finer grid only while it keeps the dense start table
+    if (pdiv > 1.0) {  // a finer grid only while its dense start table stays small beside the points
       typename GridOf<T>::type gt;
       uint64_t tc = 0;
       bool ok = w > (T)0;
@@ -1361,7 +1298,7 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
       } catch (const Error &) {
         ok = false;
       }
-      if (!ok || tc + 1 > Pipeline<T>::kDenseMaxCells) w = e;
+      if (!ok || tc > std::min<uint64_t>(Pipeline<T>::kDenseMaxCells - 1, 16ull * n + (1u << 20))) w = e;
     }
     P.tBuild = &tPh;
     tPh.start();
@@ -1411,7 +1348,6 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
       }
     }
     P.radiusAll = eps;
-    P.avgReach = (double)eps / (double)curW;
     PassResult pr = P.pass(first ? H.gpuActive : failed, nq, failed, dIds, dDists, ctr, tK, tPh);
     launches++;
     stats.overflow_queries += pr.noverflow;
@@ -1424,8 +1360,8 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
     const uint32_t nfail = pr.nfail;
     joinMs += pr.pass_ms;
     if (P.verbose)
-      printf("[knn] iter %u eps %.9g queries %u failed %u cells %u span %u rows %u overflow %u candidates %llu kernel %.3f ms\n",
-             numIter, (double)eps, nq, nfail, P.ncell, P.lastSpan, P.lastRows, pr.noverflow,
+      printf("[knn] iter %u eps %.9g queries %u failed %u cells %u rows %u overflow %u candidates %llu kernel %.3f ms\n",
+             numIter, (double)eps, nq, nfail, P.ncell, P.lastRows, pr.noverflow,
              (unsigned long long)(pr.pairs - pairs), pr.kernel_ms);
     pairs = pr.pairs;
     frac = (nfail * 1.0) / (nq * 1.0);  // main.cu:402
@@ -1459,44 +1395,31 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
   stats.kernel_launches = launches;
 }
 
-// Cells per radius-class upper bound R in the learned schedule's grids: with <= 2 indexed
-// dims 3 up to K+1 = 80 and 4 above (with the wider classes below), 1 with more indexed dims,
-// 4 on a projected grid (fewer indexed than data dims; see learned_class_bins);
-// KNN_LEARNED_GRID_DIV (1..8) overrides it for tuning.
+// Cells per radius-class upper bound R in the learned schedule's grids, and quarter-octave bins
+// per radius class (each class costs an index build over all N points, a wide class larger blocks
+// for its small radii).  Measured on MI355X with the direct kernel (ms per join, cells / bins):
+//   2-D  K=64 10M mixed:  R/3, 8 16.3;  R/4, 8 16.1;  R/3, 10 14.3;  R/4, 10 14.8;  R/5, 10 14.6
+//        K=16 10M mixed:  R/3, 8 12.0;  R/3, 10 12.0;  R/5, 10 12.4;  R/4, 8 17.6
+//        K=100 1.3M / K=128 3M mixed:  R/4, 10 6.03 / 9.89;  R/5, 10 5.81 / 8.95;  R/4, 12 6.57 / 10.1
+//   4-D  5M skewed K=32 / 300k skewed K=32 / 3M uniform K=16:  R, 2 26.8 / 9.9 / 8.4;
+//        R/1.25, 4 22.1 / 6.6 / 8.8;  R/1.5, 5 22.3 / 6.3 / 8.8;  R/1.75, 6 23.5 / 6.1 / 8.8
+//   6-D  2M skewed / 2M uniform K=32 / 200k skewed K=16:  R, 2 52.9 / 27.2 / 8.9;
+//        R/1.15, 2 40.2 / 27.2 / 9.8;  R/1.25, 3 39.1 / 25.8 / 8.7
+//   projected grids (fewer indexed than data dims), 6 bins:  1M 6-D on 4 dims, skewed K=32,
+//        R/2 78.2, R/3 62.3, R/4 73.8;  1M 4-D on 2 dims, skewed K=32, R/3 40.4, R/4 36.7, R/5 34.4
+// KNN_LEARNED_GRID_DIV (1..8) and KNN_LEARNED_CLASS_BINS (1..16) override them for tuning.
 static double learned_grid_div(uint32_t d, uint32_t nd, uint32_t k1) {
-  static const double env = []() {
-    const char *v = std::getenv("KNN_LEARNED_GRID_DIV");
-    const double x = v ? std::atof(v) : 0.0;
-    return (x >= 1.0 && x <= 8.0) ? x : 0.0;
-  }();
-  if (env > 0.0) return env;
-  if (nd < d) return 4.0;
-  return nd <= 2 ? (k1 <= 80 ? 3.0 : 4.0) : 1.0;
+  const double e = env_knob("KNN_LEARNED_GRID_DIV", 1.0, 8.0);
+  if (e > 0.0) return e;
+  if (nd < d) return nd <= 2 ? 4.0 : 3.0;
+  if (nd <= 2) return k1 <= 40 ? 3.0 : 5.0;
+  return nd <= 4 ? 1.5 : 1.25;
 }
-
-// Quarter-octave bins per radius class with <= 2 indexed dims: 8 (two octaves) up to
-// K+1 = 80, 10 above; 2 with more indexed dims.  Measured on MI355X, 10M mixed 2-D points
-// (ms per join, classes of 8 bins on cells of R/3 against 10 bins on cells of R/4): K = 16
-// 28.9 / 28.2, K = 32 30.4 / 30.2, K = 64 39.4 / 40.4, K = 96 56.0 / 50.2, K = 128 66.5 /
-// 59.7, K = 256 128.1 / 117.6.  Two-octave classes on cells of R/3 beat one-octave classes
-// on cells of R/2 everywhere (K = 64: 41.2 against 47.3 ms), since each class costs an index
-// build over all N points.  On a projected grid (fewer indexed than data dims) 6 bins on
-// cells of R/4; measured on 5M points, K = 32, learned ms (bins / cells: default of the
-// indexed dims, 4 / R/3, 6 / R/4): 4-D with 2 indexed, uniform 126 / 90 / 87, skewed
-// 202 / 213 / 191; 6-D with 4 indexed, uniform 270 / 204 / 202, skewed 1819 / 505 / 537.
-// With 3 or more dims, every one indexed: 2 bins on cells of R (1 / 2 / 3 bins, ms: 4-D
-// uniform 32.2 / 31.5 / 34.4, skewed 52.8 / 49.5 / 48.2; 6-D uniform 97.9 / 97.3 / 118, skewed
-// 146 / 144 / 209; 4 bins on cells of R/3: 4-D uniform 84.5).  KNN_LEARNED_CLASS_BINS (1..16)
-// overrides it for tuning.
-static int learned_class_bins(uint32_t d, uint32_t nd, uint32_t k1) {
-  static const int env = []() {
-    const char *v = std::getenv("KNN_LEARNED_CLASS_BINS");
-    const int x = v ? std::atoi(v) : 0;
-    return (x >= 1 && x <= 16) ? x : 0;
-  }();
-  if (env > 0) return env;
+static int learned_class_bins(uint32_t d, uint32_t nd) {
+  const int e = (int)env_knob("KNN_LEARNED_CLASS_BINS", 1.0, 16.0);
+  if (e > 0) return e;
   if (nd < d) return 6;
-  return nd <= 2 ? (k1 <= 80 ? 8 : 10) : 2;
+  return nd <= 2 ? 10 : (nd <= 4 ? 5 : 3);
 }
 
 // The learned schedule: per-query initial radius from the MLP, then passes over radius
@@ -1511,7 +1434,6 @@ static void run_learned(Pipeline<T> &P, const knnjoin_params &p, knnjoin_stats &
   const uint32_t n = P.n, nd = P.nd, K1 = P.K1;
   const RadiusModel &M = radius_model(P.d, nd);
   if (!M.ok) throw Error(KNN_ERR_MODEL, "no learned-radius model registered for this number of indexed dims");
-  P.selBuckets = (uint32_t)SEL_NB_LEARNED;
   // min/max of the indexed dims
   T hmn[KNN_MAX_INDEXED], hmx[KNN_MAX_INDEXED];
   P.index_minmax(hmn, hmx);
@@ -1587,7 +1509,7 @@ static void run_learned(Pipeline<T> &P, const knnjoin_params &p, knnjoin_stats &
     }
     // wide classes with <= 2 indexed dims and on projected grids; half an octave above, where a
     // cell up to 2x the radius would cost up to 2^nd in block volume
-    const int cHi = std::min(c + learned_class_bins(P.d, nd, P.K1) - 1, 63);
+    const int cHi = std::min(c + learned_class_bins(P.d, nd) - 1, 63);
     uint32_t nq = 0;
     for (int b = c; b <= cHi; b++) nq += h[b];
     double R;
@@ -1648,9 +1570,6 @@ static void run_learned(Pipeline<T> &P, const knnjoin_params &p, knnjoin_stats &
       curW = w;
       if (stats.eps0 == 0.0f) stats.eps0 = (float)w;
     }
-    // typical reach in cells (tile-span cost model): 1.5 on the class's own grid, the half
-    // radius in cells on a kept one
-    P.avgReach = reuse ? std::max(1.5, 0.5 * R / (double)curW) : 1.5;
     radius_class_flags(radius, failed, n, wfF, (uint32_t)c, (uint32_t)cHi, act, s);
     // growth on failure: one class (an octave; a quarter octave with >= 3 indexed dims), then
     // the next histogram, both before the pass's wait; after a heap-kernel pass (overflowing
@@ -1671,8 +1590,8 @@ static void run_learned(Pipeline<T> &P, const knnjoin_params &p, knnjoin_stats &
     prevBytes = pr.bytes_total;
     joinMs += pr.pass_ms;
     if (P.verbose)
-      printf("[knn] learned pass %u octave %d grid %.9g queries %u failed %u cells %u span %u rows %u overflow %u candidates %llu kernel %.3f ms\n",
-             passes, c, (double)P.g.eps, nq, pr.nfail, P.ncell, P.lastSpan, P.lastRows, pr.noverflow,
+      printf("[knn] learned pass %u octave %d grid %.9g queries %u failed %u cells %u rows %u overflow %u candidates %llu kernel %.3f ms\n",
+             passes, c, (double)P.g.eps, nq, pr.nfail, P.ncell, P.lastRows, pr.noverflow,
              (unsigned long long)(pr.pairs - pairs), pr.kernel_ms);
     pairs = pr.pairs;
     passes++;
@@ -2248,7 +2167,7 @@ int knnjoin_mlp_train(float *weights, const float *X, const float *Y, uint32_t n
 namespace knn {
 
 struct BatchGroup {
-  uint32_t d = 0, nsets = 0, N = 0, k1max = 0, smax = 0;
+  uint32_t d = 0, nsets = 0, N = 0, k1max = 0;
   uint64_t outElems = 0, bound = 0;
   int bits = 0;
   std::vector<uint32_t> members;  // caller set indices
@@ -2371,7 +2290,6 @@ static void batch_build(BatchPlan &B, uint32_t nsets, const uint32_t *n, const u
     G.bound = std::min<uint64_t>(1ull << 27, std::max<uint64_t>(1ull << 16, 8ull * N));
     G.bits = 1;
     while ((1ull << G.bits) < G.bound) G.bits++;
-    G.smax = std::min<uint32_t>(2 * G.k1max + 32, 512);
     const size_t sw = std::max({scan_scratch_words((uint32_t)G.bound + 1), scan_scratch_words(N + 2),
                                 radix_scratch_words(N)}) + 1024;
     G.xin = B.alloc<float>((size_t)N * d);
@@ -2446,8 +2364,8 @@ static JoinArgs batch_args(const BatchPlan &B, const BatchGroup &G) {
   a.tileCounter = G.ctr + 8;
   a.tileRanges = tile_ranges(G.d, true);
   a.segCapLog2 = seg_cap_log2();
+  a.lookupRows = lookup_rows(G.hsets.empty() ? 0u : G.hsets[0].nd);
   a.heapScratch = G.heap;
-  a.smax = G.smax;
   a.overflow = G.overflow;
   a.overflowCount = G.ctr + 2;
   a.sets = G.sets;
@@ -2473,8 +2391,7 @@ static void batch_index(BatchGroup &G, hipStream_t s) {
 }
 
 // One radius pass of a group: every set's lowest pending octave, grids matched to it, tiles of
-// those queries, the select kernel (the collect kernel with 5+ indexed dims), the heap kernel
-// for staging overflows, and radius growth of the queries that failed; G.ctr[3] = queries
+// those queries, the direct kernel, the collect kernel for its overflows, and radius growth of the queries that failed; G.ctr[3] = queries
 // still pending.
 static void batch_pass(const BatchPlan &B, BatchGroup &G, hipStream_t s) {
   const uint32_t N = G.N;
@@ -2491,10 +2408,13 @@ static void batch_pass(const BatchPlan &B, BatchGroup &G, hipStream_t s) {
   compact_active(G.ids, G.aflags, G.apos, N, G.act, s);
   batch_tiles(G.cellStart, G.apos, G.cpos + N, N, B.tq, G.ntiles, G.tileOff, G.scratch, G.tiles, s);
   fill_u32(G.ctr, 0u, 8 + TILE_QUEUES, s);
-  if (use_collect(G.hsets.empty() ? 0u : G.hsets[0].nd, G.k1max))
+  const RangeKernel rk = range_kernel(G.k1max);
+  if (rk == RK_DIRECT)
+    range_direct<float>(a, g0, s);
+  else if (rk == RK_COLLECT)
     range_collect<float>(a, g0, s);
   else
-    range_select<float>(a, g0, s);
+    range_topk<float>(a, g0, s);
 
   batch_flags_u8(G.ids, G.overflow, N, G.aflags, s);
   scan_exclusive_u32(G.aflags, G.apos, N, G.scratch, s);

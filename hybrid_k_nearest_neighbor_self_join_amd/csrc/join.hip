@@ -74,18 +74,6 @@ __global__ void k_gather_rows(const T *__restrict__ in, const uint32_t *__restri
   for (uint32_t j = 0; j < d; j++) xs[(size_t)j * n + p] = row[perm.v[j]];
 }
 
-__global__ void k_dense_counts(const uint64_t *cellKeys, const uint32_t *cellStart,
-                               uint32_t ncell, uint32_t *dense) {
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncell) return;
-  dense[cellKeys[c]] = cellStart[c + 1] - cellStart[c];
-}
-
-__device__ __forceinline__ uint64_t block_key(uint64_t id, uint32_t ncell0, uint32_t span) {
-  const uint64_t nb0 = (ncell0 + span - 1) / span;
-  return (id / ncell0) * nb0 + (id % ncell0) / span;
-}
-
 // bits[w] bit l = (src[64 w + l] != 0), for the ids below n (the last word's bits past n are 0)
 __global__ void k_pack_bits(const uint8_t *__restrict__ src, uint32_t n, uint64_t *__restrict__ bits) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -220,138 +208,6 @@ __global__ void k_compact_active(const uint32_t *sortedIds, const uint32_t *flag
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
   if (flags[p]) act[pos[p]] = sortedIds[p];
-}
-
-// Tile-block shape of a pass from the active count A = *activeCount (read on the device): a
-// tile of `rows` rows (1, or 2 when rowsMax = 2) scans the union of its lanes' blocks, about
-// (span + 2 reach) x (rows + 2 reach) cells, for min(64, span * rows * rho) queries (rho =
-// active queries per cell holding any, *activeCells when given, else per non-empty cell), so
-// the cost per query is about that area over the query count; a pass with fewer than minTiles
-// tiles leaves the persistent waves idle at its end, which costs in proportion.  shape[0] =
-// span, shape[1] = rows.
-__global__ void k_choose_span(const uint32_t *activeCount, const unsigned long long *activeCells,
-                              uint32_t ncell, double avgReach, uint32_t spanMax, uint32_t rowsMax,
-                              double minTiles, uint32_t *shape) {
-  if (threadIdx.x || blockIdx.x) return;
-  const uint32_t A = *activeCount;
-  uint32_t best = 1, bestRows = 1;
-  if (A && ncell) {
-    const unsigned long long ac = activeCells ? *activeCells : 0ull;
-    const double rhoA = (double)A / (ac ? (double)ac : (double)ncell);
-    double bc = 1e300;
-    for (uint32_t rows = 1; rows <= rowsMax; rows++) {
-      for (uint32_t w = 1; w <= spanMax; w *= 2) {
-        const double q = fmax(1.0, fmin(64.0, w * rows * rhoA));
-        const double tilesEst = (double)A / q;
-        const double cost = (w + 2.0 * avgReach) * (rows + 2.0 * avgReach) / q * fmax(1.0, minTiles / tilesEst);
-        if (cost < bc * 0.97) {
-          bc = cost;
-          best = w;
-          bestRows = rows;
-        }
-      }
-    }
-  }
-  shape[0] = best;
-  shape[1] = bestRows;
-}
-
-__global__ void k_block_flags_dev(const uint64_t *cellKeys, uint32_t ncell, uint32_t ncell0,
-                                  const uint32_t *span, uint32_t *flags) {
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncell) return;
-  const uint32_t w = *span;
-  flags[c] = (c == 0 || block_key(cellKeys[c], ncell0, w) != block_key(cellKeys[c - 1], ncell0, w)) ? 1u : 0u;
-}
-
-__global__ void k_compact_blocks_keyed(const uint64_t *cellKeys, const uint32_t *cellStart,
-                                       const uint32_t *flags, const uint32_t *pos, uint32_t ncell,
-                                       uint32_t ncell0, const uint32_t *shape, uint32_t n,
-                                       uint32_t *blockStart, uint64_t *blockKey) {
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncell) return;
-  if (flags[c]) {
-    blockStart[pos[c]] = cellStart[c];
-    blockKey[pos[c]] = block_key(cellKeys[c], ncell0, shape[0]);
-  }
-  if (c == ncell - 1) blockStart[pos[ncell]] = n;
-}
-
-constexpr uint32_t NO_PARTNER = 0xffffffffu;
-
-// first index in [lo, hi) of the increasing keys with keys[i] >= v
-__device__ __forceinline__ uint32_t lower_bound_keys(const uint64_t *keys, uint32_t lo, uint32_t hi, uint64_t v) {
-  while (lo < hi) {
-    const uint32_t mid = lo + ((hi - lo) >> 1);
-    if (keys[mid] < v) lo = mid + 1; else hi = mid;
-  }
-  return lo;
-}
-
-// per tile block b < *nblocks (0 for b up to ncell): tiles of <= 64 active queries.  With row
-// pairs (shape[1] = 2) a block of an even dim-1 coordinate takes its partner's queries (the
-// block one row up, same window; partner[b]), and a block whose partner one row down exists
-// has no tiles of its own.  Block keys are distinct and increase with b, so the partner of key
-// +- nw (nw = windows per row) lies within nw places of b: one binary search over those.
-__global__ void k_pair_tile_counts(const uint32_t *blockStart, const uint64_t *blockKey, const uint32_t *pos,
-                                   const uint32_t *nblocks, uint32_t ncell, uint32_t ncell0, uint32_t ncell1,
-                                   const uint32_t *shape, uint32_t *partner, uint32_t *ntiles) {
-  const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= ncell) return;
-  const uint32_t nb = *nblocks;
-  if (b >= nb) {
-    ntiles[b] = 0;
-    return;
-  }
-  uint32_t cnt = pos[blockStart[b + 1]] - pos[blockStart[b]];
-  uint32_t pj = NO_PARTNER;
-  if (shape[1] == 2u && ncell1 > 1u) {
-    const uint64_t key = blockKey[b];
-    const uint64_t nw = (ncell0 + shape[0] - 1) / shape[0];  // windows per row
-    const uint32_t r1 = (uint32_t)((key / nw) % ncell1);       // the block's dim-1 coordinate
-    if ((r1 & 1u) == 0u) {
-      if (r1 + 1u < ncell1) {
-        const uint32_t hiB = (uint64_t)nb - b - 1 > nw ? b + 1 + (uint32_t)nw : nb;
-        const uint32_t j = lower_bound_keys(blockKey, b + 1, hiB, key + nw);
-        if (j < nb && blockKey[j] == key + nw) {
-          pj = j;
-          cnt += pos[blockStart[j + 1]] - pos[blockStart[j]];
-        }
-      }
-    } else {
-      const uint32_t loB = (uint64_t)b > nw ? b - (uint32_t)nw : 0u;
-      const uint32_t j = lower_bound_keys(blockKey, loB, b, key - nw);
-      if (j < b && blockKey[j] == key - nw) cnt = 0;
-    }
-  }
-  partner[b] = pj;
-  ntiles[b] = (cnt + 63) / 64;
-}
-
-// tiles of block b (and its partner): runs of 64 over the block's active queries followed by
-// the partner's, each tile as {second run start, first run start, count, first run length}
-__global__ void k_write_pair_tiles(const uint32_t *blockStart, const uint32_t *pos, const uint32_t *tileOff,
-                                   const uint32_t *nblocks, const uint32_t *partner, uint32_t ncell,
-                                   uint4 *tiles) {
-  const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= ncell || b >= *nblocks) return;
-  uint32_t t = tileOff[b];
-  if (tileOff[b + 1] == t) return;
-  const uint32_t a0 = pos[blockStart[b]], n0 = pos[blockStart[b + 1]] - a0;
-  const uint32_t j = partner[b];
-  uint32_t a1 = 0, n1 = 0;
-  if (j != NO_PARTNER) {
-    a1 = pos[blockStart[j]];
-    n1 = pos[blockStart[j + 1]] - a1;
-  }
-  const uint32_t tot = n0 + n1;
-  for (uint32_t base = 0; base < tot; base += 64, t++) {
-    const uint32_t m = tot - base < 64u ? tot - base : 64u;
-    const uint32_t m0 = base < n0 ? (n0 - base < m ? n0 - base : m) : 0u;
-    const uint32_t s0 = a0 + (base < n0 ? base : n0);
-    const uint32_t s1 = a1 + (base > n0 ? base - n0 : 0u);
-    tiles[t] = make_uint4(s1, s0, m, m0);
-  }
 }
 
 // ------------------------------------------------------------------ checksum
@@ -490,10 +346,6 @@ void gather_rows(const T *in, const uint32_t *ids, uint32_t n, uint32_t d, const
 void gather_u32(const uint32_t *src, const uint32_t *idx, uint32_t n, uint32_t *dst, hipStream_t s) {
   if (n) k_gather_u32<<<(n + 255) / 256, 256, 0, s>>>(src, idx, n, dst);
 }
-void dense_cell_counts(const uint64_t *cellKeys, const uint32_t *cellStart, uint32_t ncell,
-                       uint32_t *dense, hipStream_t s) {
-  if (ncell) k_dense_counts<<<(ncell + 255) / 256, 256, 0, s>>>(cellKeys, cellStart, ncell, dense);
-}
 void pack_bits(const uint8_t *src, uint32_t n, uint64_t *bits, hipStream_t s) {
   if (n) k_pack_bits<<<(n + 255) / 256, 256, 0, s>>>(src, n, bits);
 }
@@ -530,32 +382,6 @@ void active_flags(const uint32_t *sortedIds, const uint8_t *failed, uint32_t n, 
 void compact_active(const uint32_t *sortedIds, const uint32_t *flags, const uint32_t *pos,
                     uint32_t n, uint32_t *act, hipStream_t s) {
   if (n) k_compact_active<<<(n + 255) / 256, 256, 0, s>>>(sortedIds, flags, pos, n, act);
-}
-void choose_span(const uint32_t *activeCount, const unsigned long long *activeCells, uint32_t ncell,
-                 double avgReach, uint32_t spanMax, uint32_t rowsMax, double minTiles, uint32_t *shape,
-                 hipStream_t s) {
-  k_choose_span<<<1, 64, 0, s>>>(activeCount, activeCells, ncell, avgReach, spanMax, rowsMax, minTiles, shape);
-}
-void block_flags_dev(const uint64_t *cellKeys, uint32_t ncell, uint32_t ncell0, const uint32_t *span,
-                     uint32_t *flags, hipStream_t s) {
-  if (ncell) k_block_flags_dev<<<(ncell + 255) / 256, 256, 0, s>>>(cellKeys, ncell, ncell0, span, flags);
-}
-void compact_blocks_keyed(const uint64_t *cellKeys, const uint32_t *cellStart, const uint32_t *flags,
-                          const uint32_t *pos, uint32_t ncell, uint32_t ncell0, const uint32_t *shape,
-                          uint32_t n, uint32_t *blockStart, uint64_t *blockKey, hipStream_t s) {
-  if (ncell)
-    k_compact_blocks_keyed<<<(ncell + 255) / 256, 256, 0, s>>>(cellKeys, cellStart, flags, pos, ncell, ncell0,
-                                                                shape, n, blockStart, blockKey);
-}
-void pair_tiles_dev(const uint32_t *blockStart, const uint64_t *blockKey, const uint32_t *pos,
-                    const uint32_t *nblocks, uint32_t ncell, uint32_t ncell0, uint32_t ncell1,
-                    const uint32_t *shape, uint32_t *partner, uint32_t *ntiles, uint32_t *tileOff,
-                    uint32_t *scratch, uint4 *tiles, hipStream_t s) {
-  if (!ncell) return;
-  k_pair_tile_counts<<<(ncell + 255) / 256, 256, 0, s>>>(blockStart, blockKey, pos, nblocks, ncell, ncell0, ncell1,
-                                                         shape, partner, ntiles);
-  scan_exclusive_u32(ntiles, tileOff, ncell, scratch, s);
-  k_write_pair_tiles<<<(ncell + 255) / 256, 256, 0, s>>>(blockStart, pos, tileOff, nblocks, partner, ncell, tiles);
 }
 
 template <typename T>

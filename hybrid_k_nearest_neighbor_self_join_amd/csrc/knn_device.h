@@ -71,6 +71,18 @@ __device__ __forceinline__ uint32_t cell_coord(T x, T mn, T eps, uint32_t ncell)
   return c >= ncell ? ncell - 1 : c;
 }
 
+// Constants of a dim's outward-rounded cell ranges (cell_geo in knn_range.h)
+template <typename T>
+struct CellGeo {
+  T mn, inv, del;
+  uint32_t top;         // last cell
+  double e, mnp, wide;  // eps, min - pad, eps + 2 pad
+};
+template <typename T, int N>
+struct GeoArgs {
+  CellGeo<T> c[N];
+};
+
 // Slab code of a coordinate of the first non-indexed dim: floor((x - smin) * sscale) clamped to
 // [0, 2^sb - 1], in T arithmetic; non-decreasing in x, so the points of a cell whose codes lie
 // in [code(a), code(b)] include every point with a <= x <= b.

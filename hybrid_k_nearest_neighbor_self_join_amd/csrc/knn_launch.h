@@ -8,27 +8,6 @@
 
 namespace knn {
 
-// Select-kernel bucket counts (knn_range.h, select.hip).
-// The select kernel is built for two bucket counts (select.hip is compiled once per count): fewer
-// buckets take less LDS, so more workgroups per CU, but stage and rank more items per query.
-// The learned schedule's passes run with SEL_NB_LEARNED (40: 14 workgroups per CU), every other
-// pass with SEL_NB_OTHER (56: 12 per CU).  Measured on one MI355X, 10M mixed 2-D points (ms per
-// join, learned K=16 / K=64 / K=128 / plain K=64): 64 buckets 15.1 / 19.4 / 29.4 / 31.7, 56
-// 14.6 / 18.6 / 27.9 / 30.4, 48 14.6 / 18.2 / 27.3 / 31.9, 40 14.1 / 17.5 / 26.9 / 35.3, 32
-// 13.8 / 17.8 / 26.2 / 35.6.
-#ifndef KNN_SELECT_BUCKETS_LEARNED
-#define KNN_SELECT_BUCKETS_LEARNED 40
-#endif
-#ifndef KNN_SELECT_BUCKETS_OTHER
-#define KNN_SELECT_BUCKETS_OTHER 56
-#endif
-constexpr int SEL_NB_LEARNED = KNN_SELECT_BUCKETS_LEARNED;
-constexpr int SEL_NB_OTHER = KNN_SELECT_BUCKETS_OTHER;
-// persistent grid of the select kernel with nb buckets: as many one-wave workgroups per CU (256
-// CUs) as its LDS admits at K = 64 (11 at 64 buckets, 12 at 56, 14 at 40)
-constexpr uint32_t sel_pass_grid(uint32_t nb) { return nb <= 40 ? 3584u : (nb <= 48 ? 3328u : (nb <= 56 ? 3072u : 2816u)); }
-
-
 // ---------------------------------------------------------------- primitives (prims.hip)
 // Exclusive scan of n u32 values into out[0..n); out[n] = total.  `scratch` must hold
 // scan_scratch_words(n) u32 words.  in may alias out.
@@ -114,8 +93,6 @@ void gather_rows(const T *in, const uint32_t *ids, uint32_t n, uint32_t d, const
 // Dense cell-start table (totalCells + 1 entries): denseStart[id] = first sorted position of
 // linear cell id (number of points in cells < id).  counts are scattered from the compacted
 // cell table, then scanned in place.
-void dense_cell_counts(const uint64_t *cellKeys, const uint32_t *cellStart, uint32_t ncell,
-                       uint32_t *dense, hipStream_t s);
 
 // Active flags per sorted position with the own-block pre-check: queries whose own cell
 // block holds fewer than k1 points get failed[q] = 1 and flag 0.  activeBits (pack_bits of the
@@ -135,31 +112,6 @@ void active_flags(const uint32_t *sortedIds, const uint8_t *failed, uint32_t n, 
                   hipStream_t s);
 void compact_active(const uint32_t *sortedIds, const uint32_t *flags, const uint32_t *pos,
                     uint32_t n, uint32_t *act, hipStream_t s);
-
-// Tile blocks: runs of cells in one row (dims 1.. equal) whose dim-0 coordinate falls in the
-// same window of `span` cells (blockStart[b] = first sorted position of block b, blockStart[B]
-// = n; flags/pos are ncell + 1 scratch words), built with every count read on the device (no
-// host round trip; pos is the exclusive scan of the active flags, pos[n] = total): the block
-// shape from the active count *activeCount (k_choose_span's cost model: shape[0] = span,
-// shape[1] = rows), block flags at that span, and tiles of the *nblocks blocks (ntiles /
-// tileOff hold ncell + 1 words; tileOff[ncell] = tile count, read by the range kernels through
-// JoinArgs::ntilesDev).
-void choose_span(const uint32_t *activeCount, const unsigned long long *activeCells, uint32_t ncell,
-                 double avgReach, uint32_t spanMax, uint32_t rowsMax, double minTiles, uint32_t *shape,
-                 hipStream_t s);
-void block_flags_dev(const uint64_t *cellKeys, uint32_t ncell, uint32_t ncell0, const uint32_t *span,
-                     uint32_t *flags, hipStream_t s);
-// Row pairs: with shape[1] = 2 (k_choose_span's choice when rowsMax = 2), the tiles of the
-// block at (row r, window w) of an even dim-1 coordinate r also take the active queries of the
-// block at (r + 1, w), so a tile's queries fill a window of two rows; blockKey[b] = row *
-// windows per row + window of block b (compact_blocks_keyed).  partner holds ncell words.
-void compact_blocks_keyed(const uint64_t *cellKeys, const uint32_t *cellStart, const uint32_t *flags,
-                          const uint32_t *pos, uint32_t ncell, uint32_t ncell0, const uint32_t *shape,
-                          uint32_t n, uint32_t *blockStart, uint64_t *blockKey, hipStream_t s);
-void pair_tiles_dev(const uint32_t *blockStart, const uint64_t *blockKey, const uint32_t *pos,
-                    const uint32_t *nblocks, uint32_t ncell, uint32_t ncell0, uint32_t ncell1,
-                    const uint32_t *shape, uint32_t *partner, uint32_t *ntiles, uint32_t *tileOff,
-                    uint32_t *scratch, uint4 *tiles, hipStream_t s);
 
 // Tile queues of the persistent range kernels: one per XCD (the chip's 8 L2 domains), each
 // over a contiguous eighth of the tiles.
@@ -189,24 +141,29 @@ struct JoinArgs {
   uint32_t *tileCounter; // TILE_QUEUES dynamic tile queue heads (zeroed before the launch)
   uint32_t tileRanges;   // 1: one queue over all tiles; TILE_QUEUES: one range per XCD
   uint32_t segCapLog2;   // positions per chunk of the segment-start bitmap, log2 (6..11; 11 by default)
-  uint32_t selBuckets;   // select kernel: SEL_NB_LEARNED for the learned schedule's passes, else SEL_NB_OTHER (0 = other)
   void *heapScratch;     // heap kernel: global heap storage when K+1 does not fit in LDS
-  uint32_t smax;         // select kernel: LDS staging slots per query
-  uint8_t *overflow;     // select kernel: per point, 1 = needs the overflow (collect or heap) kernel
+  uint8_t *overflow;     // direct kernel: per point, 1 = needs the overflow (collect or heap) kernel
   uint32_t *overflowCount;
   // batched joins: per-set grids / K+1 / row offsets (sets[setOf[q]]), and the tile count
   // read from device memory at kernel start (null: single set, `ntiles`)
   const SetDesc *sets;
   const uint32_t *setOf;
   const uint32_t *ntilesDev;
+  // direct and collect kernels without tiles (tiles null): the active query count (device); a
+  // work unit is then a chunk of consecutive active queries
+  const uint32_t *activeCount;
+  uint32_t lookupRows;   // direct kernel, <= 2 indexed dims: rows of a block looked up per step (1 or 2)
 };
-// Two-pass select kernel (histogram, then bucket-ordered collect); queries whose candidates
-// do not fit in `smax` staging slots are flagged in `overflow` for the overflow kernel.
+// Direct kernel (wave = query, direct.hip): the range kernel of every pass with K+1 <= DR_MAX_K1.
+// A query whose candidates do not fit its lists is flagged in `overflow` for the overflow kernel.
 template <typename T>
-void range_select(const JoinArgs &a, const typename GridOf<T>::type &g, hipStream_t s);
-template <typename T>
-size_t range_select_lds_bytes(uint32_t smax, uint32_t nb);
-uint32_t range_select_grid(uint32_t ntiles);
+void range_direct(const JoinArgs &a, const typename GridOf<T>::type &g, hipStream_t s);
+constexpr uint32_t DR_NB = 256;   // buckets of the key, 4 per lane
+constexpr uint32_t DR_RMAX = 10;  // rows of a query's block kept per chunk (<= 2 indexed dims)
+// Built for three list sizes: H rounds of 64 list items are ranked in registers, up to K+1 =
+// direct_k1(H).
+constexpr uint32_t direct_k1(int h) { return h == 3 ? 40u : (h == 4 ? 224u : 448u); }
+constexpr uint32_t DR_MAX_K1 = direct_k1(8);
 // Collect kernel (wave = query, one pass over its block into an LDS top-(K+1) collector): for
 // queries with many candidates per neighbour.  K+1 <= BRUTE_MAX_K1.
 template <typename T>

@@ -1,4 +1,4 @@
-// knn_range.h -- device helpers shared by the range kernels (select.hip, range.hip).
+// knn_range.h -- device helpers shared by the range kernels (direct.hip, range.hip).
 //
 // Per-query search geometry on the grid: a query with radius r scans the cells
 // [coord(x - r, rounded down), coord(x + r, rounded up)] per indexed dim (kernel.cu:61-110 scans
@@ -18,38 +18,9 @@
 
 namespace knn {
 
-// Select kernel layout (select.hip): SEL_NB buckets of the FP64 key (the last one for keys
-// beyond the query's threshold), two 16-bit counters per LDS word; after the histogram the
-// same LDS region H holds each query's bucket cursors as a row of SEL_RS words (one word of
-// padding against bank conflicts).  Sub-blocks of at most SEL_RMAX rows have their row ranges
-// looked up for the whole tile at once.
-#ifndef KNN_SELECT_BUCKETS
-#define KNN_SELECT_BUCKETS KNN_SELECT_BUCKETS_OTHER
-#endif
-#ifndef KNN_SELECT_RMAX
-#define KNN_SELECT_RMAX 5
-#endif
-constexpr int SEL_NB = KNN_SELECT_BUCKETS;
-static_assert(SEL_NB % 2 == 0 && SEL_NB >= 8 && SEL_NB <= 64, "select buckets: even, 8..64");
-constexpr int SEL_NBIN = SEL_NB - 1;
-constexpr uint32_t SEL_RMAX = KNN_SELECT_RMAX;
-constexpr uint32_t SEL_RS = SEL_NB / 2 + 1;
-// LDS words of the select kernel with nb buckets before its staging arrays: H (the histogram's
-// nb x 32 words, or 64 rows of nb / 2 + 1 cursor words), rowB/rowX[64], prB/prX[SEL_RMAX][64],
-// prT/prR[64], the collecting query's 32-bit cursors qc[64]
-constexpr uint32_t sel_hwords(uint32_t nb) { return nb * 32 > 64 * (nb / 2 + 1) ? nb * 32 : 64 * (nb / 2 + 1); }
-constexpr uint32_t sel_fixed_words(uint32_t nb) { return sel_hwords(nb) + 128 + SEL_RMAX * 128 + 128 + 64; }
-constexpr uint32_t SEL_HWORDS = sel_hwords(SEL_NB);
-constexpr uint32_t SEL_FIXED_WORDS = sel_fixed_words(SEL_NB);
-
-// persistent grid of the select kernel when the tile count is known on the host: 11 one-wave
-// workgroups per CU on 256 CUs
-constexpr uint32_t SELECT_MAX_GRID = 2816;
-
-// Select kernel launch for D data dims and nd indexed dims, built with NB buckets (select.hip,
-// compiled once per bucket count).
-template <typename T, int D, int NB>
-void select_launch(const JoinArgs &a, const typename GridOf<T>::type &g, uint32_t nd, hipStream_t s);
+// Direct kernel launch for D data dims (direct.hip).
+template <typename T, int D>
+void direct_launch(const JoinArgs &a, const typename GridOf<T>::type &g, hipStream_t s);
 
 namespace {
 
@@ -99,7 +70,8 @@ template <> struct Num<float> {
     }
     return s;
   }
-  __device__ static __forceinline__ float bound(double key) { return (float)(key * (1.0 + 0x1p-16)); }
+  // (2^-140: the roundings of sums near the denormals, where they are absolute)
+  __device__ static __forceinline__ float bound(double key) { return (float)(key * (1.0 + 0x1p-16)) + 0x1p-140f; }
 };
 template <> struct Num<double> {
   template <int D>
@@ -399,6 +371,23 @@ __device__ __forceinline__ uint32_t tile_count(const JoinArgs &a) {
   return a.ntilesDev ? *a.ntilesDev : a.ntiles;
 }
 
+// Work units of a wave = query kernel: the tiles (batched groups), or, without tiles, chunks of Q
+// consecutive active queries, Q small enough for every wave of the launch to take `per` of them
+// (a pass of few queries then still fills the chip) and at most 64.
+__device__ __forceinline__ uint32_t work_count(const JoinArgs &a, uint32_t per, uint32_t &Q) {
+  Q = 64;
+  if (a.tiles) return tile_count(a);
+  const uint32_t A = *a.activeCount;
+  Q = A / (gridDim.x * per);
+  Q = Q < 1u ? 1u : (Q > 64u ? 64u : Q);
+  return (A + Q - 1u) / Q;
+}
+__device__ __forceinline__ uint4 work_tile(const JoinArgs &a, uint32_t t, uint32_t Q) {
+  if (a.tiles) return a.tiles[t];
+  const uint32_t q0 = t * Q, left = *a.activeCount - q0, nq = left < Q ? left : Q;
+  return make_uint4(q0, q0, nq, nq);
+}
+
 // Per-wave counters of a persistent kernel (wave-uniform), added to the global counters once
 // when the wave runs out of tiles: per-tile atomics on the same three addresses serialise.
 struct WaveTally {
@@ -540,15 +529,76 @@ __device__ __forceinline__ uint64_t block_rows(const G &g, const uint32_t *lo, c
   return R;
 }
 
-// Inclusive wave prefix sum.
-__device__ __forceinline__ uint32_t wave_incl_sum(uint32_t v, uint32_t lane) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t t = (uint32_t)__shfl_up((int)v, o, 64);
-    if (lane >= (uint32_t)o) v += t;
-  }
+// Inclusive wave prefix sum on the DPP network: row shifts within 16 lanes, then the row
+// broadcasts (six additions, no LDS round trips).  Every lane of the wave must be active.
+__device__ __forceinline__ uint32_t wave_incl_sum(uint32_t v, uint32_t) {
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);
   return v;
 }
+
+// Outward-rounded cell geometry without divisions.  A point x lies in cell
+// trunc(fl(fl(x - min) / eps)) of its dim (cell_coord), non-decreasing in x.  For any x >= a the
+// cell is at least floor((a - min) * (1 / eps) - del), and for x <= a at most floor(... + del):
+// del = 2^-21 (2^-50 for double) of (|min| + |max| + eps) / eps covers the rounding of both
+// sides' subtraction, product and quotient (a few units of 2^-24, 2^-53).  pad covers the same
+// rounding for the coordinates of a cell's edges (2^-18 of the coordinates).
+template <typename T, typename G>
+__host__ __device__ __forceinline__ CellGeo<T> cell_geo(const G &g, uint32_t j) {
+  CellGeo<T> c;
+  const double mn = (double)g.minArr[j], e = (double)g.eps;
+  const double ext = fabs(mn) + fabs(mn + (double)g.nCells[j] * e) + e;
+  c.mn = (T)g.minArr[j];
+  c.inv = (T)1 / (T)g.eps;
+  const double del = ext / e * (sizeof(T) == 4 ? 0x1p-21 : 0x1p-50);
+  c.del = (double)c.inv < 0x1p120 && del <= 0.25 ? (T)del : (T)1;
+  c.top = g.nCells[j] - 1u;
+  c.e = e;
+  c.mnp = mn - 0x1p-18 * ext;
+  c.wide = e + 0x1p-17 * ext;
+  return c;
+}
+template <typename T>
+__device__ __forceinline__ uint32_t cell_floor(T t, uint32_t top) {
+  t = t > (T)0 ? t : (T)0;
+  t = t < (T)4294967040.0 ? t : (T)4294967040.0;
+  const uint32_t c = (uint32_t)t;
+  return c < top ? c : top;
+}
+// cells of [x - h, x + h] (c.del <= 1/4)
+template <typename T>
+__device__ __forceinline__ void cell_span_fast(const CellGeo<T> &c, T x, T h, uint32_t &l, uint32_t &u) {
+  l = cell_floor<T>(((x - h) - c.mn) * c.inv - c.del, c.top);
+  u = cell_floor<T>(((x + h) - c.mn) * c.inv + c.del, c.top);
+}
+// the same on any grid: one so fine (or an eps so small) that del is no small part of a cell takes
+// cell_coord's own division
+template <typename T>
+__device__ __forceinline__ void cell_span(const CellGeo<T> &c, T x, T h, uint32_t &l, uint32_t &u) {
+  if (c.del <= (T)0.25) {
+    cell_span_fast<T>(c, x, h, l, u);
+  } else {
+    l = cell_coord<T>(next_down(x - h), c.mn, (T)c.e, c.top + 1u);
+    u = cell_coord<T>(next_up(x + h), c.mn, (T)c.e, c.top + 1u);
+  }
+}
+// distance^2 from q to the slab of cell cur
+template <typename T>
+__device__ __forceinline__ double cell_gap2(const CellGeo<T> &c, uint32_t cur, double q) {
+  const double a = (double)cur * c.e + c.mnp - q;
+  const double gap = fmax(fmax(a, -a - c.wide), 0.0);
+  return gap * gap;
+}
+// half chord sqrt(d2) = r sqrt(d2 / r^2), rounded up (0 <= d2 <= about r^2; the ratio keeps the
+// hardware root, which flushes denormals, away from them)
+__device__ __forceinline__ float half_chord(double d2, float r, double invr2) {
+  return r * __builtin_amdgcn_sqrtf((float)(d2 * invr2)) * (1.0f + 0x1p-20f);
+}
+__device__ __forceinline__ double half_chord(double d2, double, double) { return sqrt(d2) * (1.0 + 0x1p-20); }
 
 // Segments whose lengths average this many positions or more are streamed one at a time (the
 // partly empty last round of each then costs less than looking up every candidate's segment).

@@ -2,12 +2,12 @@
 //
 // Replace kernel.cu:61-225 (range query over the adjacent cells), the pair buffer and the two
 // thrust::stable_sort_by_key of GPU.cu:1629-1634, and the host top-k of GPU.cu:3610-3704, with
-// the select kernel (select.hip):
-// k_range_collect (5 or more indexed dims): wave = query, one pass over the query's own block
-//   into the LDS top-(K+1) collector of knn_collect.h, FP32-prefiltered against its threshold.
+// the direct kernel (direct.hip):
+// k_range_collect: wave = query, one pass over the query's own block into the LDS top-(K+1)
+//   collector of knn_collect.h, FP32-prefiltered against its threshold; takes the direct kernel's
+//   overflow queries and every query above its K+1.
 // k_range_heap: per-lane max-heap of (key, id), in LDS when K+1 fits, else in global scratch;
-//   takes the select kernel's overflow queries above the collector's K+1 (the collect kernel
-//   takes them below).
+//   takes the queries above the collector's K+1.
 #include "knn_collect.h"
 #include "knn_range.h"
 
@@ -22,12 +22,10 @@ namespace {
 // T bound of the collector's threshold (first Tq = r^2 (1 - 2^-20), then the (K+1)-th key
 // held), and only candidates that pass get their FP64 key and enter the LDS collector.  The
 // query succeeds when K+1 pairs with key <= Tq were collected: they are then its exact
-// top-(K+1), since every point with key <= Tq lies in the block.  One pass over the
-// candidates, against the select kernel's two (the tile's union, then the query's sub-block):
-// the better choice when a query has many candidates per neighbour, as with 5 or more indexed
-// dims.  Built per number of indexed dims ND where that equals D or is 6 (every per-dim array
-// then lives in registers), else for the runtime count (ND = 0).  On a grid in slab order the
-// fixed-dims builds cut each cell of the block to the query's slab, as the select kernel does.
+// top-(K+1), since every point with key <= Tq lies in the block.  Built per number of indexed dims
+// ND where that equals D or is 6 (every per-dim array then lives in registers), else for the
+// runtime count (ND = 0).  On a grid in slab order the fixed-dims builds cut each cell of the
+// block to the query's slab, as the direct kernel does.
 template <typename T, int D, int ND, typename G>
 __global__ __launch_bounds__(64) void k_range_collect(JoinArgs a, G g0) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -38,13 +36,14 @@ __global__ __launch_bounds__(64) void k_range_collect(JoinArgs a, G g0) {
   const T *__restrict__ xs = reinterpret_cast<const T *>(a.xs);
   const T *__restrict__ x = reinterpret_cast<const T *>(a.x);
   const size_t n = a.n;
-  const uint32_t NT = tile_count(a);
+  uint32_t Q;
+  const uint32_t NT = work_count(a, 4u, Q);
   constexpr int PR = D <= 8 ? 4 : 2;
   WaveTally tally;
   for (;;) {
     const uint32_t t = next_tile(a.tileCounter, NT, a.tileRanges, lane);
     if (t >= NT) break;
-    const uint4 tl = a.tiles[t];
+    const uint4 tl = work_tile(a, t, Q);
     const TileCtx<G> C = tile_ctx<G>(a, g0, tl);
     const G &g = C.g;
     const uint32_t nd = nd_of<ND>(g);
@@ -331,7 +330,7 @@ void launch_heap(const JoinArgs &a, const G &g, hipStream_t s) {
 template <typename T, int D, typename G>
 void launch_collect(const JoinArgs &a, const G &g, hipStream_t s) {
   if (a.ntiles == 0) return;
-  const uint32_t grid = a.ntilesDev ? a.ntiles : range_select_grid(a.ntiles);
+  const uint32_t grid = a.ntiles;  // persistent; the work count is on the device
   const size_t lds = range_collect_lds_bytes(a.k1);
   if constexpr (D <= KNN_MAX_INDEXED) {
     if (g.nd == (uint32_t)D) {
@@ -350,16 +349,6 @@ void launch_collect(const JoinArgs &a, const G &g, hipStream_t s) {
 }
 
 }  // namespace
-
-uint32_t range_select_grid(uint32_t ntiles) {
-  return ntiles < SELECT_MAX_GRID ? (ntiles ? ntiles : 1u) : SELECT_MAX_GRID;
-}
-
-template <typename T>
-size_t range_select_lds_bytes(uint32_t smax, uint32_t nb) {
-  return (size_t)sel_fixed_words(nb) * sizeof(uint32_t) + (size_t)smax * 8 +
-         (size_t)(smax + (smax & 1)) * 4 + (size_t)smax * sizeof(T);
-}
 
 #define DISPATCH_D(FN)                              \
   switch (a.d) {                                    \
@@ -382,23 +371,15 @@ size_t range_select_lds_bytes(uint32_t smax, uint32_t nb) {
     default: break;                                 \
   }
 
-// the learned schedule's bucket count when a.selBuckets names it, else the other one
 template <typename T>
-void range_select(const JoinArgs &a, const typename GridOf<T>::type &g, hipStream_t s) {
-  const bool learned = a.selBuckets == (uint32_t)SEL_NB_LEARNED;
-#define SEL_CASE(DD)                                                        \
-  case DD:                                                                  \
-    if (learned)                                                            \
-      select_launch<T, DD, SEL_NB_LEARNED>(a, g, g.nd, s);                  \
-    else                                                                    \
-      select_launch<T, DD, SEL_NB_OTHER>(a, g, g.nd, s);                    \
-    break;
+void range_direct(const JoinArgs &a, const typename GridOf<T>::type &g, hipStream_t s) {
+#define DR_CASE(DD) case DD: direct_launch<T, DD>(a, g, s); break;
   switch (a.d) {
-    SEL_CASE(1) SEL_CASE(2) SEL_CASE(3) SEL_CASE(4) SEL_CASE(5) SEL_CASE(6) SEL_CASE(7) SEL_CASE(8)
-    SEL_CASE(9) SEL_CASE(10) SEL_CASE(11) SEL_CASE(12) SEL_CASE(13) SEL_CASE(14) SEL_CASE(15) SEL_CASE(16)
+    DR_CASE(1) DR_CASE(2) DR_CASE(3) DR_CASE(4) DR_CASE(5) DR_CASE(6) DR_CASE(7) DR_CASE(8)
+    DR_CASE(9) DR_CASE(10) DR_CASE(11) DR_CASE(12) DR_CASE(13) DR_CASE(14) DR_CASE(15) DR_CASE(16)
     default: break;
   }
-#undef SEL_CASE
+#undef DR_CASE
 }
 
 template <typename T>
@@ -427,8 +408,7 @@ size_t range_heap_scratch_bytes(uint32_t ntiles, uint32_t k1) {
 }
 
 #define INST(T)                                                                          \
-  template void range_select<T>(const JoinArgs &, const GridOf<T>::type &, hipStream_t); \
-  template size_t range_select_lds_bytes<T>(uint32_t, uint32_t);                                   \
+  template void range_direct<T>(const JoinArgs &, const GridOf<T>::type &, hipStream_t); \
   template void range_topk<T>(const JoinArgs &, const GridOf<T>::type &, hipStream_t);   \
   template void range_collect<T>(const JoinArgs &, const GridOf<T>::type &, hipStream_t); \
   template size_t range_heap_scratch_bytes<T>(uint32_t, uint32_t);

@@ -1,0 +1,67 @@
+"""GPU tests of the direct range kernel (csrc/direct.hip) at the edges of its lists and tables:
+K+1 around the sizes its three builds end at (40, 224, 448), point counts around a wave and a
+chunk, blocks from empty to crowded, equal keys and equal coordinates, root arguments below the
+fast path's range.  Rows are compared with FP64 brute force (ids, and FP32 distance bits)."""
+import numpy as np
+import pytest
+
+from hybrid_k_nearest_neighbor_self_join_amd import _lib, learned_radius, synthetic
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(oracle, pts, k, **kw):
+    ids, dist, st = _lib.knnjoin_ex(pts, k, brute_fallback=0, **kw)
+    perm, _ = oracle.reorder(pts)
+    bi, bd = oracle.bruteforce(np.ascontiguousarray(pts[:, perm]), k)
+    assert np.array_equal(ids, bi)
+    assert np.array_equal(dist.view(np.uint32), bd.view(np.uint32))
+    return st
+
+
+@pytest.mark.parametrize("k", [1, 38, 39, 40, 63, 64, 127, 128, 191, 223, 224, 300, 447, 448])
+def test_list_sizes(oracle, k):
+    st = _check(oracle, synthetic.mixed_box(6007, seed=k), k, beta=0.025)
+    assert st.overflow_queries == 0
+
+
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 129, 4097])
+@pytest.mark.parametrize("d,nd", [(1, 1), (2, 2), (3, 2), (3, 3), (5, 4), (6, 5), (8, 6), (9, 7)])
+def test_point_counts_and_dims(oracle, n, d, nd):
+    pts = np.random.default_rng(n * 10 + d).uniform(-3.0, 5.0, (n, d)).astype(np.float32)
+    _check(oracle, pts, min(5, n - 1), num_indexed_dims=nd, beta=0.05)
+
+
+@pytest.mark.parametrize("mode", [_lib.KNN_MODE_BETA, _lib.KNN_MODE_LEARNED])
+def test_crowded_and_empty_blocks(oracle, mode):
+    # one dense cluster (blocks of thousands of points: shrunk radii, tightened lists), a sparse
+    # background and far outliers (many passes)
+    learned_radius.register_default_models()
+    rng = np.random.default_rng(5)
+    pts = np.concatenate([rng.normal(0.0, 0.01, (6000, 2)), rng.uniform(-50, 50, (3000, 2)),
+                          rng.uniform(400, 500, (5, 2))]).astype(np.float32)
+    _check(oracle, pts[rng.permutation(len(pts))], 20, mode=mode)
+
+
+@pytest.mark.parametrize("d,nd", [(2, 2), (3, 3), (4, 2)])
+def test_equal_keys(oracle, d, nd):
+    # a coarse lattice: every distance is shared by many points, ranked by id
+    rng = np.random.default_rng(d)
+    pts = (rng.integers(0, 24 if d == 2 else 8, (5000, d)) / 8.0).astype(np.float32)
+    _check(oracle, pts, 30, num_indexed_dims=nd, beta=0.025)
+
+
+@pytest.mark.parametrize("scale", [1e-18, 3e-17, 1e-10])
+def test_small_distances(oracle, scale):
+    # squared distances around and below 2^-96, where the root needs its scaled form
+    pts = (np.random.default_rng(3).uniform(0, 1, (3000, 2)) * scale).astype(np.float32)
+    _check(oracle, pts, 8)
+
+
+def test_double_rows(oracle):
+    pts = np.random.default_rng(9).uniform(0, 1, (5000, 3))
+    ids, dist, _ = _lib.knnjoin_ex(pts, 24, brute_fallback=0)
+    perm, _ = oracle.reorder(pts)
+    bi, bd = oracle.bruteforce(np.ascontiguousarray(pts[:, perm]), 24)
+    assert np.array_equal(ids, bi)
+    assert np.array_equal(dist.view(np.uint64), bd.view(np.uint64))
