@@ -1968,6 +1968,43 @@ int knnjoin_outlier_scores(const int32_t *ids, const float *dists, uint32_t n, u
 }  // extern "C"
 
 // ------------------------------------------------------------------ learned-radius entries
+namespace knn {
+// Training buffers in the S_TRAIN slot: parameters, Adam moments, gradients, n samples with their
+// shuffled order, one batch's activations, nloss losses (every array on a 16-byte boundary).
+struct MlpBuffers {
+  float *W, *M, *V, *G, *H1, *H2, *dH1, *dH2, *Xb, *err, *dout;
+  uint32_t *idx;
+};
+static MlpBuffers mlp_buffers(uint32_t n, uint32_t B, uint32_t nloss, float *&X, float *&Y, float *&loss) {
+  auto up = [](size_t w) { return (w + 3) & ~(size_t)3; };
+  const size_t pw = up(MLP_NW), hw = (size_t)B * MLP_H;
+  const size_t words = 4 * pw + up((size_t)n * MLP_IN) + 2 * up(n) + 4 * hw + up((size_t)B * MLP_IN) + 2 * up(B) + up(nloss);
+  float *b = reinterpret_cast<float *>(g_cache.get(S_TRAIN, sizeof(float) * words));
+  auto take = [&](size_t w) {
+    float *r = b;
+    b += w;
+    return r;
+  };
+  MlpBuffers m;
+  m.W = take(pw);
+  m.M = take(pw);
+  m.V = take(pw);
+  m.G = take(pw);
+  m.H1 = take(hw);
+  m.H2 = take(hw);
+  m.dH1 = take(hw);
+  m.dH2 = take(hw);
+  m.Xb = take(up((size_t)B * MLP_IN));
+  m.err = take(up(B));
+  m.dout = take(up(B));
+  X = take(up((size_t)n * MLP_IN));
+  Y = take(up(n));
+  m.idx = reinterpret_cast<uint32_t *>(take(up(n)));
+  loss = take(up(nloss));
+  return m;
+}
+}  // namespace knn
+
 extern "C" {
 
 int knnjoin_set_radius_model_dims(uint32_t ndim, uint32_t nd, const float *weights, uint32_t nweights,
@@ -2079,15 +2116,13 @@ int knnjoin_mlp_grad(const float *weights, const float *X, const float *Y, uint3
     using namespace knn;
     if (!weights || !X || !Y || !grads) throw Error(KNN_ERR_ARG, "null argument");
     hipStream_t s = lib_stream();
-    const size_t words = (size_t)2 * MLP_NW + 1 + (size_t)B * (MLP_IN + 1 + 4 * MLP_H + 2);
-    float *buf = reinterpret_cast<float *>(g_cache.get(S_TRAIN, sizeof(float) * words));
-    float *Wd = buf, *Gd = Wd + MLP_NW, *Ld = Gd + MLP_NW, *Xd = Ld + 1, *Yd = Xd + (size_t)B * MLP_IN;
-    float *H1 = Yd + B, *H2 = H1 + (size_t)B * MLP_H, *dH1 = H2 + (size_t)B * MLP_H, *dH2 = dH1 + (size_t)B * MLP_H;
-    float *o = dH2 + (size_t)B * MLP_H, *dout = o + B;
-    HIP_CHECK(hipMemcpyAsync(Wd, weights, sizeof(float) * MLP_NW, hipMemcpyHostToDevice, s));
+    float *Xd, *Yd, *Ld;
+    const MlpBuffers m = mlp_buffers(B, B, 1, Xd, Yd, Ld);
+    HIP_CHECK(hipMemcpyAsync(m.W, weights, sizeof(float) * MLP_NW, hipMemcpyHostToDevice, s));
     HIP_CHECK(hipMemcpyAsync(Xd, X, sizeof(float) * (size_t)B * MLP_IN, hipMemcpyHostToDevice, s));
     HIP_CHECK(hipMemcpyAsync(Yd, Y, sizeof(float) * B, hipMemcpyHostToDevice, s));
-    mlp_grad_batch(Wd, Xd, Yd, B, H1, H2, o, dout, dH1, dH2, Gd, Ld, s);
+    float *Gd = m.G;
+    mlp_step(m.W, Xd, Yd, nullptr, B, m.Xb, m.err, m.H1, m.H2, m.dout, m.dH1, m.dH2, Gd, Ld, nullptr, s);
     HIP_CHECK(hipMemcpyAsync(grads, Gd, sizeof(float) * MLP_NW, hipMemcpyDeviceToHost, s));
     if (loss) HIP_CHECK(hipMemcpyAsync(loss, Ld, sizeof(float), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
@@ -2104,19 +2139,15 @@ int knnjoin_mlp_train(float *weights, const float *X, const float *Y, uint32_t n
     if (!weights || !X || !Y || n == 0 || batch == 0) throw Error(KNN_ERR_ARG, "bad training arguments");
     hipStream_t s = lib_stream();
     const uint32_t B = std::min(batch, n);
-    const size_t words = (size_t)4 * MLP_NW + 1 + (size_t)n * (MLP_IN + 1) +
-                         (size_t)B * (MLP_IN + 1 + 4 * MLP_H + 2) + n;
-    float *buf = reinterpret_cast<float *>(g_cache.get(S_TRAIN, sizeof(float) * words));
-    float *Wd = buf, *Gd = Wd + MLP_NW, *Md = Gd + MLP_NW, *Vd = Md + MLP_NW, *Ld = Vd + MLP_NW;
-    float *Xall = Ld + 1, *Yall = Xall + (size_t)n * MLP_IN;
-    float *Xb = Yall + n, *Yb = Xb + (size_t)B * MLP_IN;
-    float *H1 = Yb + B, *H2 = H1 + (size_t)B * MLP_H, *dH1 = H2 + (size_t)B * MLP_H, *dH2 = dH1 + (size_t)B * MLP_H;
-    float *o = dH2 + (size_t)B * MLP_H, *dout = o + B;
-    uint32_t *idx = reinterpret_cast<uint32_t *>(dout + B);
-    HIP_CHECK(hipMemcpyAsync(Wd, weights, sizeof(float) * MLP_NW, hipMemcpyHostToDevice, s));
+    const uint32_t nb = n / B;
+    float *Xall, *Yall, *lossD;
+    const MlpBuffers m = mlp_buffers(n, B, nb, Xall, Yall, lossD);
+    uint32_t *idx = m.idx;
+    HIP_CHECK(hipMemcpyAsync(m.W, weights, sizeof(float) * MLP_NW, hipMemcpyHostToDevice, s));
     HIP_CHECK(hipMemcpyAsync(Xall, X, sizeof(float) * (size_t)n * MLP_IN, hipMemcpyHostToDevice, s));
     HIP_CHECK(hipMemcpyAsync(Yall, Y, sizeof(float) * n, hipMemcpyHostToDevice, s));
-    fill_u32(reinterpret_cast<uint32_t *>(Md), 0u, 2 * (size_t)MLP_NW, s);
+    fill_u32(reinterpret_cast<uint32_t *>(m.M), 0u, MLP_NW, s);
+    fill_u32(reinterpret_cast<uint32_t *>(m.V), 0u, MLP_NW, s);
     std::vector<uint32_t> order(n);
     for (uint32_t i = 0; i < n; i++) order[i] = i;
     uint64_t st = seed;
@@ -2128,32 +2159,31 @@ int knnjoin_mlp_train(float *weights, const float *X, const float *Y, uint32_t n
     };
     const float b1 = 0.9f, b2 = 0.999f, epsA = 1e-8f;
     uint64_t step = 0;
-    const uint32_t nb = n / B;
+    std::vector<float> hl(nb);
     for (uint32_t e = 0; e < epochs; e++) {
       for (uint32_t i = n - 1; i > 0; i--) {
         const uint32_t j = (uint32_t)(next() % (uint64_t)(i + 1));
         std::swap(order[i], order[j]);
       }
       HIP_CHECK(hipMemcpyAsync(idx, order.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice, s));
-      double lsum = 0;
       for (uint32_t bi = 0; bi < nb; bi++) {
-        gather_rows(Xall, idx + (size_t)bi * B, B, MLP_IN, Xb, s);
-        gather_rows(Yall, idx + (size_t)bi * B, B, 1, Yb, s);
-        mlp_grad_batch(Wd, Xb, Yb, B, H1, H2, o, dout, dH1, dH2, Gd, Ld, s);
         step++;
         const float c1 = (float)(1.0 - std::pow(0.9, (double)step));
         const float c2 = (float)(1.0 - std::pow(0.999, (double)step));
-        adam_step(Wd, Gd, Md, Vd, lr, b1, b2, c1, c2, epsA, s);
-        float hl = 0;
-        if (loss_per_epoch) {
-          HIP_CHECK(hipMemcpyAsync(&hl, Ld, sizeof(float), hipMemcpyDeviceToHost, s));
-          HIP_CHECK(hipStreamSynchronize(s));
-          lsum += hl;
-        }
+        const AdamStep ad{m.W, m.M, m.V, lr, b1, b2, c1, c2, epsA};
+        mlp_step(m.W, Xall, Yall, idx + (size_t)bi * B, B, m.Xb, m.err, m.H1, m.H2, m.dout, m.dH1, m.dH2, nullptr,
+                 lossD + bi, &ad, s);
       }
-      if (loss_per_epoch) loss_per_epoch[e] = nb ? (float)(lsum / nb) : 0.0f;
+      LAUNCH_CHECK();
+      if (loss_per_epoch) HIP_CHECK(hipMemcpyAsync(hl.data(), lossD, sizeof(float) * nb, hipMemcpyDeviceToHost, s));
+      HIP_CHECK(hipStreamSynchronize(s));  // the epoch's order and losses are the host's again
+      if (loss_per_epoch) {
+        double lsum = 0;
+        for (uint32_t bi = 0; bi < nb; bi++) lsum += hl[bi];
+        loss_per_epoch[e] = nb ? (float)(lsum / nb) : 0.0f;
+      }
     }
-    HIP_CHECK(hipMemcpyAsync(weights, Wd, sizeof(float) * MLP_NW, hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipMemcpyAsync(weights, m.W, sizeof(float) * MLP_NW, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
     return KNN_OK;
   });

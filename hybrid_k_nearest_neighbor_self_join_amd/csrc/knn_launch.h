@@ -211,14 +211,18 @@ void grow_radius(T *radius, const uint8_t *failed, uint32_t n, T factor, hipStre
 // largest radius among failed queries into out (8 bytes: float bits or double bits)
 void max_failed_radius(const float *radius, const uint8_t *failed, uint32_t n, void *out, hipStream_t s);
 void max_failed_radius(const double *radius, const uint8_t *failed, uint32_t n, void *out, hipStream_t s);
-void gather_rows(const float *in, const uint32_t *idx, uint32_t B, uint32_t w, float *out, hipStream_t s);
 void mlp_forward_batch(const float *W, const float *X, uint32_t B, float *H1, float *H2, float *out,
                        hipStream_t s);
-void mlp_grad_batch(const float *W, const float *X, const float *Y, uint32_t B, float *H1,
-                    float *H2, float *out, float *dout, float *dH1, float *dH2, float *G,
-                    float *loss, hipStream_t s);
-void adam_step(float *W, const float *G, float *M, float *V, float lr, float b1, float b2, float c1,
-               float c2, float eps, hipStream_t s);
+// One training step over the samples idx[0..B) (0..B-1 without idx): forward, backward, the
+// parameters' gradients (G, optional) and the mean squared error (loss, optional), and with
+// `step` the Adam update of its parameters (c1, c2: the bias corrections).
+struct AdamStep {
+  float *W, *M, *V;
+  float lr, b1, b2, c1, c2, eps;
+};
+void mlp_step(const float *W, const float *X, const float *Y, const uint32_t *idx, uint32_t B, float *Xb,
+              float *err, float *H1, float *H2, float *dout, float *dH1, float *dH2, float *G, float *loss,
+              const AdamStep *step, hipStream_t s);
 
 // ------------------------------------------------------------- batched sets (batched.hip)
 // Group arrays hold the concatenated points of sets with one dimensionality d; sets[si]

@@ -378,14 +378,6 @@ __global__ void k_max_radius_d(const double *radius, const uint8_t *failed, uint
 }
 
 // gather rows of a (n x w) float matrix: out[b] = in[idx[b]]
-__global__ void k_gather_rows(const float *in, const uint32_t *idx, uint32_t B, uint32_t w, float *out) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= B * w) return;
-  const uint32_t b = t / w, j = t % w;
-  out[t] = in[(size_t)idx[b] * w + j];
-}
-
-// ---------------------------------------------------------------- training kernels
 __global__ void k_mlp_fwd(const float *__restrict__ Wg, const float *__restrict__ X, uint32_t B,
                           float *H1, float *H2, float *out) {
   __shared__ float W[MLP_NW];
@@ -399,81 +391,194 @@ __global__ void k_mlp_fwd(const float *__restrict__ Wg, const float *__restrict_
   out[b] = mlp_forward(W, f, H1 + (size_t)b * MLP_H, H2 + (size_t)b * MLP_H);
 }
 
-// per sample: dout = 2 (out - y) / B, dH2 = dout w3 [h2 > 0], dH1 = (W2^T dH2) [h1 > 0]
-__global__ void k_mlp_bwd_samples(const float *__restrict__ Wg, const float *__restrict__ Y,
-                                  uint32_t B, const float *H1, const float *H2, const float *out,
-                                  float *dout, float *dH1, float *dH2) {
-  __shared__ float W[MLP_NW];
-  for (uint32_t i = threadIdx.x; i < MLP_NW; i += blockDim.x) W[i] = Wg[i];
+// Forward and backward of B samples (rows idx[b] of X and Y, b itself without idx): the samples'
+// inputs in batch order (Xb: k_mlp_wgrad then reads them without the index), activations
+// H1, H2, err = out - y, dout = 2 err / B, dH2 = dout w3 [h2 > 0], dH1 = (W2^T dH2) [h1 > 0].  Wave = 4
+// samples, lane = unit: a layer's inputs are broadcast from the lanes that hold them, so each
+// unit's sum keeps the oracle's order (bias, then inputs ascending) while 64 units and 4 samples
+// advance together; W2 in LDS with rows of 65 words serves both directions without conflicts.
+// A thread per sample left 32 of 256 CUs with work: 4096 samples took 46 us forward and 91 us
+// backward; this kernel takes both in 18 us.
+constexpr int FB_S = 4;  // samples per wave
+__global__ __launch_bounds__(256) void k_mlp_fb(const float *__restrict__ Wg, const float *__restrict__ X,
+                                                const float *__restrict__ Y, const uint32_t *__restrict__ idx,
+                                                uint32_t B, float *__restrict__ Xb, float *__restrict__ err,
+                                                float *__restrict__ H1, float *__restrict__ H2,
+                                                float *__restrict__ dout, float *__restrict__ dH1,
+                                                float *__restrict__ dH2) {
+  __shared__ float W2s[MLP_H * 65];
+  __shared__ float W1s[MLP_H * 13];
+  for (uint32_t i = threadIdx.x; i < MLP_H * MLP_H; i += 256) W2s[(i >> 6) * 65 + (i & 63u)] = Wg[832 + i];
+  for (uint32_t i = threadIdx.x; i < MLP_H * MLP_IN; i += 256) W1s[(i / MLP_IN) * 13 + i % MLP_IN] = Wg[i];
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t b0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * FB_S;
+  const float b1 = Wg[768 + lane], b2 = Wg[4928 + lane], w3 = Wg[4992 + lane], b3 = Wg[5056];
+  float f[FB_S], y[FB_S];
+#pragma unroll
+  for (int s = 0; s < FB_S; s++) {
+    const uint32_t b = b0 + s < B ? b0 + s : B - 1u;
+    const uint32_t r = idx ? idx[b] : b;
+    f[s] = lane < MLP_IN ? X[(size_t)r * MLP_IN + lane] : 0.0f;
+    y[s] = Y[r];
+  }
   __syncthreads();
-  const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
-  const float *W2 = W + 832, *w3 = W + 4992;
-  const float d = 2.0f * (out[b] - Y[b]) / (float)B;
-  dout[b] = d;
-  float g2[MLP_H];
+  float h1[FB_S], h2[FB_S], o[FB_S], g1[FB_S], g2[FB_S];
 #pragma unroll
-  for (int i = 0; i < MLP_H; i++) {
-    g2[i] = H2[(size_t)b * MLP_H + i] > 0.0f ? d * w3[i] : 0.0f;
-    dH2[(size_t)b * MLP_H + i] = g2[i];
+  for (int s = 0; s < FB_S; s++) {
+    h1[s] = b1;
+    h2[s] = b2;
+    o[s] = b3;
+    g1[s] = 0.0f;
   }
+#pragma unroll
+  for (int t = 0; t < MLP_IN; t++) {
+    const float w = W1s[lane * 13 + t];
+#pragma unroll
+    for (int s = 0; s < FB_S; s++) h1[s] = fmaf(w, readlane<float>(f[s], t), h1[s]);
+  }
+#pragma unroll
+  for (int s = 0; s < FB_S; s++) h1[s] = relu(h1[s]);
+#pragma unroll 16
   for (int j = 0; j < MLP_H; j++) {
-    float a = 0.0f;
+    const float w = W2s[lane * 65 + j];
 #pragma unroll
-    for (int i = 0; i < MLP_H; i++) a = fmaf(W2[i * MLP_H + j], g2[i], a);
-    dH1[(size_t)b * MLP_H + j] = H1[(size_t)b * MLP_H + j] > 0.0f ? a : 0.0f;
+    for (int s = 0; s < FB_S; s++) h2[s] = fmaf(w, readlane<float>(h1[s], j), h2[s]);
+  }
+#pragma unroll
+  for (int s = 0; s < FB_S; s++) h2[s] = relu(h2[s]);
+#pragma unroll 16
+  for (int i = 0; i < MLP_H; i++) {
+    const float w = readlane<float>(w3, i);
+#pragma unroll
+    for (int s = 0; s < FB_S; s++) o[s] = fmaf(w, readlane<float>(h2[s], i), o[s]);
+  }
+#pragma unroll
+  for (int s = 0; s < FB_S; s++) {
+    const float d = 2.0f * (o[s] - y[s]) / (float)B;
+    g2[s] = h2[s] > 0.0f ? d * w3 : 0.0f;
+    if (b0 + s < B) {
+      if (lane < MLP_IN) Xb[(size_t)(b0 + s) * MLP_IN + lane] = f[s];
+      if (lane == 0) {
+        err[b0 + s] = o[s] - y[s];
+        dout[b0 + s] = d;
+      }
+    }
+  }
+#pragma unroll 16
+  for (int i = 0; i < MLP_H; i++) {
+    const float w = W2s[i * 65 + lane];
+#pragma unroll
+    for (int s = 0; s < FB_S; s++) g1[s] = fmaf(w, readlane<float>(g2[s], i), g1[s]);
+  }
+#pragma unroll
+  for (int s = 0; s < FB_S; s++) {
+    if (b0 + s >= B) break;
+    const size_t at = (size_t)(b0 + s) * MLP_H + lane;
+    H1[at] = h1[s];
+    H2[at] = h2[s];
+    dH2[at] = g2[s];
+    dH1[at] = h1[s] > 0.0f ? g1[s] : 0.0f;
   }
 }
 
-// one thread per parameter: gradients summed over the batch in sample order
-__global__ void k_mlp_wgrad(const float *__restrict__ X, uint32_t B, const float *H1, const float *H2,
-                            const float *dout, const float *dH1, const float *dH2, float *G) {
-  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= MLP_NW) return;
+// Gradients of the 5057 parameters and the loss, each a sum over the batch in sample order (a
+// serial chain per parameter: B dependent fused multiply-adds bound this kernel), then, with W,
+// the parameters' Adam step: m = b1 m + (1-b1) g, v = b2 v + (1-b2) g^2,
+// w -= lr (m / c1) / (sqrt(v / c2) + eps).
+// Every gradient is sum_b u[b] M[b][lane] for a matrix M of 64 columns: the four waves of a block
+// take four u of one M, whose rows they stage together in LDS, the next tile's loads in flight
+// while this tile's chains run.
+//   blocks 0..15   W2[i][lane]: M = H1,  u = dH2[:, i], i = 4 block + wave
+//   blocks 16..19  W1[lane][j]: M = dH1, u = X[:, j],   j = 4 (block - 16) + wave; j = 12: b1, u = 1
+//   block 20       M = H2: w3, u = dout; wave 1: b3, the sum of dout; wave 2: the loss
+//   block 21       M = dH2: b2, u = 1
+// A thread per parameter reading both factors from memory took 913 us for 4096 samples and the
+// loss kernel 215 us; this kernel takes 67 us (16 ns a step of the chains: 2 LDS reads and a
+// dependent multiply-add each).
+constexpr uint32_t WG_ROWS = 256;  // samples per tile: its chains outlast the next tile's loads
+constexpr uint32_t WG_BLOCKS = 22;
+struct AdamArgs {
+  float *W, *M, *V;  // W null: gradients only
+  float lr, b1, b2, c1, c2, eps;
+};
+__global__ __launch_bounds__(256) void k_mlp_wgrad(const float *__restrict__ Xb, const float *__restrict__ err, uint32_t B,
+                                                   const float *__restrict__ H1, const float *__restrict__ H2,
+                                                   const float *__restrict__ dout,
+                                                   const float *__restrict__ dH1, const float *__restrict__ dH2,
+                                                   float *__restrict__ G, float *__restrict__ loss, AdamArgs ad) {
+  __shared__ __align__(16) float tile[2][WG_ROWS * MLP_H];
+  __shared__ __align__(16) float ut[2][4][WG_ROWS];
+  const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6, k = blockIdx.x;
+  const float *Mx = k < 16 ? H1 : (k < 20 ? dH1 : (k == 20 ? H2 : dH2));
+  const uint32_t j = k < 16 ? 4u * k + wv : 4u * (k - 16u) + wv;  // this wave's column of u
+  auto u_of = [&](uint32_t b) -> float {
+    if (b >= B) return 0.0f;
+    if (k < 16u) return dH2[(size_t)b * MLP_H + j];
+    if (k < 20u) return j < MLP_IN ? Xb[(size_t)b * MLP_IN + j] : 1.0f;
+    if (k == 20u) return wv < 2u ? dout[b] : err[b];
+    return 1.0f;
+  };
+  constexpr int V4 = WG_ROWS * MLP_H / 4 / 256;
+  float4 nx[V4];
+  constexpr int U64 = WG_ROWS / 64;
+  float nu[U64];
+  const size_t total4 = (size_t)B * MLP_H / 4;
+  auto load = [&](uint32_t t) {
+#pragma unroll
+    for (int q = 0; q < V4; q++) {
+      const size_t at = (size_t)t * (WG_ROWS * MLP_H / 4) + q * 256u + threadIdx.x;
+      nx[q] = at < total4 ? reinterpret_cast<const float4 *>(Mx)[at] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int q = 0; q < U64; q++) nu[q] = u_of(t * WG_ROWS + q * 64u + lane);
+  };
+  auto store = [&](uint32_t buf) {
+#pragma unroll
+    for (int q = 0; q < V4; q++) reinterpret_cast<float4 *>(tile[buf])[q * 256u + threadIdx.x] = nx[q];
+#pragma unroll
+    for (int q = 0; q < U64; q++) ut[buf][wv][q * 64u + lane] = nu[q];
+  };
+  const uint32_t nt = (B + WG_ROWS - 1u) / WG_ROWS;
   float a = 0.0f;
-  if (p < 768) {  // W1[i][j] = sum dH1[b][i] X[b][j]
-    const uint32_t i = p / MLP_IN, j = p % MLP_IN;
-    for (uint32_t b = 0; b < B; b++) a = fmaf(dH1[(size_t)b * MLP_H + i], X[(size_t)b * MLP_IN + j], a);
-  } else if (p < 832) {  // b1
-    const uint32_t i = p - 768;
-    for (uint32_t b = 0; b < B; b++) a += dH1[(size_t)b * MLP_H + i];
-  } else if (p < 4928) {  // W2[i][j] = sum dH2[b][i] H1[b][j]
-    const uint32_t i = (p - 832) / MLP_H, j = (p - 832) % MLP_H;
-    for (uint32_t b = 0; b < B; b++) a = fmaf(dH2[(size_t)b * MLP_H + i], H1[(size_t)b * MLP_H + j], a);
-  } else if (p < 4992) {  // b2
-    const uint32_t i = p - 4928;
-    for (uint32_t b = 0; b < B; b++) a += dH2[(size_t)b * MLP_H + i];
-  } else if (p < 5056) {  // w3[i] = sum dout[b] H2[b][i]
-    const uint32_t i = p - 4992;
-    for (uint32_t b = 0; b < B; b++) a = fmaf(dout[b], H2[(size_t)b * MLP_H + i], a);
-  } else {  // b3
-    for (uint32_t b = 0; b < B; b++) a += dout[b];
+  load(0);
+  store(0);
+  __syncthreads();
+  for (uint32_t t = 0; t < nt; t++) {
+    const uint32_t cur = t & 1u;
+    if (t + 1u < nt) load(t + 1u);
+    const uint32_t rows = B - t * WG_ROWS < WG_ROWS ? B - t * WG_ROWS : WG_ROWS;
+    const float *m = tile[cur] + lane, *u = ut[cur][wv];
+    // one column's sums: b3 (u = dout) and the loss (u = the errors, squared)
+    const bool sq = k == 20u && wv == 2u, self = k == 20u && wv == 1u;
+    if (rows == WG_ROWS && !(sq | self)) {
+#pragma unroll 32
+      for (uint32_t r = 0; r < WG_ROWS; r++) a = fmaf(u[r], m[r * MLP_H], a);
+    } else if (rows == WG_ROWS) {
+#pragma unroll 32
+      for (uint32_t r = 0; r < WG_ROWS; r++) a = fmaf(u[r], sq ? u[r] : 1.0f, a);
+    } else {
+      for (uint32_t r = 0; r < rows; r++) a = fmaf(u[r], sq ? u[r] : (self ? 1.0f : m[r * MLP_H]), a);
+    }
+    if (t + 1u < nt) store(cur ^ 1u);
+    __syncthreads();
   }
-  G[p] = a;
-}
-
-// mean squared error of the batch, summed in sample order
-__global__ void k_mlp_loss(const float *out, const float *Y, uint32_t B, float *loss) {
-  if (threadIdx.x || blockIdx.x) return;
-  float s = 0.0f;
-  for (uint32_t b = 0; b < B; b++) {
-    const float e = out[b] - Y[b];
-    s = fmaf(e, e, s);
-  }
-  *loss = s / (float)B;
-}
-
-// Adam: m = b1 m + (1-b1) g, v = b2 v + (1-b2) g^2, w -= lr * (m / c1) / (sqrt(v / c2) + eps)
-__global__ void k_adam(float *W, const float *G, float *M, float *V, float lr, float b1, float b2,
-                       float c1, float c2, float eps) {
-  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+  uint32_t p = MLP_NW;
+  if (k < 16u) p = 832u + j * MLP_H + lane;
+  else if (k < 20u && j < MLP_IN) p = lane * MLP_IN + j;
+  else if (k < 20u && j == MLP_IN) p = 768u + lane;
+  else if (k == 20u && wv == 0u) p = 4992u + lane;
+  else if (k == 20u && wv == 1u && lane == 0u) p = 5056u;
+  else if (k == 21u && wv == 0u) p = 4928u + lane;
+  if (k == 20u && wv == 2u && lane == 0u && loss) *loss = a / (float)B;
   if (p >= MLP_NW) return;
-  const float g = G[p];
-  const float m = b1 * M[p] + (1.0f - b1) * g;
-  const float v = b2 * V[p] + (1.0f - b2) * (g * g);
-  M[p] = m;
-  V[p] = v;
-  W[p] = W[p] - lr * ((m / c1) / (sqrtf(v / c2) + eps));
+  if (G) G[p] = a;
+  if (ad.W) {
+    const float m = ad.b1 * ad.M[p] + (1.0f - ad.b1) * a;
+    const float v = ad.b2 * ad.V[p] + (1.0f - ad.b2) * (a * a);
+    ad.M[p] = m;
+    ad.V[p] = v;
+    ad.W[p] = ad.W[p] - ad.lr * ((m / ad.c1) / (sqrtf(v / ad.c2) + ad.eps));
+  }
 }
 
 }  // namespace
@@ -538,28 +643,19 @@ void max_failed_radius(const double *radius, const uint8_t *failed, uint32_t n, 
   fill_u32(reinterpret_cast<uint32_t *>(out), 0u, 2, s);
   if (n) k_max_radius_d<<<(n + 255) / 256, 256, 0, s>>>(radius, failed, n, reinterpret_cast<unsigned long long *>(out));
 }
-void gather_rows(const float *in, const uint32_t *idx, uint32_t B, uint32_t w, float *out, hipStream_t s) {
-  if (B) k_gather_rows<<<(B * w + 255) / 256, 256, 0, s>>>(in, idx, B, w, out);
-}
-
 void mlp_forward_batch(const float *W, const float *X, uint32_t B, float *H1, float *H2, float *out,
                        hipStream_t s) {
   if (B) k_mlp_fwd<<<(B + 127) / 128, 128, 0, s>>>(W, X, B, H1, H2, out);
 }
 
-void mlp_grad_batch(const float *W, const float *X, const float *Y, uint32_t B, float *H1,
-                    float *H2, float *out, float *dout, float *dH1, float *dH2, float *G,
-                    float *loss, hipStream_t s) {
+void mlp_step(const float *W, const float *X, const float *Y, const uint32_t *idx, uint32_t B, float *Xb,
+              float *err, float *H1, float *H2, float *dout, float *dH1, float *dH2, float *G, float *loss,
+              const AdamStep *step, hipStream_t s) {
   if (!B) return;
-  k_mlp_fwd<<<(B + 127) / 128, 128, 0, s>>>(W, X, B, H1, H2, out);
-  k_mlp_bwd_samples<<<(B + 127) / 128, 128, 0, s>>>(W, Y, B, H1, H2, out, dout, dH1, dH2);
-  k_mlp_wgrad<<<(MLP_NW + 63) / 64, 64, 0, s>>>(X, B, H1, H2, dout, dH1, dH2, G);
-  if (loss) k_mlp_loss<<<1, 64, 0, s>>>(out, Y, B, loss);
-}
-
-void adam_step(float *W, const float *G, float *M, float *V, float lr, float b1, float b2, float c1,
-               float c2, float eps, hipStream_t s) {
-  k_adam<<<(MLP_NW + 255) / 256, 256, 0, s>>>(W, G, M, V, lr, b1, b2, c1, c2, eps);
+  k_mlp_fb<<<(B + 4 * FB_S - 1) / (4 * FB_S), 256, 0, s>>>(W, X, Y, idx, B, Xb, err, H1, H2, dout, dH1, dH2);
+  AdamArgs ad{};
+  if (step) ad = AdamArgs{step->W, step->M, step->V, step->lr, step->b1, step->b2, step->c1, step->c2, step->eps};
+  k_mlp_wgrad<<<WG_BLOCKS, 256, 0, s>>>(Xb, err, B, H1, H2, dout, dH1, dH2, G, loss, ad);
 }
 
 #define INST(T)                                                                                   \

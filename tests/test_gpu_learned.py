@@ -132,3 +132,18 @@ def test_trained_model_gains_over_plain_schedule(oracle):
     # the gain: fewer passes and fewer (query, candidate) evaluations than the BETA schedule
     assert st_l.iterations < st_p.iterations
     assert st_l.candidates < st_p.candidates
+
+
+@pytest.mark.parametrize("n,batch", [(255, 255), (256, 256), (257, 257), (1000, 513), (15, 7)])
+def test_training_step_at_tile_edges(oracle, n, batch):
+    # the gradient kernel's sample tiles (256) and the forward kernel's blocks (16): whole tiles,
+    # one sample more or less, and a last batch that the epoch drops
+    rng = np.random.default_rng(n)
+    W0 = learned_radius.init_weights(n)
+    X = rng.normal(0, 1, (n, 12)).astype(np.float32)
+    Y = rng.normal(0, 1, n).astype(np.float32)
+    g, loss = _lib.mlp_grad(W0, X, Y)
+    g2, loss2 = oracle.mlp_grad(W0, X, Y)
+    assert np.array_equal(bits(g), bits(g2)) and loss == loss2
+    w, _ = _lib.mlp_train(W0, X, Y, epochs=2, batch=batch, lr=1e-3, seed=7)
+    assert np.array_equal(bits(w), bits(oracle.mlp_train(W0, X, Y, 2, batch, 1e-3, 7)))
