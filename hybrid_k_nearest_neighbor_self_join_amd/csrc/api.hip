@@ -2208,12 +2208,12 @@ struct BatchGroup {
            *idsTmp = nullptr, *cflags = nullptr, *cpos = nullptr, *cellStart = nullptr,
            *dense = nullptr, *aflags = nullptr, *apos = nullptr, *act = nullptr,
            *ntiles = nullptr, *tileOff = nullptr, *scratch = nullptr, *status = nullptr,
-           *setMaxBits = nullptr, *ctr = nullptr;
+           *ctr = nullptr;
   uint64_t *cellKeys = nullptr;
   unsigned long long *cand = nullptr;
   uint4 *tiles = nullptr;
-  uint8_t *failed = nullptr, *overflow = nullptr, *bin = nullptr, *actq = nullptr;
-  uint32_t *setMinBin = nullptr;
+  uint8_t *failed = nullptr, *overflow = nullptr, *bin = nullptr;
+  uint32_t *setMinBin = nullptr, *setClass = nullptr, *chunkOff = nullptr;
   SetDesc *sets = nullptr;
   int32_t *outIds = nullptr;
   void *heap = nullptr;
@@ -2348,14 +2348,14 @@ static void batch_build(BatchPlan &B, uint32_t nsets, const uint32_t *n, const u
     G.tiles = B.alloc<uint4>((size_t)N + 1);
     G.scratch = B.alloc<uint32_t>(sw);
     G.status = B.alloc<uint32_t>(4);
-    G.setMaxBits = B.alloc<uint32_t>(G.nsets);
     G.ctr = B.alloc<uint32_t>(8 + TILE_QUEUES);  // [8..]: the tile queue heads
     G.cand = B.alloc<unsigned long long>(4);
     G.failed = B.alloc<uint8_t>(N);
     G.overflow = B.alloc<uint8_t>(N);
     G.bin = B.alloc<uint8_t>(N);
-    G.actq = B.alloc<uint8_t>(N);
     G.setMinBin = B.alloc<uint32_t>(G.nsets);
+    G.setClass = B.alloc<uint32_t>(G.nsets);
+    G.chunkOff = B.alloc<uint32_t>((size_t)G.nsets + 1);
     G.sets = B.alloc<SetDesc>(G.nsets);
     G.outIds = B.alloc<int32_t>(G.outElems);
     G.outDists = B.alloc<float>(G.outElems);
@@ -2404,11 +2404,11 @@ static JoinArgs batch_args(const BatchPlan &B, const BatchGroup &G) {
   return a;
 }
 
-// Index of a group at the sets' current widths: per-set grids, cell keys, radix sort, cell
+// Index of a group at the sets' current widths (classes: those of their lowest pending radius class): per-set grids, cell keys, radix sort, cell
 // table, cell-sorted coordinates, dense cell-start table.
-static void batch_index(BatchGroup &G, hipStream_t s) {
+static void batch_index(BatchGroup &G, bool classes, hipStream_t s) {
   const uint32_t N = G.N;
-  batch_grids(G.sets, G.nsets, G.mnmx, G.width, G.bound, G.status, s);
+  batch_grids(G.sets, G.nsets, G.mnmx, G.width, G.bound, G.status, classes ? G.setMinBin : nullptr, G.setClass, s);
   batch_cell_keys(G.x, N, G.sets, G.setOf, G.keys, G.ids, s);
   radix_sort_pairs_u32(G.keys, G.ids, G.keysTmp, G.idsTmp, N, G.bits, G.scratch, s);
   boundary_flags_u32(G.keys, N, 0u, G.cflags, s);
@@ -2420,44 +2420,56 @@ static void batch_index(BatchGroup &G, hipStream_t s) {
   scan_exclusive_u32(G.dense, G.dense, (uint32_t)G.bound, G.scratch, s);
 }
 
-// One radius pass of a group: every set's lowest pending octave, grids matched to it, tiles of
-// those queries, the direct kernel, the collect kernel for its overflows, and radius growth of the queries that failed; G.ctr[3] = queries
-// still pending.
+// The queries the range kernel of a pass could not list, on the overflow kernel, and the radius
+// growth of those that failed there.
+static void batch_overflow(const BatchPlan &B, BatchGroup &G, const JoinArgs &a, const GridParams &g0, hipStream_t s) {
+  const uint32_t N = G.N;
+  batch_flags_u8(G.ids, G.overflow, N, G.aflags, s);
+  scan_exclusive_u32(G.aflags, G.apos, N, G.scratch, s);
+  compact_active(G.ids, G.aflags, G.apos, N, G.act, s);
+  batch_tiles(G.cellStart, G.apos, G.cpos + N, N, std::min(B.tq, 16u), G.ntiles, G.tileOff, G.scratch, G.tiles, s);
+  fill_u32(G.ctr + 8, 0u, TILE_QUEUES, s);
+  if (overflow_by_collect(G.k1max))
+    range_collect<float>(a, g0, s);
+  else
+    range_topk<float>(a, g0, s);
+  fill_u32(G.ctr + 3, 0u, 1, s);
+  fill_u32(G.setMinBin, 64u, G.nsets, s);
+  batch_grow_class(G.sets, G.setOf, G.setClass, g0.nd, G.failed, G.overflow, true, N, G.radius, G.bin, G.ctr + 3,
+                   G.setMinBin, s);
+}
+
+// One radius pass of a group: every set's lowest pending class, grids matched to it, tiles of
+// those queries, the range kernel, the overflow kernel for what it could not list, and radius
+// growth of the queries that failed; G.ctr[3] = queries still pending.
 static void batch_pass(const BatchPlan &B, BatchGroup &G, hipStream_t s) {
   const uint32_t N = G.N;
-  batch_class(G.sets, G.nsets, G.setOf, G.failed, G.bin, N, G.setMinBin, G.width, G.actq, s);
-  batch_index(G, s);
+  batch_index(G, true, s);
 
   const JoinArgs a = batch_args(B, G);
   // every tile takes its set's grid; g0 carries only the group's number of indexed dims (one
   // per group: it depends on the dimensionality alone), which picks the kernel build
   GridParams g0{};
   g0.nd = G.hsets.empty() ? 0u : G.hsets[0].nd;
-  batch_flags_u8(G.ids, G.actq, N, G.aflags, s);
+  batch_class_flags(G.ids, G.setOf, G.failed, G.bin, G.setClass, g0.nd, N, G.aflags, s);
   scan_exclusive_u32(G.aflags, G.apos, N, G.scratch, s);
   compact_active(G.ids, G.aflags, G.apos, N, G.act, s);
-  batch_tiles(G.cellStart, G.apos, G.cpos + N, N, B.tq, G.ntiles, G.tileOff, G.scratch, G.tiles, s);
   fill_u32(G.ctr, 0u, 8 + TILE_QUEUES, s);
   const RangeKernel rk = range_kernel(G.k1max);
-  if (rk == RK_DIRECT)
+  if (rk == RK_DIRECT) {
+    batch_chunks(G.sets, G.nsets, g0.nd, G.apos, N, B.grid, B.tq, G.chunkOff, G.tileOff + N + 1, G.ctr + 4, G.tiles,
+                 s);
     range_direct<float>(a, g0, s);
-  else if (rk == RK_COLLECT)
-    range_collect<float>(a, g0, s);
-  else
-    range_topk<float>(a, g0, s);
-
-  batch_flags_u8(G.ids, G.overflow, N, G.aflags, s);
-  scan_exclusive_u32(G.aflags, G.apos, N, G.scratch, s);
-  compact_active(G.ids, G.aflags, G.apos, N, G.act, s);
-  batch_tiles(G.cellStart, G.apos, G.cpos + N, N, B.tq, G.ntiles, G.tileOff, G.scratch, G.tiles, s);
-  fill_u32(G.ctr + 8, 0u, TILE_QUEUES, s);
-  if (overflow_by_collect(G.k1max))
-    range_collect<float>(a, g0, s);
-  else
-    range_topk<float>(a, g0, s);
-  fill_u8(G.overflow, 0, N, s);
-
-  batch_grow_class(G.sets, G.setOf, G.actq, G.failed, N, G.radius, G.bin, G.ctr + 3, s);
+  } else {
+    batch_tiles(G.cellStart, G.apos, G.cpos + N, N, B.tq, G.ntiles, G.tileOff, G.scratch, G.tiles, s);
+    if (rk == RK_COLLECT)
+      range_collect<float>(a, g0, s);
+    else
+      range_topk<float>(a, g0, s);
+  }
+  batch_grow_class(G.sets, G.setOf, G.setClass, g0.nd, G.failed, G.overflow, false, N, G.radius, G.bin, G.ctr + 3,
+                   G.setMinBin, s);
+  batch_overflow(B, G, a, g0, s);
 }
 
 static void batch_body(const BatchPlan &B, hipStream_t s) {
@@ -2465,11 +2477,11 @@ static void batch_body(const BatchPlan &B, hipStream_t s) {
     batch_variance_perm(G.xin, G.sets, G.nsets, G.d, B.reorder, G.var, G.perm, s);
     batch_permute(G.xin, G.N, G.d, G.setOf, G.perm, G.x, s);
     batch_minmax(G.x, G.N, G.sets, G.nsets, G.mnmx, s);
-    batch_init_width(G.sets, G.nsets, G.mnmx, G.width, G.N, G.failed, s);
+    batch_init_width(G.sets, G.nsets, G.mnmx, G.width, G.setMinBin, G.N, G.failed, s);
     fill_u8(G.overflow, 0, G.N, s);
     fill_u32(reinterpret_cast<uint32_t *>(G.cand), 0u, 8, s);
-    batch_index(G, s);
-    batch_density_radius(G.x, G.N, G.sets, G.setOf, G.dense, G.radius, G.bin, s);
+    batch_index(G, false, s);
+    batch_density_radius(G.x, G.N, G.sets, G.setOf, G.dense, G.radius, G.bin, G.setMinBin, s);
     for (uint32_t p = 0; p < B.passes; p++) batch_pass(B, G, s);
   }
 }
@@ -2497,10 +2509,14 @@ static int run_batched(uint32_t nsets, const float *const *points, const uint32_
     if (!tq) tq = g_tunedTq;
     if (!grid) grid = g_tunedGrid;
   }
-  // defaults: the best pair of the autotuner's sweep on the 256-set mix of 2-6 dims (the 6-D
-  // group on the collect kernel favours small tiles and a wide grid: 79 ms against 131 ms at
-  // 64 x 2048; the other groups change by under 5 %)
-  if (!tq) tq = 16;
+  // defaults: whole chunks of 64 queries for the direct kernel, which looks all their rows up at
+  // once; 16-query tiles of one cell for the collect kernel
+  if (!tq) {
+    uint32_t k1max = 0;
+    for (uint32_t i = 0; i < nsets; i++)
+      if (n[i]) k1max = std::max(k1max, k[i] + 1);
+    tq = range_kernel(k1max) == RK_DIRECT ? 64u : 16u;
+  }
   if (!grid) grid = 4096;
   if (tq > 64) throw Error(KNN_ERR_ARG, "tile_queries must be <= 64");
   if (grid > kBatchMaxGrid) throw Error(KNN_ERR_ARG, "grid_blocks must be <= 8192");

@@ -234,20 +234,21 @@ void batch_permute(const float *xin, uint32_t N, uint32_t d, const uint32_t *set
                    float *x, hipStream_t s);
 void batch_minmax(const float *x, uint32_t N, const SetDesc *sets, uint32_t nsets, float *mnmx,
                   hipStream_t s);
-void batch_init_width(SetDesc *sets, uint32_t nsets, const float *mnmx, float *width, uint32_t N,
-                      uint8_t *failed, hipStream_t s);
-// initial per-query radius from the density around each query on the wf grid (dense table of
-// the current index); bin = quarter-octave of radius / wf
+void batch_init_width(SetDesc *sets, uint32_t nsets, const float *mnmx, float *width, uint32_t *setMinBin,
+                      uint32_t N, uint8_t *failed, hipStream_t s);
+// initial radii from local densities, and each set's lowest radius bin
 void batch_density_radius(const float *x, uint32_t N, const SetDesc *sets, const uint32_t *setOf,
-                          const uint32_t *dense, float *radius, uint8_t *bin, hipStream_t s);
-// per set: lowest pending octave, the pass's grid width, and the pass's active flags
-void batch_class(const SetDesc *sets, uint32_t nsets, const uint32_t *setOf, const uint8_t *failed,
-                 const uint8_t *bin, uint32_t N, uint32_t *setMinBin, float *width, uint8_t *act, hipStream_t s);
-// radius * 2 for the pass's failed queries; *pending = queries still pending
-void batch_grow_class(const SetDesc *sets, const uint32_t *setOf, const uint8_t *act, const uint8_t *failed,
-                      uint32_t N, float *radius, uint8_t *bin, uint32_t *pending, hipStream_t s);
+                          const uint32_t *dense, float *radius, uint8_t *bin, uint32_t *setMinBin, hipStream_t s);
+// the pass's queries, by sorted position: pending, with a radius bin in their set's class
+void batch_class_flags(const uint32_t *sortedIds, const uint32_t *setOf, const uint8_t *failed, const uint8_t *bin,
+                       const uint32_t *setClass, uint32_t nd, uint32_t N, uint32_t *aflags, hipStream_t s);
+// radius growth of the pass's failed queries (over: of those the overflow kernel took)
+void batch_grow_class(const SetDesc *sets, const uint32_t *setOf, const uint32_t *setClass, uint32_t nd,
+                      const uint8_t *failed, uint8_t *overflow, bool over, uint32_t N, float *radius, uint8_t *bin,
+                      uint32_t *pending, uint32_t *setMinBin, hipStream_t s);
+// per-set radius classes (with setMinBin) and grids
 void batch_grids(SetDesc *sets, uint32_t nsets, const float *mnmx, float *width, uint64_t bound,
-                 uint32_t *status, hipStream_t s);
+                 uint32_t *status, uint32_t *setMinBin, uint32_t *setClass, hipStream_t s);
 void batch_cell_keys(const float *x, uint32_t N, const SetDesc *sets, const uint32_t *setOf,
                      uint32_t *keys, uint32_t *ids, hipStream_t s);
 void batch_dense_counts(const uint64_t *cellKeys, const uint32_t *cellStart, const uint32_t *ncell,
@@ -258,6 +259,9 @@ void batch_flags_u8(const uint32_t *sortedIds, const uint8_t *f, uint32_t N, uin
 void batch_tiles(const uint32_t *cellStart, const uint32_t *pos, const uint32_t *ncell, uint32_t N,
                  uint32_t tq, uint32_t *ntiles, uint32_t *tileOff, uint32_t *scratch, uint4 *tiles,
                  hipStream_t s);
+// direct-kernel tiles: chunks of consecutive active queries of one set
+void batch_chunks(const SetDesc *sets, uint32_t nsets, uint32_t nd, const uint32_t *pos, uint32_t N, uint32_t waves, uint32_t cap,
+                  uint32_t *chunkOff, uint32_t *ntiles, uint32_t *q, uint4 *tiles, hipStream_t s);
 
 
 // ------------------------------------------------------------- outlier scores (outlier.hip)

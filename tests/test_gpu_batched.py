@@ -157,3 +157,23 @@ def test_batched_new_set_shapes_after_graph_replays():
     ids, dists, st = batched.knnjoin_batched(pa, ka)
     assert st.graph_replayed == 0
     _check_against_single(a, ids, dists)
+
+
+@pytest.mark.parametrize("nsets,d", [(1, 2), (65, 2), (64, 3), (300, 1), (259, 6)])
+def test_batched_set_boundaries(nsets, d, oracle):
+    # sets from K+1 points up, more of them than a block's and a wave's lanes, with a set of
+    # equal points longer than the direct kernel's list and one far denser than the others (in
+    # 6-D the single-set join refuses that one's grid: the rows are compared with brute force)
+    rng = np.random.default_rng(100 * nsets + d)
+    ks = [int(k) for k in rng.choice((1, 8, 40), nsets)]
+    pts = [rng.random((k + 1 + int(rng.integers(0, 150)), d)).astype(np.float32) for k in ks]
+    pts[nsets // 2] = np.concatenate([np.full((3000, d), 0.25, np.float32), pts[nsets // 2]])
+    pts[-1] = np.concatenate([pts[-1], (pts[-1][:1] + 1e-4 * rng.random((4097, d))).astype(np.float32)])
+    for graph in (False, True):
+        ids, dists, _ = batched.knnjoin_batched(pts, ks, use_graph=graph)
+        for i, (p_, k) in enumerate(zip(pts, ks)):
+            q = np.random.default_rng(i).choice(len(p_), min(300, len(p_)), replace=False)
+            perm, _ = oracle.reorder(p_)
+            bi, bd = oracle.bruteforce(np.ascontiguousarray(p_[:, perm]), k, queries=q)
+            assert np.array_equal(ids[i][q], bi), f"set {i}: n={len(p_)} k={k} graph={graph}"
+            assert np.array_equal(bits(dists[i][q]), bits(bd)), f"set {i}"
