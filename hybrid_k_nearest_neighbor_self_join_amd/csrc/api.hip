@@ -2193,8 +2193,19 @@ int knnjoin_mlp_train(float *weights, const float *X, const float *Y, uint32_t n
 
 // ================================================================== batched sets
 // Host side of batched.hip: a plan per set-shape signature (allocations, descriptors, and the
-// captured hipGraph of the whole join), replayed while the caller's shapes stay the same.
+// captured hipGraphs of every group's passes), replayed while the caller's shapes stay the same.
+//
+// A group's pass is some fifty short kernels around one that fills the chip, so the groups run
+// on streams of their own and fill each other's gaps, and after each pass the host reads how many
+// queries of the group are pending and could not be listed: a pass or an overflow kernel that has
+// nothing to do is not launched.  48 sets in 4 groups (21.6 ms in one graph of 8 passes on one
+// stream, half of it small kernels and their gaps): 13.6 ms.
 namespace knn {
+
+struct BatchGraph {
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec = nullptr;
+};
 
 struct BatchGroup {
   uint32_t d = 0, nsets = 0, N = 0, k1max = 0;
@@ -2217,14 +2228,17 @@ struct BatchGroup {
   SetDesc *sets = nullptr;
   int32_t *outIds = nullptr;
   void *heap = nullptr;
+  hipStream_t stream = nullptr;
+  BatchGraph gStart, gPass, gOver;  // set-up and first pass; one pass; the overflow kernel's part
+  uint32_t passesRun = 0;           // of the current call
 };
 
 struct BatchPlan {
   std::vector<uint64_t> sig;
   std::vector<BatchGroup> groups;
   std::vector<void *> allocs;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
+  uint32_t *pin = nullptr;  // pinned, 2 words per group: overflowed and pending queries of a pass
+  bool captured = false;
   uint32_t tq = 64, grid = 2048, passes = 3;
   int reorder = 1;
   bool useGraph = true;
@@ -2235,25 +2249,38 @@ struct BatchPlan {
     allocs.push_back(p);
     return reinterpret_cast<U *>(p);
   }
-  // The graph's kernel nodes hold pointers into `allocs`: it is destroyed first, and only
-  // once the device has finished every launch of it, then the buffers are freed.
-  void drop_graph() {
-    if (exec || graph) HIP_CHECK(hipDeviceSynchronize());
-    hipGraphExec_t e = exec;
-    hipGraph_t g = graph;
-    exec = nullptr;
-    graph = nullptr;
-    if (e) HIP_CHECK(hipGraphExecDestroy(e));
-    if (g) HIP_CHECK(hipGraphDestroy(g));
+  // The graphs' kernel nodes hold pointers into `allocs`: they are destroyed first, and only
+  // once the device has finished every launch of them, then the buffers are freed.
+  void drop_graphs() {
+    bool any = false;
+    for (BatchGroup &G : groups)
+      for (BatchGraph *b : {&G.gStart, &G.gPass, &G.gOver}) any |= b->exec || b->graph;
+    captured = false;
+    if (!any) return;
+    HIP_CHECK(hipDeviceSynchronize());
+    for (BatchGroup &G : groups)
+      for (BatchGraph *b : {&G.gStart, &G.gPass, &G.gOver}) {
+        const BatchGraph t = *b;
+        *b = BatchGraph{};
+        if (t.exec) HIP_CHECK(hipGraphExecDestroy(t.exec));
+        if (t.graph) HIP_CHECK(hipGraphDestroy(t.graph));
+      }
   }
   void free_all() {
-    drop_graph();
-    if (!allocs.empty()) HIP_CHECK(hipDeviceSynchronize());
+    drop_graphs();
+    if (!allocs.empty() || pin) HIP_CHECK(hipDeviceSynchronize());
     std::vector<void *> a;
     a.swap(allocs);
+    std::vector<hipStream_t> st;
+    for (BatchGroup &G : groups)
+      if (G.stream) st.push_back(G.stream);
     groups.clear();
     sig.clear();
+    uint32_t *p0 = pin;
+    pin = nullptr;
     for (void *p : a) HIP_CHECK(hipFree(p));
+    for (hipStream_t s : st) HIP_CHECK(hipStreamDestroy(s));
+    if (p0) HIP_CHECK(hipHostFree(p0));
   }
 };
 
@@ -2314,7 +2341,10 @@ static void batch_build(BatchPlan &B, uint32_t nsets, const uint32_t *n, const u
     G.hsets.push_back(sd);
     G.members.push_back(si);
   }
+  if (!B.groups.empty())
+    HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&B.pin), sizeof(uint32_t) * 2 * B.groups.size(), hipHostMallocDefault));
   for (BatchGroup &G : B.groups) {
+    HIP_CHECK(hipStreamCreateWithFlags(&G.stream, hipStreamNonBlocking));
     G.nsets = (uint32_t)G.hsets.size();
     const uint32_t N = G.N, d = G.d;
     G.bound = std::min<uint64_t>(1ull << 27, std::max<uint64_t>(1ull << 16, 8ull * N));
@@ -2420,37 +2450,18 @@ static void batch_index(BatchGroup &G, bool classes, hipStream_t s) {
   scan_exclusive_u32(G.dense, G.dense, (uint32_t)G.bound, G.scratch, s);
 }
 
-// The queries the range kernel of a pass could not list, on the overflow kernel, and the radius
-// growth of those that failed there.
-static void batch_overflow(const BatchPlan &B, BatchGroup &G, const JoinArgs &a, const GridParams &g0, hipStream_t s) {
-  const uint32_t N = G.N;
-  batch_flags_u8(G.ids, G.overflow, N, G.aflags, s);
-  scan_exclusive_u32(G.aflags, G.apos, N, G.scratch, s);
-  compact_active(G.ids, G.aflags, G.apos, N, G.act, s);
-  batch_tiles(G.cellStart, G.apos, G.cpos + N, N, std::min(B.tq, 16u), G.ntiles, G.tileOff, G.scratch, G.tiles, s);
-  fill_u32(G.ctr + 8, 0u, TILE_QUEUES, s);
-  if (overflow_by_collect(G.k1max))
-    range_collect<float>(a, g0, s);
-  else
-    range_topk<float>(a, g0, s);
-  fill_u32(G.ctr + 3, 0u, 1, s);
-  fill_u32(G.setMinBin, 64u, G.nsets, s);
-  batch_grow_class(G.sets, G.setOf, G.setClass, g0.nd, G.failed, G.overflow, true, N, G.radius, G.bin, G.ctr + 3,
-                   G.setMinBin, s);
-}
-
 // One radius pass of a group: every set's lowest pending class, grids matched to it, tiles of
-// those queries, the range kernel, the overflow kernel for what it could not list, and radius
-// growth of the queries that failed; G.ctr[3] = queries still pending.
+// those queries, the range kernel, and radius growth of the queries that failed.  G.ctr[2] =
+// queries the kernel could not list (left to batch_overflow), G.ctr[3] = queries still pending,
+// those included.  Every tile takes its set's grid; g0 carries only the group's number of indexed
+// dims (one per group: it depends on the dimensionality alone), which picks the kernel build.
 static void batch_pass(const BatchPlan &B, BatchGroup &G, hipStream_t s) {
   const uint32_t N = G.N;
   batch_index(G, true, s);
 
   const JoinArgs a = batch_args(B, G);
-  // every tile takes its set's grid; g0 carries only the group's number of indexed dims (one
-  // per group: it depends on the dimensionality alone), which picks the kernel build
   GridParams g0{};
-  g0.nd = G.hsets.empty() ? 0u : G.hsets[0].nd;
+  g0.nd = G.hsets[0].nd;
   batch_class_flags(G.ids, G.setOf, G.failed, G.bin, G.setClass, g0.nd, N, G.aflags, s);
   scan_exclusive_u32(G.aflags, G.apos, N, G.scratch, s);
   compact_active(G.ids, G.aflags, G.apos, N, G.act, s);
@@ -2469,22 +2480,64 @@ static void batch_pass(const BatchPlan &B, BatchGroup &G, hipStream_t s) {
   }
   batch_grow_class(G.sets, G.setOf, G.setClass, g0.nd, G.failed, G.overflow, false, N, G.radius, G.bin, G.ctr + 3,
                    G.setMinBin, s);
-  batch_overflow(B, G, a, g0, s);
 }
 
-static void batch_body(const BatchPlan &B, hipStream_t s) {
-  for (BatchGroup &G : const_cast<BatchPlan &>(B).groups) {
-    batch_variance_perm(G.xin, G.sets, G.nsets, G.d, B.reorder, G.var, G.perm, s);
-    batch_permute(G.xin, G.N, G.d, G.setOf, G.perm, G.x, s);
-    batch_minmax(G.x, G.N, G.sets, G.nsets, G.mnmx, s);
-    batch_init_width(G.sets, G.nsets, G.mnmx, G.width, G.setMinBin, G.N, G.failed, s);
-    fill_u8(G.overflow, 0, G.N, s);
-    fill_u32(reinterpret_cast<uint32_t *>(G.cand), 0u, 8, s);
-    batch_index(G, false, s);
-    batch_density_radius(G.x, G.N, G.sets, G.setOf, G.dense, G.radius, G.bin, G.setMinBin, s);
-    for (uint32_t p = 0; p < B.passes; p++) batch_pass(B, G, s);
-  }
+// The queries the range kernel of the last pass could not list, on the overflow kernel, and the
+// radius growth of those that failed there; G.ctr[3] = queries still pending.
+static void batch_overflow(const BatchPlan &B, BatchGroup &G, hipStream_t s) {
+  const uint32_t N = G.N;
+  const JoinArgs a = batch_args(B, G);
+  GridParams g0{};
+  g0.nd = G.hsets[0].nd;
+  batch_flags_u8(G.ids, G.overflow, N, G.aflags, s);
+  scan_exclusive_u32(G.aflags, G.apos, N, G.scratch, s);
+  compact_active(G.ids, G.aflags, G.apos, N, G.act, s);
+  batch_tiles(G.cellStart, G.apos, G.cpos + N, N, std::min(B.tq, 16u), G.ntiles, G.tileOff, G.scratch, G.tiles, s);
+  fill_u32(G.ctr + 8, 0u, TILE_QUEUES, s);
+  if (overflow_by_collect(G.k1max))
+    range_collect<float>(a, g0, s);
+  else
+    range_topk<float>(a, g0, s);
+  fill_u32(G.ctr + 3, 0u, 1, s);
+  fill_u32(G.setMinBin, 64u, G.nsets, s);
+  batch_grow_class(G.sets, G.setOf, G.setClass, g0.nd, G.failed, G.overflow, true, N, G.radius, G.bin, G.ctr + 3,
+                   G.setMinBin, s);
 }
+
+static void batch_start(const BatchPlan &B, BatchGroup &G, hipStream_t s) {
+  batch_variance_perm(G.xin, G.sets, G.nsets, G.d, B.reorder, G.var, G.perm, s);
+  batch_permute(G.xin, G.N, G.d, G.setOf, G.perm, G.x, s);
+  batch_minmax(G.x, G.N, G.sets, G.nsets, G.mnmx, s);
+  batch_init_width(G.sets, G.nsets, G.mnmx, G.width, G.setMinBin, G.N, G.failed, s);
+  fill_u8(G.overflow, 0, G.N, s);
+  fill_u32(reinterpret_cast<uint32_t *>(G.cand), 0u, 8, s);
+  batch_index(G, false, s);
+  batch_density_radius(G.x, G.N, G.sets, G.setOf, G.dense, G.radius, G.bin, G.setMinBin, s);
+  batch_pass(B, G, s);
+}
+
+template <typename F>
+static void batch_capture(BatchGraph &b, hipStream_t s, F &&body) {
+  HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+  {
+    CaptureGuard cap(s);
+    body();
+    b.graph = cap.end();
+  }
+  hipGraphExec_t ex = nullptr;
+  HIP_CHECK(hipGraphInstantiate(&ex, b.graph, nullptr, nullptr, 0));
+  b.exec = ex;
+}
+
+// Waits for every group's stream when a call ends, also by an exception: the next call copies
+// its inputs into the buffers that the launches of this one read.
+struct BatchDrain {
+  BatchPlan &B;
+  ~BatchDrain() {
+    for (BatchGroup &G : B.groups)
+      if (G.stream) (void)hipStreamSynchronize(G.stream);
+  }
+};
 
 static int run_batched(uint32_t nsets, const float *const *points, const uint32_t *n,
                        const uint32_t *ndim, const uint32_t *k, const knnjoin_batch_params &p,
@@ -2533,68 +2586,85 @@ static int run_batched(uint32_t nsets, const float *const *points, const uint32_
   }
   if (B.tq != tq || B.grid != grid || B.passes != passes || B.reorder != (p.reorder ? 1 : 0) ||
       B.useGraph != (p.use_graph != 0)) {
-    B.drop_graph();
+    B.drop_graphs();
     B.tq = tq;
     B.grid = grid;
     B.passes = passes;
     B.reorder = p.reorder ? 1 : 0;
     B.useGraph = p.use_graph != 0;
   }
-  // inputs
+  BatchDrain drain{B};
+  // inputs, on the groups' streams
   const hipMemcpyKind kin = p.device_ptrs ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
   for (BatchGroup &G : B.groups)
     for (uint32_t i = 0; i < G.nsets; i++) {
       const uint32_t si = G.members[i];
       if (!points[si]) throw Error(KNN_ERR_ARG, "null set pointer");
       HIP_CHECK(hipMemcpyAsync(G.xin + (size_t)G.hsets[i].pStart * G.d, points[si],
-                               sizeof(float) * (size_t)n[si] * G.d, kin, s));
+                               sizeof(float) * (size_t)n[si] * G.d, kin, G.stream));
     }
   bool replay = false;
-  if (B.useGraph && !B.exec) {
-    HIP_CHECK(hipStreamSynchronize(s));
-    HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    {
-      CaptureGuard cap(s);
-      batch_body(B, s);
-      B.graph = cap.end();
+  for (BatchGroup &G : B.groups) HIP_CHECK(hipStreamSynchronize(G.stream));
+  if (B.useGraph && !B.captured) {
+    B.drop_graphs();  // (what an interrupted capture left)
+    for (BatchGroup &G : B.groups) {
+      batch_capture(G.gStart, G.stream, [&]() { batch_start(B, G, G.stream); });
+      batch_capture(G.gPass, G.stream, [&]() { batch_pass(B, G, G.stream); });
+      batch_capture(G.gOver, G.stream, [&]() { batch_overflow(B, G, G.stream); });
     }
-    hipGraphExec_t ex = nullptr;
-    HIP_CHECK(hipGraphInstantiate(&ex, B.graph, nullptr, nullptr, 0));
-    B.exec = ex;
+    B.captured = true;
   } else if (B.useGraph) {
     replay = true;
   }
-  HIP_CHECK(hipStreamSynchronize(s));
   stats.ms_setup = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - w0).count();
   tAll.start();
-  if (B.useGraph) {
-    HIP_CHECK(hipGraphLaunch(B.exec, s));
-  } else {
-    batch_body(B, s);
-    LAUNCH_CHECK();
-  }
-  // leftover failures: eager passes until none remain
-  uint32_t eager = 0;
-  for (;;) {
-    bool any = false;
-    for (BatchGroup &G : B.groups) {
-      uint32_t f = 0;  // queries still pending after the last pass
-      HIP_CHECK(hipMemcpyAsync(&f, G.ctr + 3, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-      HIP_CHECK(hipStreamSynchronize(s));
-      if (f) {
-        any = true;
-        batch_pass(B, G, s);
-        LAUNCH_CHECK();
-      }
+  // A group's passes: the first `passes` from its graphs, then (rare) eager ones until none of
+  // its queries is pending.  The groups' launches are all in flight; the host waits for them in
+  // turn.
+  auto launch = [&](BatchGroup &G, uint32_t gi, const BatchGraph &graph,
+                    void (*body)(const BatchPlan &, BatchGroup &, hipStream_t)) {
+    if (B.useGraph && G.passesRun < B.passes) {
+      HIP_CHECK(hipGraphLaunch(graph.exec, G.stream));
+    } else {
+      body(B, G, G.stream);
+      LAUNCH_CHECK();
     }
-    if (!any) break;
-    if (++eager > 200) throw Error(KNN_ERR_NO_PROGRESS, "batched join: queries still failing after 200 extra passes");
+    HIP_CHECK(hipMemcpyAsync(B.pin + 2 * gi, G.ctr + 2, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, G.stream));
+  };
+  std::vector<uint32_t> live;
+  for (uint32_t gi = 0; gi < B.groups.size(); gi++) {
+    BatchGroup &G = B.groups[gi];
+    G.passesRun = 0;
+    launch(G, gi, G.gStart, batch_start);
+    live.push_back(gi);
+  }
+  uint32_t eager = 0;
+  while (!live.empty()) {
+    std::vector<uint32_t> next;
+    for (uint32_t gi : live) {
+      BatchGroup &G = B.groups[gi];
+      HIP_CHECK(hipStreamSynchronize(G.stream));
+      if (B.pin[2 * gi]) {
+        launch(G, gi, G.gOver, batch_overflow);
+        HIP_CHECK(hipStreamSynchronize(G.stream));
+      }
+      G.passesRun++;
+      if (!B.pin[2 * gi + 1]) continue;
+      if (G.passesRun >= B.passes) {
+        if (G.passesRun - B.passes >= 200)
+          throw Error(KNN_ERR_NO_PROGRESS, "batched join: queries still failing after 200 extra passes");
+        eager = std::max(eager, G.passesRun - B.passes + 1);
+      }
+      launch(G, gi, G.gPass, batch_pass);
+      next.push_back(gi);
+    }
+    live.swap(next);
   }
   stats.ms_device = tAll.stop();
   for (BatchGroup &G : B.groups) {
     unsigned long long c[2] = {0, 0};
-    HIP_CHECK(hipMemcpyAsync(c, G.cand, sizeof(c), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    HIP_CHECK(hipMemcpyAsync(c, G.cand, sizeof(c), hipMemcpyDeviceToHost, G.stream));
+    HIP_CHECK(hipStreamSynchronize(G.stream));
     stats.candidates += c[0];
     stats.algo_bytes += c[1];
     stats.points += G.N;
@@ -2607,10 +2677,10 @@ static int run_batched(uint32_t nsets, const float *const *points, const uint32_
       const SetDesc &sd = G.hsets[i];
       const size_t cnt = (size_t)sd.n * sd.k1;
       if (!outIds[si] || !outDists[si]) throw Error(KNN_ERR_ARG, "null output pointer");
-      HIP_CHECK(hipMemcpyAsync(outIds[si], G.outIds + sd.outOff, sizeof(int32_t) * cnt, kout, s));
-      HIP_CHECK(hipMemcpyAsync(outDists[si], G.outDists + sd.outOff, sizeof(float) * cnt, kout, s));
+      HIP_CHECK(hipMemcpyAsync(outIds[si], G.outIds + sd.outOff, sizeof(int32_t) * cnt, kout, G.stream));
+      HIP_CHECK(hipMemcpyAsync(outDists[si], G.outDists + sd.outOff, sizeof(float) * cnt, kout, G.stream));
     }
-  HIP_CHECK(hipStreamSynchronize(s));
+  for (BatchGroup &G : B.groups) HIP_CHECK(hipStreamSynchronize(G.stream));
   stats.groups = (uint32_t)B.groups.size();
   stats.graph_replayed = replay ? 1u : 0u;
   stats.passes_graph = B.passes;

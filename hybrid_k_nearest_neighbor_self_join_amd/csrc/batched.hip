@@ -18,9 +18,9 @@
 // provably inside its block) and equal the rows of a single-set join of the same set.
 //
 // Every kernel reads its sizes (cells, tiles) from device memory, so a pass is a fixed
-// sequence of launches: the whole join (input copy, reorder, grids, indexes, P passes) is
-// captured once in a hipGraph and replayed for later calls with the same set shapes.
-// Passes left after the graph (rare) run eagerly.
+// sequence of launches: a group's set-up and first pass, a further pass, and the overflow kernel's
+// part are captured once in hipGraphs and replayed for later calls with the same set shapes, on a
+// stream per group, each pass only while queries of the group are pending.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
