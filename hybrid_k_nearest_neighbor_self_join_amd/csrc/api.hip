@@ -916,8 +916,11 @@ static uint32_t run_brute(Pipeline<T> &P, const uint8_t *sel, uint8_t *failed, i
   a.chunk = pl.chunk;
   a.nchunks = pl.nchunks;
   if (pl.partialEntries) {
-    a.partKey = P.template buf<double>(S_BRUTE_PK, pl.partialEntries);
-    a.partId = P.template buf<uint32_t>(S_BRUTE_PI, pl.partialEntries);
+    a.partKey = P.template buf<double>(S_BRUTE_PK, pl.partialEntries + nq);
+    a.partId = P.template buf<uint32_t>(S_BRUTE_PI, pl.partialEntries + nq);
+    a.partCount = a.partId + pl.partialEntries;
+    a.sample = pl.sample;
+    a.bound = pl.sample ? a.partKey + pl.partialEntries : nullptr;
   }
   a.outIds = dIds;
   a.outDists = dDists;

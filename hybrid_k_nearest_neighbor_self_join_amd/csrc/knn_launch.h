@@ -285,6 +285,9 @@ struct BruteArgs {
   uint32_t qw, chunk, nchunks;  // from brute_plan
   double *partKey;          // nq * nchunks * k1 entries each when nchunks > 1
   uint32_t *partId;
+  uint32_t *partCount;      // nq words when nchunks > 1
+  uint32_t sample;          // sampled points (from brute_plan) and the bounds' nq entries, or 0, null
+  double *bound;
   int32_t *outIds;
   void *outDists;
   uint8_t *failed;          // optional: failed[q] = 0 for every row written
@@ -293,6 +296,7 @@ struct BruteArgs {
 struct BrutePlan {
   uint32_t qw, chunk, nchunks;
   uint64_t partialEntries;
+  uint32_t sample;
 };
 // partial tables of at most maxPartialEntries entries (a single chunk always fits: no table)
 BrutePlan brute_plan(uint32_t n, uint32_t nq, uint32_t k1, uint64_t maxPartialEntries = 1ull << 26);

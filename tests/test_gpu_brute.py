@@ -104,3 +104,25 @@ def test_learned_fallback_default(oracle):
     assert a[2].brute_queries > 0 and b[2].brute_queries == 0
     assert np.array_equal(a[0], b[0]) and np.array_equal(bits(a[1]), bits(b[1]))
     assert_rows(oracle, pts, 32, a[0], a[1])
+
+
+@pytest.mark.parametrize("n,d,k,nfar,dtype", [
+    (4096, 2, 1, 1, np.float32),      # the smallest set whose chunks share a sampled bound
+    (20011, 3, 63, 20, np.float64),
+    (50021, 2, 100, 5, np.float32),
+    (30000, 9, 8, 3, np.float32),
+])
+def test_brute_tail_rows(oracle, n, d, k, nfar, dtype):
+    # a few far points, some of them at one place, and a cloud with repeated points
+    rng = np.random.default_rng(n)
+    c = rng.normal(0.0, 1.0, (n - nfar, d))
+    c[: n // 4] = c[n // 4: 2 * (n // 4)]
+    far = rng.uniform(300.0, 400.0, (nfar, d))
+    far[nfar // 2:] = far[nfar // 2]
+    pts = np.concatenate([c, far]).astype(dtype)
+    ids, dist, st = _lib.knnjoin_ex(pts, k, beta=0.025, brute_fallback=1)
+    assert st.brute_queries > 0
+    q = np.concatenate([rng.choice(n - nfar, 200, replace=False), np.arange(n - nfar, n)])
+    perm, _ = oracle.reorder(pts)
+    bi, bd = oracle.bruteforce(np.ascontiguousarray(pts[:, perm]), k, queries=q)
+    assert np.array_equal(ids[q], bi) and np.array_equal(dist[q], bd)
