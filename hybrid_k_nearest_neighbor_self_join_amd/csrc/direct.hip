@@ -83,12 +83,18 @@ __device__ __forceinline__ double root_of(double s) { return sqrt(s); }
 
 // waves per SIMD the register budget is set for: 4 (128 registers), 2 for the largest lists
 constexpr int waves_per_simd(int h) { return h <= 4 ? 4 : 2; }
+// Windows of 64 candidates that a chunk's row tables cover, and those kept in registers: the last
+// two of the 8 at H = 4 live in LDS (1 KB, within the 10 KB of 16 waves per CU).  All 8 in
+// registers spill 18 of the 128: range-kernel ms, 10M mixed 2-D K=64 learned 8.9 / 8.1 and plain
+// 13.5 / 11.6, 3M K=128 learned 6.8 / 6.4, 3M K=200 plain 9.1 / 8.7.
+constexpr uint32_t windows(int h) { return h >= 4 ? 8 : 4; }
+constexpr uint32_t reg_windows(int h) { return h == 4 ? 6 : windows(h); }
 // LDS: DR_NB bucket counters and 64 dummies, H * 64 sorted (key, id) slots and four sentinels, a
-// list of positions, and with a row table DR_RMAX words per query of a chunk
+// list of positions, and with a row table DR_RMAX words and the last windows per query of a chunk
 constexpr uint32_t list_cap(int h, bool tab) { return h * 64 + (tab && h == 3 ? 128 : 256); }
 constexpr size_t lds_bytes(int h, bool tab) {
   return ((size_t)(DR_NB + 64) * 4 + (size_t)(h * 64 + 4) * 12 + (size_t)list_cap(h, tab) * 4 +
-          (tab ? 64 * DR_RMAX * 4 : 0) + 15) & ~(size_t)15;
+          (tab ? 64 * DR_RMAX * 4 + 64 * (windows(h) - reg_windows(h)) * 8 : 0) + 15) & ~(size_t)15;
 }
 
 // Rounds of a selection of NR rounds that hold 64 items each, whatever its item count: 1..4 rounds
@@ -163,7 +169,7 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
   constexpr bool TAB = ND == 1 || ND == 2;
   constexpr int PR = TAB ? 2 : (D <= 4 ? 3 : (D <= 8 ? 2 : 1));
   constexpr uint32_t RM = ND == 1 ? 1 : DR_RMAX;
-  constexpr uint32_t NW = H >= 4 ? 8 : 4;  // windows of 64 candidates a chunk's row tables cover
+  constexpr uint32_t NW = windows(H), NWR = reg_windows(H);
   constexpr uint32_t CAP = list_cap(H, TAB);  // list slots
   constexpr uint32_t ROOM = CAP - 64u * PR;
   uint32_t *hist = reinterpret_cast<uint32_t *>(smem);  // DR_NB counters, 64 dummies
@@ -171,6 +177,7 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
   uint32_t *sid = reinterpret_cast<uint32_t *>(skey + H * 64 + 4);
   uint32_t *list = sid + H * 64 + 4;
   uint32_t *rowB = list + CAP;  // TAB: position offsets of the chunk's rows, DR_RMAX per query
+  uint64_t *winH = reinterpret_cast<uint64_t *>(rowB + 64 * DR_RMAX);  // TAB: windows from NWR on
   uint32_t *segB = sid, *segX = sid + 64;  // a stream's segment tables (the sorted ids come later)
   const uint32_t lane = threadIdx.x;
   const T *__restrict__ xs = reinterpret_cast<const T *>(a.xs);
@@ -224,7 +231,7 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
     // f + rowB[k]; the row of f is counted from a bitmap of the starts (bit X_k - 1, so that the
     // bits below a lane's own are the starts at or before its candidate)
     uint32_t RL = 0, totL = 0;
-    uint64_t winL[NW] = {};
+    uint64_t winL[NWR] = {};
     wave_lds_sync();
     T rs = rL;  // the radius searched first
     if constexpr (TAB) {
@@ -237,7 +244,9 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
         RL = 0;
         totL = 0;
 #pragma unroll
-        for (uint32_t w = 0; w < NW; w++) winL[w] = 0;
+        for (uint32_t w = 0; w < NWR; w++) winL[w] = 0;
+#pragma unroll
+        for (uint32_t w = NWR; w < NW; w++) winH[lane * (NW - NWR) + w - NWR] = 0;
         const bool fits = h1 - l1 < RM;
         const double r2 = (double)rr * (double)rr * (1.0 + 0x1p-15), invr2 = rr > (T)0 ? 1.0 / ((double)rr * (double)rr) : 0.0;
         // ranges of row k (none past the block or outside the ball): start, point count
@@ -267,8 +276,10 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
           rowB[lane * DR_RMAX + RL] = pB - totL;
           const uint32_t b = totL - 1u;
 #pragma unroll
-          for (int w = 0; w < (int)NW; w++)
+          for (int w = 0; w < (int)NWR; w++)
             if (RL && (b >> 6) == (uint32_t)w) winL[w] |= 1ull << (b & 63u);
+          if (NWR < NW && RL && (b >> 6) >= NWR && (b >> 6) < NW)
+            winH[lane * (NW - NWR) + (b >> 6) - NWR] |= 1ull << (b & 63u);
           RL++;
           totL += len;
         };
@@ -512,8 +523,16 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
           uint32_t pv[NR], cnt[NR];
 #pragma unroll
           for (int u = 0; u < NR; u++) {
-            const uint64_t wm = winL[W0 + u];
-            const uint64_t w = (uint64_t)rl((uint32_t)wm, i) | ((uint64_t)rl((uint32_t)(wm >> 32), i) << 32);
+            uint64_t w;
+            if constexpr (W0 + NR > (int)NWR) {
+              const uint64_t wm = W0 + u < (int)NWR ? winL[W0 + u < (int)NWR ? W0 + u : 0]
+                                                    : winH[i * (NW - NWR) + (uint32_t)(W0 + u) - NWR];
+              const uint32_t from = W0 + u < (int)NWR ? i : 0u;
+              w = (uint64_t)rl((uint32_t)wm, from) | ((uint64_t)rl((uint32_t)(wm >> 32), from) << 32);
+            } else {
+              const uint64_t wm = winL[W0 + u];
+              w = (uint64_t)rl((uint32_t)wm, i) | ((uint64_t)rl((uint32_t)(wm >> 32), i) << 32);
+            }
             const uint32_t k = run + mbcnt64(w);
             run += (uint32_t)__popcll(w);
             const uint32_t f0 = 64u * (W0 + u), fi = f0 + lane;
