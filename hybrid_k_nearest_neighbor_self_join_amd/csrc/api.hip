@@ -52,7 +52,7 @@ struct Error : std::runtime_error {
 enum Slot {
   S_PTS, S_X, S_XS, S_KEYS, S_KEYS_TMP, S_IDS, S_IDS_TMP, S_CELLKEYS, S_CELLSTART, S_FLAGS, S_POS,
   S_ACT, S_NTILES, S_TILEOFF, S_TILES, S_FAILED, S_ROWSUM, S_OUTIDS, S_OUTDISTS, S_SCRATCH,
-  S_HEAP, S_SMALL, S_PART, S_CTR, S_CSUM, S_HOSTFLAGS, S_OVERFLOW, S_STAGE, S_DENSE, S_CELLOF, S_CELLMAX, S_FCNT, S_RADIUS, S_RHIST, S_MODEL, S_TRAIN, S_OCC, S_ACTQ, S_BRUTE_PK, S_BRUTE_PI, S_BLIST, S_TILEMETA, S_HCPU, S_HGPU, S_HLIST, S_HROWI, S_HROWD, S_XS2, S_SIDS, S_SIDS2, S_ABITS, S_NSLOTS
+  S_HEAP, S_SMALL, S_PART, S_CTR, S_CSUM, S_HOSTFLAGS, S_OVERFLOW, S_STAGE, S_DENSE, S_CELLOF, S_CELLMAX, S_FCNT, S_RADIUS, S_RHIST, S_MODEL, S_TRAIN, S_OCC, S_ACTQ, S_BRUTE_PK, S_BRUTE_PI, S_BLIST, S_TILEMETA, S_HCPU, S_HGPU, S_HLIST, S_HROWI, S_HROWD, S_XS2, S_SIDS, S_SIDS2, S_ABITS, S_TRYR, S_NSLOTS
 };
 
 // Slots of one no-allocation call: regions of the static device scratch array handed out in
@@ -324,15 +324,16 @@ struct Pipeline {
   // ordered array (nearby positions, cached lines) instead of the input's random order.
   // Within a cell the points then follow the previous order; every row and count is the same
   // (rows are ranked by (key, id)).  The no-allocation path keeps one copy (original order).
-  void build_index(const T *mn, const T *mx, T eps) {
-    grid_dims<T>(mn, mx, nd, eps, g, totalCells);
+  // The grid is over the first gd dims.
+  void build_index(const T *mn, const T *mx, uint32_t gd, T eps) {
+    grid_dims<T>(mn, mx, gd, eps, g, totalCells);
     const int bits = bits_for(totalCells);
     // slab order within cells (u32 keys only: the slab code takes the key bits the cell id
     // leaves, up to 16, and at least 8)
-    if (slab && bits <= 24 && slabMax > slabMin) {
+    if (gd < slabDims && bits <= 24 && mx[gd] > mn[gd]) {
       g.sb = (uint32_t)std::min(16, 32 - bits);
-      g.smin = slabMin;
-      g.sscale = (T)(std::ldexp(1.0, (int)g.sb) / ((double)slabMax - (double)slabMin));
+      g.smin = mn[gd];
+      g.sscale = (T)(std::ldexp(1.0, (int)g.sb) / ((double)mx[gd] - (double)mn[gd]));
     }
     const bool fromPrev = xs != nullptr && sortedIds != nullptr && !g_arena;
     const T *keySrc = fromPrev ? xs : x;
@@ -422,27 +423,50 @@ struct Pipeline {
     sync();
     ncell = pin[PW_NCELL];
   }
-  // slab order (fewer indexed than data dims): on when index_minmax has found the range of
-  // the first non-indexed dim; the stage entry points leave it off
-  bool slab = false;
-  T slabMin = 0, slabMax = 0;
-  // min/max of the indexed dims into hmn/hmx (nd values each), and of the first non-indexed
-  // dim for the slab order (KNN_SLAB=0 turns the slab order off)
+  // dims whose range index_minmax found, when the slab order may use one of them past the grid's;
+  // 0 turns it off (the stage entry points, and KNN_SLAB=0, which prunes by the indexed dims alone)
+  uint32_t slabDims = 0;
+  // min/max of the dims a grid may be over, max_grid_dims(), and of the one after them for the
+  // slab order, into hmn/hmx (KNN_MAX_INDEXED entries)
   void index_minmax(T *hmn, T *hmx) {
-    const char *ev = std::getenv("KNN_SLAB");
-    const bool want = nd < d && nd < KNN_MAX_INDEXED && !(ev && ev[0] == '0');
-    const uint32_t nde = want ? nd + 1 : nd;
+    const uint32_t m = std::max(nd, max_grid_dims());
+    const uint32_t nde = m < d && m < KNN_MAX_INDEXED ? m + 1 : m;
     T *mm = buf<T>(S_PART, 2 * KNN_MAX_INDEXED + minmax_scratch_elems(n, nde));
     minmax_soa<T>(x, n, nde, mm, mm + KNN_MAX_INDEXED, mm + 2 * KNN_MAX_INDEXED, s);
-    T lo[KNN_MAX_INDEXED], hi[KNN_MAX_INDEXED];
-    HIP_CHECK(hipMemcpyAsync(lo, mm, sizeof(T) * nde, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(hi, mm + KNN_MAX_INDEXED, sizeof(T) * nde, hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipMemcpyAsync(hmn, mm, sizeof(T) * nde, hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipMemcpyAsync(hmx, mm + KNN_MAX_INDEXED, sizeof(T) * nde, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
-    std::memcpy(hmn, lo, sizeof(T) * nd);
-    std::memcpy(hmx, hi, sizeof(T) * nd);
-    slab = want;
-    slabMin = want ? lo[nd] : (T)0;
-    slabMax = want ? hi[nd] : (T)0;
+    slabDims = indexed_dims_only() ? 0u : nde;
+  }
+  // Dims of the range passes' grids: the join's indexed dims define its schedule and its radius
+  // features, while a grid may be over more of the data's dims (any grid gives the same rows and
+  // the same failures at a radius).
+  // Up to 6 dims, as a join that indexes them all (ms per join, the indexed dims' grid against
+  // one over all dims): 1M skewed 6-D points on 4 indexed dims K=32, learned 62.3 / 46.5, 3M
+  // uniform 4-D on 2 K=16 29.6 / 8.8; plain, 500k uniform 6-D on 4 K=16 8.3 / 5.7, 500k skewed
+  // 4-D on 2 K=16 18.2 / 11.9, 200k uniform 6-D on 2 K=8 5.8 / 2.9, 500k mixed 3-D on 1 K=8 28.3 /
+  // 20.0.  A grid falls back to fewer dims where its cells outgrow the points.  The no-allocation
+  // scratch and the hybrid split keep the indexed dims' grid.  KNN_GRID_DIMS=0..6 overrides the 6.
+  static bool indexed_dims_only() {
+    const char *v = std::getenv("KNN_SLAB");
+    return v && v[0] == '0';
+  }
+  bool moreDims = true;
+  uint32_t max_grid_dims() const {
+    const char *ev = std::getenv("KNN_GRID_DIMS");
+    const uint32_t top = ev ? (uint32_t)std::atoi(ev) : 6u;
+    return g_arena || !moreDims || indexed_dims_only() ? nd : std::max(nd, std::min(d, std::min(top, 6u)));
+  }
+  bool grid_fits(const T *mn, const T *mx, uint32_t gd, T w, uint64_t cells) const {
+    typename GridOf<T>::type gt;
+    uint64_t tc = 0;
+    try {
+      if (!(w > (T)0)) return false;
+      grid_dims<T>(mn, mx, gd, w, gt, tc);
+    } catch (const Error &) {
+      return false;
+    }
+    return tc <= cells;
   }
   const uint32_t *ncellDev = nullptr;  // device copy of ncell (the scan total of the build)
   Slot xsSlot = S_XS;                   // the slot holding the current cell-sorted copy
@@ -481,6 +505,7 @@ struct Pipeline {
   uint32_t lastActive = 0;   // queries left to the range kernel after the pre-check
   static constexpr uint32_t kCollectGrid = 2816;  // persistent collect-kernel workgroups
   static constexpr uint32_t kHeapGrid = 512;   // persistent heap-kernel workgroups
+  T *tryR = nullptr;  // radii the direct kernel searches first, from the last make_active
   const uint32_t *activeDev = nullptr;         // active count of the last make_active (device)
 };
 
@@ -675,6 +700,7 @@ void Pipeline<T>::make_active(const uint8_t *activeFailed, uint32_t *&act, uint8
   uint32_t *flags = buf<uint32_t>(S_FLAGS, n + 1);
   uint32_t *pos = buf<uint32_t>(S_POS, n + 1);
   bool all = !activeFailed;
+  tryR = nullptr;
   if (denseStart && failed) {
     // own-block pre-check (exact early failures) + per-cell candidate accounting
     uint32_t *cellMax = buf<uint32_t>(S_CELLMAX, (size_t)ncell + 1);
@@ -684,8 +710,11 @@ void Pipeline<T>::make_active(const uint8_t *activeFailed, uint32_t *&act, uint8
       activeBits = buf<uint64_t>(S_ABITS, ((size_t)n + 63) / 64);
       pack_bits(activeFailed, n, activeBits, s);
     }
+    // (none with the no-allocation scratch, which is sized without it)
+    tryR = g.nd == d && g.nd > 2 && !g_arena ? buf<T>(S_TRYR, n) : nullptr;
+    const float want = (float)K1 + 2.5f * std::sqrt((float)K1) + 1.0f;
     prefilter<T>(xs, n, g, radius, uniform_radius(), denseStart, sortedIds, activeBits, failed, K1, cellOf, cellMax,
-                 flags, s);
+                 flags, tryR, want, s);
     if (cellAcc) cell_bytes(cellMax, ncell, cellAcc, s);
     all = false;
   } else {
@@ -742,6 +771,7 @@ PassResult Pipeline<T>::pass(const uint8_t *activeFailed, uint32_t nq, uint8_t *
   a.denseStart = denseStart;
   a.act = act;
   a.activeCount = activeDev;
+  a.tryRadius = tryR;
   a.n = n;
   a.d = d;
   a.k1 = K1;
@@ -755,7 +785,7 @@ PassResult Pipeline<T>::pass(const uint8_t *activeFailed, uint32_t nq, uint8_t *
   a.tileCounter = tileCounter;
   a.tileRanges = tile_ranges(d, false);
   a.segCapLog2 = seg_cap_log2();
-  a.lookupRows = lastRows = lookup_rows(nd);
+  a.lookupRows = lastRows = lookup_rows(g.nd);
   a.overflow = overflow;
   a.overflowCount = overflowCount;
   PassResult r{};
@@ -826,7 +856,7 @@ PassResult Pipeline<T>::pass(const uint8_t *activeFailed, uint32_t nq, uint8_t *
   unsigned long long hctr[6];
   std::memcpy(hctr, pin + PW_CTR, sizeof(hctr));
   uint64_t cellsScanned = 1;
-  for (uint32_t j = 0; j < nd; j++) cellsScanned *= 3;
+  for (uint32_t j = 0; j < g.nd; j++) cellsScanned *= 3;
   accBytes += hctr[4] * (sizeof(T) * d + 4ull) + hctr[5] * cellsScanned * 8ull;
   r.bytes_total = hctr[1] + accBytes;
   r.pairs = hctr[0];
@@ -1283,31 +1313,28 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
 
   // ---- min/max of the indexed dims (main.cu:2439-2456)
   T hmn[KNN_MAX_INDEXED], hmx[KNN_MAX_INDEXED];
+  P.moreDims = !prm.hybrid_threads;  // (the host share's cells are those of the indexed dims)
   P.index_minmax(hmn, hmx);
   if (eps0 == (T)0) eps0 = fallback_eps<T>(hmn, hmx, nd, n, K1);
   stats.eps0 = (float)eps0;
 
   // ---- the join loop (main.cu:305-430)
-  const double pdiv = plain_grid_div(d, nd, K1), preach = plain_max_reach(d, nd, K1);
   T curW = (T)0;
+  uint32_t curDims = nd;
   auto build = [&](T e) -> double {
+    const uint64_t small = std::min<uint64_t>(Pipeline<T>::kDenseMaxCells - 1, 16ull * n + (1u << 20));
+    uint32_t gd = P.max_grid_dims();
+    while (gd > nd && !P.grid_fits(hmn, hmx, gd, (T)((double)e / plain_grid_div(d, gd, K1)), small)) gd--;
+    const double pdiv = plain_grid_div(d, gd, K1);
     T w = (T)((double)e / pdiv);
-    if (pdiv > 1.0) {  // a finer grid only while its dense start table stays small beside the points
-      typename GridOf<T>::type gt;
-      uint64_t tc = 0;
-      bool ok = w > (T)0;
-      try {
-        if (ok) grid_dims<T>(hmn, hmx, nd, w, gt, tc);
-      } catch (const Error &) {
-        ok = false;
-      }
-      if (!ok || tc > std::min<uint64_t>(Pipeline<T>::kDenseMaxCells - 1, 16ull * n + (1u << 20))) w = e;
-    }
+    // a finer grid only while its dense start table stays small beside the points
+    if (pdiv > 1.0 && !P.grid_fits(hmn, hmx, gd, w, small)) w = e;
     P.tBuild = &tPh;
     tPh.start();
-    P.build_index(hmn, hmx, w);
+    P.build_index(hmn, hmx, gd, w);
     P.tBuild = nullptr;
     curW = w;
+    curDims = gd;
     return tPh.elapsed();
   };
   P.radius = nullptr;  // every query searches the same radius, passed by value
@@ -1340,7 +1367,7 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
           throw Error(KNN_ERR_NO_PROGRESS, "eps + eps0/2 == eps: epsilon cannot grow");
         }
         eps = grown;
-        if ((double)eps > preach * (double)curW) stats.ms_index += build(eps);
+        if ((double)eps > plain_max_reach(d, curDims, K1) * (double)curW) stats.ms_index += build(eps);
         reindexes++;  // the reference's re-index count: eps growths
       } else {
         // The reference reruns the failed queries at the same eps (main.cu:330 is false);
@@ -1404,25 +1431,28 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
 //   2-D  K=64 10M mixed:  R/3, 8 16.3;  R/4, 8 16.1;  R/3, 10 14.3;  R/4, 10 14.8;  R/5, 10 14.6
 //        K=16 10M mixed:  R/3, 8 12.0;  R/3, 10 12.0;  R/5, 10 12.4;  R/4, 8 17.6
 //        K=100 1.3M / K=128 3M mixed:  R/4, 10 6.03 / 9.89;  R/5, 10 5.81 / 8.95;  R/4, 12 6.57 / 10.1
-//   4-D  5M skewed K=32 / 300k skewed K=32 / 3M uniform K=16:  R, 2 26.8 / 9.9 / 8.4;
-//        R/1.25, 4 22.1 / 6.6 / 8.8;  R/1.5, 5 22.3 / 6.3 / 8.8;  R/1.75, 6 23.5 / 6.1 / 8.8
-//   6-D  2M skewed / 2M uniform K=32 / 200k skewed K=16:  R, 2 52.9 / 27.2 / 8.9;
-//        R/1.15, 2 40.2 / 27.2 / 9.8;  R/1.25, 3 39.1 / 25.8 / 8.7
-//   projected grids (fewer indexed than data dims), 6 bins:  1M 6-D on 4 dims, skewed K=32,
-//        R/2 78.2, R/3 62.3, R/4 73.8;  1M 4-D on 2 dims, skewed K=32, R/3 40.4, R/4 36.7, R/5 34.4
+//   4-D  5M skewed K=32 / 3M uniform K=16 / 1M on 2 indexed dims, skewed K=32, with failures
+//        growing x2^(1/4):  R/1.5, 5 21.6 / 8.7 / 9.5;  x2^(1/2):  R/1.5, 5 19.2 / 7.9 / 7.6;
+//        R/1.75, 6 19.3 / 8.0 / 7.6;  R/2, 8 18.4 / 8.3 / 9.0
+//   6-D  1M on 4 indexed dims, skewed K=32 / 2M skewed K=32 / 2M uniform K=32 / 200k skewed K=16,
+//        x2^(1/4):  R/1.25, 3 39.0 / 36.1 / 24.2 / 8.3;  R/1.5, 3 26.8 / 36.1 / 25.1 / 8.6;
+//        R/1.5, 4 27.5 / 35.4 / 24.3 / 7.1;  R/1.75, 5 29.2 / 39.5 / 24.6 / 8.3;
+//        x2^(1/2):  R/1.5, 4 29.3 / 37.9 / 23.3 / 6.6
+//   grids of fewer dims than the data's, 6 bins:  1M 6-D on 4 dims, skewed K=32, R/2 78.2, R/3
+//        62.3, R/4 73.8;  1M 4-D on 2 dims, skewed K=32, R/3 40.4, R/4 36.7, R/5 34.4
 // KNN_LEARNED_GRID_DIV (1..8) and KNN_LEARNED_CLASS_BINS (1..16) override them for tuning.
 static double learned_grid_div(uint32_t d, uint32_t nd, uint32_t k1) {
   const double e = env_knob("KNN_LEARNED_GRID_DIV", 1.0, 8.0);
   if (e > 0.0) return e;
-  if (nd < d) return nd <= 2 ? 4.0 : 3.0;
-  if (nd <= 2) return k1 <= 40 ? 3.0 : 5.0;
-  return nd <= 4 ? 1.5 : 1.25;
+  if (nd <= 2) return nd < d ? 4.0 : (k1 <= 40 ? 3.0 : 5.0);
+  if (nd <= 4) return nd < d ? 3.0 : 1.75;
+  return 1.5;
 }
 static int learned_class_bins(uint32_t d, uint32_t nd) {
   const int e = (int)env_knob("KNN_LEARNED_CLASS_BINS", 1.0, 16.0);
   if (e > 0) return e;
-  if (nd < d) return 6;
-  return nd <= 2 ? 10 : (nd <= 4 ? 5 : 3);
+  if (nd <= 2) return nd < d ? 6 : 10;
+  return nd <= 4 ? 6 : 4;
 }
 
 // The learned schedule: per-query initial radius from the MLP, then passes over radius
@@ -1459,10 +1489,8 @@ static void run_learned(Pipeline<T> &P, const knnjoin_params &p, knnjoin_stats &
   P.radius = radius;
 
   // ---- radius classes: the pending queries whose radius lies in the lowest occupied class
-  // of bins [c, c + learned_class_bins) (two or two and a half octaves with <= 2 indexed dims,
-  // one and a half on projected grids, half an octave above) are joined on a grid matched to R
-  // (cell width R / learned_grid_div);
-  // queries that fail grow their radius (x2, or x2^(1/4) with 3 or more indexed dims), which
+  // of bins [c, c + learned_class_bins) are joined on a grid matched to R (cell width
+  // R / learned_grid_div); queries that fail grow their radius, which
   // moves them to a later class.  One index build per occupied class.
   unsigned long long *ctr = P.template buf<unsigned long long>(S_CTR, 64);
   fill_u32(reinterpret_cast<uint32_t *>(ctr), 0u, 16, s);
@@ -1510,15 +1538,21 @@ static void run_learned(Pipeline<T> &P, const knnjoin_params &p, knnjoin_stats &
       passes++;
       break;
     }
-    // wide classes with <= 2 indexed dims and on projected grids; half an octave above, where a
-    // cell up to 2x the radius would cost up to 2^nd in block volume
-    const int cHi = std::min(c + learned_class_bins(P.d, nd) - 1, 63);
+    // the grid's dims (while its dense start table has at most 64 cells per point: 0.2 ms a build
+    // at 1M points), and with them the class and its largest radius R
+    uint32_t gd = P.max_grid_dims();
+    int cHi = 0;
+    double R = 0;
+    for (;; gd--) {
+      cHi = std::min(c + learned_class_bins(P.d, gd) - 1, 63);
+      R = (double)wfF * std::exp2((cHi + 1 - 32) / 4.0);
+      if (gd == nd || P.grid_fits(hmn, hmx, gd, (T)(R / learned_grid_div(P.d, gd, K1)),
+                                  std::min<uint64_t>(Pipeline<T>::kDenseMaxCells - 1, 64ull * n + (1u << 20))))
+        break;
+    }
     uint32_t nq = 0;
     for (int b = c; b <= cHi; b++) nq += h[b];
-    double R;
-    if (cHi < 63) {
-      R = (double)wfF * std::exp2((cHi + 1 - 32) / 4.0);
-    } else {
+    if (cHi == 63) {
       // the top bin is open-ended: the class's largest radius bounds it
       max_failed_radius(radius, failed, n, maxr, s);
       HIP_CHECK(hipMemcpyAsync(pin + PW_MAXR, maxr, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
@@ -1535,9 +1569,7 @@ static void run_learned(Pipeline<T> &P, const knnjoin_params &p, knnjoin_stats &
       }
       R = R * (1.0 + 1e-6);
     }
-    // cell width R/3 with <= 2 indexed dims (R/4 on projected grids); above, R (<= 3 cells per
-    // dim), since every extra cell of reach multiplies the rows of a block
-    T w = (T)(R / learned_grid_div(P.d, nd, P.K1));
+    T w = (T)(R / learned_grid_div(P.d, gd, P.K1));
     if (!(w > (T)0)) w = F.wf;
     // a small tail of pending queries (at most N/64) keeps the current grid when its blocks
     // stay within 1024 cells: an index build over all N points costs more than the wider
@@ -1546,25 +1578,17 @@ static void run_learned(Pipeline<T> &P, const knnjoin_params &p, knnjoin_stats &
     bool reuse = false;
     if (curW > (T)0 && (uint64_t)nq * reuse_tail_div() <= (uint64_t)n) {
       const double reach = std::ceil(R / (double)curW);
-      reuse = std::pow(2.0 * reach + 1.0, (double)nd) <= 1024.0;
+      reuse = std::pow(2.0 * reach + 1.0, (double)P.g.nd) <= 1024.0;
     }
-    if (reuse) w = curW;
-    for (;;) {  // keep the grid within 2^30 cells
-      typename GridOf<T>::type gt;
-      uint64_t tc = 0;
-      bool ok = true;
-      try {
-        grid_dims<T>(hmn, hmx, nd, w, gt, tc);
-      } catch (const Error &) {
-        ok = false;
-      }
-      if (ok && tc <= (1ull << 30)) break;
-      w = w * (T)2;
+    if (reuse) {
+      w = curW;
+      gd = P.g.nd;
     }
-    if (w != curW) {
+    while (!P.grid_fits(hmn, hmx, gd, w, 1ull << 30)) w = w * (T)2;  // keep the grid within 2^30 cells
+    if (w != curW || gd != P.g.nd) {
       P.tBuild = &tPh;
       tPh.start();
-      P.build_index(hmn, hmx, w);
+      P.build_index(hmn, hmx, gd, w);
       P.tBuild = nullptr;
       const double bms = tPh.elapsed();
       stats.ms_index += bms;
@@ -1574,10 +1598,10 @@ static void run_learned(Pipeline<T> &P, const knnjoin_params &p, knnjoin_stats &
       if (stats.eps0 == 0.0f) stats.eps0 = (float)w;
     }
     radius_class_flags(radius, failed, n, wfF, (uint32_t)c, (uint32_t)cHi, act, s);
-    // growth on failure: one class (an octave; a quarter octave with >= 3 indexed dims), then
+    // growth on failure (an octave; half an octave on a grid of 3 or 4 dims, a quarter above), then
     // the next histogram, both before the pass's wait; after a heap-kernel pass (overflowing
     // staging) only the histogram again
-    const T factor = nd <= 2 ? (T)2 : (T)1.189207115002721;
+    const T factor = P.g.nd <= 2 ? (T)2 : (P.g.nd <= 4 ? (T)1.4142135623730951 : (T)1.189207115002721);
     PassResult pr = P.pass(act, nq, failed, dIds, dDists, ctr, tK, tPh,
                            [&]() {
                              grow_class_radius(radius, act, failed, n, factor, s);
@@ -1867,7 +1891,7 @@ int knnjoin_stage_index(const float *points, uint32_t n, uint32_t ndim, uint32_t
     stage_setup(P, points, n, ndim, nd, 0);
     float hmn[KNN_MAX_INDEXED], hmx[KNN_MAX_INDEXED];
     stage_minmax(P, hmn, hmx);
-    P.build_index(hmn, hmx, eps);
+    P.build_index(hmn, hmx, P.nd, eps);
     if (min_arr) std::memcpy(min_arr, P.g.minArr, sizeof(float) * nd);
     if (n_cells) std::memcpy(n_cells, P.g.nCells, sizeof(uint32_t) * nd);
     if (total_cells) *total_cells = P.totalCells;
@@ -1897,7 +1921,7 @@ int knnjoin_stage_join_pass(const float *points, uint32_t n, uint32_t ndim, uint
     stage_setup(P, points, n, ndim, nd, k);
     float hmn[KNN_MAX_INDEXED], hmx[KNN_MAX_INDEXED];
     stage_minmax(P, hmn, hmx);
-    P.build_index(hmn, hmx, eps);
+    P.build_index(hmn, hmx, P.nd, eps);
     const uint32_t K1 = k + 1;
     std::vector<uint8_t> act(n, 0);
     for (uint32_t i = 0; i < nq; i++) {

@@ -234,6 +234,7 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
     uint64_t winL[NWR] = {};
     wave_lds_sync();
     T rs = rL;  // the radius searched first
+    if (!TAB && !SETS && a.tryRadius) rs = reinterpret_cast<const T *>(a.tryRadius)[qL];
     if constexpr (TAB) {
       const double q1 = ND >= 2 ? (double)qcL[ND - 1] : 0.0;
       auto lookup = [&](T rr) {
@@ -314,7 +315,7 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
     }
     const double TqL = (double)rs * (double)rs * (1.0 - 0x1p-20);
     const double scL = TqL > 0.0 ? (double)(DR_NB - 1) / TqL : 0.0;
-    const uint64_t shrunk = TAB ? ballot64(rs < rL) : 0ull;
+    const uint64_t shrunk = ballot64(rs < rL);
     wave_lds_sync();
     uint64_t okMask = 0, ovMask = 0;
     unsigned long long seen = 0;
@@ -513,7 +514,7 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
         okMask |= 1ull << i;
       };
       // ---- stream
-      for (uint32_t tryFull = (TAB && Ri) ? 0u : 1u;; tryFull = 1u) {
+      for (uint32_t tryFull = (TAB ? Ri != 0u : ((shrunk >> i) & 1ull) != 0ull) ? 0u : 1u;; tryFull = 1u) {
       if (TAB && !tryFull) {
         const uint32_t tot = rl(totL, i);
         seen += tot;
@@ -557,7 +558,7 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
         else if (tot > 64u) tabled(IntC<2>(), IntC<0>());
         else if (tot) tabled(IntC<1>(), IntC<0>());
       } else {
-        const T r = readlane<T>(rL, (int)i);
+        const T r = readlane<T>(TAB || tryFull ? rL : rs, (int)i);
         auto group = [&](const uint32_t (&pv)[PR], const bool (&)[PR], uint32_t f0, uint32_t tot) {
           if (ovf) return;
           if (M > ROOM) {

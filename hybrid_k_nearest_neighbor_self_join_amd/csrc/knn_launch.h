@@ -103,7 +103,8 @@ template <typename T>
 void prefilter(const T *xs, uint32_t n, const typename GridOf<T>::type &g, const T *radius,
                T rAll, const uint32_t *dense, const uint32_t *sortedIds, const uint64_t *activeBits,
                uint8_t *failed, uint32_t k1, const uint32_t *cellOf, uint32_t *cellMax,
-               uint32_t *flags, hipStream_t s);
+               uint32_t *flags, T *tryR,
+               float want, hipStream_t s);
 void cell_bytes(const uint32_t *cellMax, uint32_t ncell, unsigned long long *out, hipStream_t s);
 void cell_of(const uint32_t *flags, const uint32_t *pos, uint32_t n, uint32_t *cellOf, hipStream_t s);
 
@@ -152,6 +153,7 @@ struct JoinArgs {
   // direct and collect kernels without tiles (tiles null): the active query count (device); a
   // work unit is then a chunk of consecutive active queries
   const uint32_t *activeCount;
+  const void *tryRadius;  // direct kernel, > 2 indexed dims: per point, the radius searched first (null: radius)
   uint32_t lookupRows;   // direct kernel, <= 2 indexed dims: rows of a block looked up per step (1 or 2)
 };
 // Direct kernel (wave = query, direct.hip): the range kernel of every pass with K+1 <= DR_MAX_K1.

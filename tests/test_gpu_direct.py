@@ -65,3 +65,41 @@ def test_double_rows(oracle):
     bi, bd = oracle.bruteforce(np.ascontiguousarray(pts[:, perm]), 24)
     assert np.array_equal(ids, bi)
     assert np.array_equal(dist.view(np.uint64), bd.view(np.uint64))
+
+
+@pytest.mark.parametrize("d,nd,k,dtype,mode", [
+    (3, 1, 8, np.float32, "plain"), (4, 2, 40, np.float64, "plain"), (6, 4, 16, np.float32, "plain"),
+    (6, 1, 5, np.float32, "plain"), (9, 3, 16, np.float32, "plain"), (16, 2, 4, np.float64, "plain"),
+    (7, 7, 8, np.float32, "plain"), (4, 2, 16, np.float32, "learned"), (6, 4, 33, np.float64, "learned"),
+    (6, 4, 450, np.float32, "learned"),
+])
+@pytest.mark.parametrize("data", ["mixed", "flat", "far"])
+def test_grid_dims(oracle, monkeypatch, d, nd, k, dtype, mode, data):
+    # a grid over more dims than the join indexes gives the rows, the schedule and the failures of
+    # the indexed dims' grid: "flat" has constant dims, "far" one whose cells do not fit a table
+    rng = np.random.default_rng(7 * d + nd)
+    n = 6000
+    pts = rng.random((n, d))
+    pts[n // 2:] = 0.5 + 0.01 * rng.normal(size=(n - n // 2, d))
+    pts[100:140] = pts[100]
+    if data == "flat":
+        pts[:, nd:] = 0.25
+    if data == "far":
+        pts *= 0.5 ** np.arange(d)  # the indexed dims are those of the largest variance
+        pts[0] *= 10.0
+    pts = pts.astype(dtype)
+    if mode == "learned":
+        learned_radius.register_default_models()
+    m = _lib.KNN_MODE_LEARNED if mode == "learned" else _lib.KNN_MODE_BETA
+    res = []
+    for dims in ("0", "6"):
+        monkeypatch.setenv("KNN_GRID_DIMS", dims)
+        res.append(_lib.knnjoin_ex(pts, k, num_indexed_dims=nd, mode=m, brute_fallback=0))
+    (i0, d0, s0), (i1, d1, s1) = res
+    perm, _ = oracle.reorder(pts)
+    q = rng.choice(n, 300, replace=False)
+    bi, bd = oracle.bruteforce(np.ascontiguousarray(pts[:, perm]), k, queries=q)
+    assert np.array_equal(i1[q], bi) and np.array_equal(d1[q], bd)
+    assert np.array_equal(i0, i1) and np.array_equal(d0, d1)
+    if mode == "plain":
+        assert (s0.iterations, s0.reindexes, s0.eps0, s0.eps_final) == (s1.iterations, s1.reindexes, s1.eps0, s1.eps_final)
