@@ -1976,12 +1976,15 @@ int knnjoin_outlier_scores(const int32_t *ids, const float *dists, uint32_t n, u
       dD = b;
     }
     const size_t sw = radix_scratch_words(n) + 1024;
-    uint32_t *w = reinterpret_cast<uint32_t *>(g_cache.get(S_TRAIN, sizeof(uint32_t) * ((size_t)8 * n + sw)));
+    const OutlierPlan pl = outlier_plan(n, k1);
+    uint32_t *w = reinterpret_cast<uint32_t *>(g_cache.get(S_TRAIN, sizeof(uint32_t) * ((size_t)8 * n + sw + 4 + pl.words)));
     float *ds = reinterpret_cast<float *>(w);
     uint32_t *dr = w + n, *dg = w + 2 * (size_t)n, *gr = w + 3 * (size_t)n;
     uint32_t *k0 = w + 4 * (size_t)n, *v0 = w + 5 * (size_t)n, *k1t = w + 6 * (size_t)n, *v1t = w + 7 * (size_t)n;
     uint32_t *scr = w + 8 * (size_t)n;
-    outlier_scores(dIds, dD, n, k1, ds, dr, dg, gr, k0, v0, k1t, v1t, scr, s);
+    uint32_t *bins = scr + ((sw + 3) & ~(size_t)3);
+    outlier_scores(dIds, dD, n, k1, ds, dr, dg, gr, k0, v0, k1t, v1t, scr, pl, bins, pinned(), s);
+    LAUNCH_CHECK();
     const hipMemcpyKind kout = device_ptrs ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
     HIP_CHECK(hipMemcpyAsync(dist_sum, ds, sizeof(float) * n, kout, s));
     HIP_CHECK(hipMemcpyAsync(dist_rank, dr, sizeof(uint32_t) * n, kout, s));

@@ -67,3 +67,24 @@ def test_gpu_ties_ranked_by_id(oracle):
     want = oracle.outlier_scores(ids, d)
     for g, w in zip(got, want):
         assert np.array_equal(g, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k1", [
+    (70001, 60),      # just past the entry count from which the ids are dealt into bins
+    (600000, 7),      # bins of 2048 ids
+    (1 << 21, 2),     # every bin full
+    (2100000, 17),    # two slabs of rows
+])
+def test_gpu_indegrees_by_bins(oracle, n, k1):
+    rng = np.random.default_rng(n)
+    ids = rng.integers(0, n, (n, k1)).astype(np.int32)
+    ids[:, 0] = np.arange(n)
+    ids[::3, 1] = n - 1          # an in-degree past 16 bits, in the last bin
+    ids[::5, k1 - 1] = 0
+    d = np.round(rng.uniform(0, 2, (n, k1)), 2).astype(np.float32)
+    got = _lib.outlier_scores(ids, d)
+    want = np_outlier(ids, d)
+    assert np.array_equal(got[0].view(np.uint32), want[0].view(np.uint32))
+    for g, w in zip(got[1:], want[1:]):
+        assert np.array_equal(g, w)
