@@ -121,10 +121,28 @@ __global__ void k_prefilter(const T *__restrict__ xs, uint32_t n, G g, const T *
       hi[j] = cell_coord<T>(next_up(xj + r), (T)g.minArr[j], eps, g.nCells[j]);
       cur[j] = lo[j];
     }
-    do {
-      const uint64_t rowBase = row_base<ND>(g, cur);
-      cnt += dense[rowBase + hi[0] + 1] - dense[rowBase + lo[0]];
-    } while (next_row<ND>(cur, lo, hi, nd));
+    if (ND == 1) {
+      cnt = dense[g.keyBase + hi[0] + 1] - dense[g.keyBase + lo[0]];
+    } else {
+      // four rows along dim 1 at a time, their eight reads in flight together (the table has at
+      // most 2^28 entries)
+      const uint32_t m1 = nd > 1 ? (uint32_t)g.mult[1] : 0u;
+      const uint32_t l1 = nd > 1 ? lo[1] : 0u, h1 = nd > 1 ? hi[1] : 0u;
+      do {
+        const uint32_t base = (uint32_t)row_base<ND>(g, cur);  // (of row l1)
+        for (uint32_t c = 0; c <= h1 - l1; c += 4) {
+          uint32_t b[4], e[4];
+#pragma unroll
+          for (uint32_t u = 0; u < 4; u++) {
+            const uint32_t at = base + (c + u <= h1 - l1 ? c + u : c) * m1;
+            b[u] = dense[at + lo[0]];
+            e[u] = dense[at + hi[0] + 1];
+          }
+#pragma unroll
+          for (uint32_t u = 0; u < 4; u++) cnt += c + u <= h1 - l1 ? e[u] - b[u] : 0u;
+        }
+      } while (next_row<ND, 2>(cur, lo, hi, nd));
+    }
     if (tryR) {
       float est = (float)cnt * volD;  // points of the ball at the block's density
       const float reach = (float)(r / eps);
