@@ -167,7 +167,10 @@ template <typename T, int D, int ND, int H, bool SETS, typename G>
 __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G g0, GeoArgs<T, (ND > 0 ? ND : 1)> ga) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr bool TAB = ND == 1 || ND == 2;
-  constexpr int PR = TAB ? 2 : (D <= 4 ? 3 : (D <= 8 ? 2 : 1));
+  // rounds of a stream loaded together (ms per join with one more / one less: 1M skewed 6-D K=32 on 4
+  // dims 22.2 / 23.1 / 25.5, 2M uniform 6-D K=32 plain 23.1 / 22.9 / 23.7, 300k uniform 8-D K=16
+  // - / 15.0 / 16.9, 3M uniform 4-D K=32 plain 8.2 / 8.3 / 8.5)
+  constexpr int PR = TAB ? 2 : (D <= 4 ? 4 : (D <= 8 ? 3 : 1));
   constexpr uint32_t RM = ND == 1 ? 1 : DR_RMAX;
   constexpr uint32_t NW = windows(H), NWR = reg_windows(H);
   constexpr uint32_t CAP = list_cap(H, TAB);  // list slots
