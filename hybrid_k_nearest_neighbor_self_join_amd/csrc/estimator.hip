@@ -18,58 +18,47 @@ namespace knn {
 
 namespace {
 
-// One block per dim.  Waves 1..3 stage the sampled values (rows 0,100,...) of the next chunk
-// in LDS while lane 0 of wave 0 adds the current chunk in row order, so the sequential sum
-// (whose rounding decides the dimension order) runs at LDS rather than HBM latency.
-constexpr uint32_t VAR_CHUNK = 2048;
+// One block per dim.  Waves 1..15 stage the sampled values (rows 0,100,...) of the next chunk, in
+// the second pass their squared deviations, in LDS while lane 0 of wave 0 adds the current chunk in
+// row order, so the sequential sum (whose rounding decides the dimension order) runs at LDS rather
+// than HBM latency.  A staging thread has its chunk's loads in flight together.  5M 4-D points
+// (3 staging waves, one load after the other, squares in the chain: 0.93 ms): 0.62 ms.
+constexpr uint32_t VAR_THREADS = 1024;
 template <typename T>
+constexpr uint32_t var_chunk() { return 16384 / sizeof(T); }
+template <typename T, bool SQ>
 __device__ __forceinline__ void stage_chunk(const T *__restrict__ pts, uint32_t d, uint32_t i, uint64_t base,
-                                            uint32_t cnt, T *buf) {
+                                            uint32_t cnt, T avg, T *buf) {
   if (threadIdx.x < 64) return;
-  for (uint32_t t = threadIdx.x - 64; t < cnt; t += blockDim.x - 64)
-    buf[t] = pts[(base + t) * 100 * (uint64_t)d + i];
+  constexpr uint32_t W = VAR_THREADS - 64, U = (var_chunk<T>() + W - 1) / W;
+  T v[U];
+#pragma unroll
+  for (uint32_t u = 0; u < U; u++) {
+    const uint32_t t = threadIdx.x - 64 + W * u;
+    v[u] = pts[(base + (t < cnt ? t : 0u)) * 100 * (uint64_t)d + i];
+  }
+#pragma unroll
+  for (uint32_t u = 0; u < U; u++) {
+    const uint32_t t = threadIdx.x - 64 + W * u;
+    const T df = v[u] - avg;
+    const T sq = df * df;
+    if (t < cnt) buf[t] = SQ ? sq : v[u];
+  }
 }
 template <typename T, bool SQ>
 __device__ T sequential_pass(const T *__restrict__ pts, uint32_t n, uint32_t d, uint32_t i, T avg,
-                             T (*buf)[VAR_CHUNK]) {
+                             T (*buf)[var_chunk<T>()]) {
+  constexpr uint32_t C = var_chunk<T>();
   const uint64_t m = ((uint64_t)n + 99) / 100;
   T sum = 0;
   uint32_t cur = 0;
-  if (m) stage_chunk<T>(pts, d, i, 0, (uint32_t)(m < VAR_CHUNK ? m : VAR_CHUNK), buf[0]);
+  if (m) stage_chunk<T, SQ>(pts, d, i, 0, (uint32_t)(m < C ? m : C), avg, buf[0]);
   __syncthreads();
-  for (uint64_t base = 0; base < m; base += VAR_CHUNK) {
-    const uint32_t cnt = (uint32_t)(m - base < VAR_CHUNK ? m - base : VAR_CHUNK);
-    const uint64_t nb = base + VAR_CHUNK;
-    if (nb < m) stage_chunk<T>(pts, d, i, nb, (uint32_t)(m - nb < VAR_CHUNK ? m - nb : VAR_CHUNK), buf[cur ^ 1]);
-    if (threadIdx.x == 0) {
-      const T *b = buf[cur];
-      // 8 LDS reads issued ahead of 8 dependent adds (same order of additions)
-      uint32_t t = 0;
-      for (; t + 8 <= cnt; t += 8) {
-        T v[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = b[t + u];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-          if (SQ) {
-            T df = v[u] - avg;
-            T sq = df * df;
-            sum += sq;
-          } else {
-            sum += v[u];
-          }
-        }
-      }
-      for (; t < cnt; t++) {
-        if (SQ) {
-          T df = b[t] - avg;
-          T sq = df * df;
-          sum += sq;
-        } else {
-          sum += b[t];
-        }
-      }
-    }
+  for (uint64_t base = 0; base < m; base += C) {
+    const uint32_t cnt = (uint32_t)(m - base < C ? m - base : C);
+    const uint64_t nb = base + C;
+    if (nb < m) stage_chunk<T, SQ>(pts, d, i, nb, (uint32_t)(m - nb < C ? m - nb : C), avg, buf[cur ^ 1]);
+    if (threadIdx.x == 0) sum = ordered_sum(buf[cur], cnt, sum);
     __syncthreads();
     cur ^= 1;
   }
@@ -77,8 +66,8 @@ __device__ T sequential_pass(const T *__restrict__ pts, uint32_t n, uint32_t d, 
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_variance(const T *__restrict__ pts, uint32_t n, uint32_t d, T *var) {
-  __shared__ T buf[2][VAR_CHUNK];
+__global__ __launch_bounds__(VAR_THREADS) void k_variance(const T *__restrict__ pts, uint32_t n, uint32_t d, T *var) {
+  __shared__ __align__(16) T buf[2][var_chunk<T>()];
   __shared__ T shAvg;
   const uint32_t i = blockIdx.x;
   const T inv = (T)(1.0 / (100 * 1.0));
@@ -162,19 +151,30 @@ __global__ __launch_bounds__(256) void k_avg_seg(const T *__restrict__ x, uint32
 #pragma unroll
     for (uint32_t j = 0; j < KNN_MAXDIM; j++) q[j] = j < d ? x[(size_t)j * n + tid] : (T)0;
     const uint64_t i0 = (uint64_t)(g % 256) + 1000ull * L * sg;
-    for (uint32_t k = 0; k < L; k++) {
-      const uint64_t i = i0 + 1000ull * k;
-      if (i >= n) break;
-      double run = 0;
+    // (eight pairs' loads in flight per dim; 100k 2-D points: 36 us one at a time, now 14)
+    for (uint32_t k0 = 0; k0 < L; k0 += 8) {
+      if (i0 + 1000ull * k0 >= n) break;
+      double run[8] = {};
 #pragma unroll
       for (uint32_t j = 0; j < KNN_MAXDIM; j++) {
         if (j < d) {
-          T df = x[(size_t)j * n + i] - q[j];
-          T sq = df * df;
-          run += (double)sq;
+          T c[8];
+#pragma unroll
+          for (uint32_t u = 0; u < 8; u++) {
+            const uint64_t i = i0 + 1000ull * (k0 + u);
+            c[u] = x[(size_t)j * n + (i < n ? i : i0)];
+          }
+#pragma unroll
+          for (uint32_t u = 0; u < 8; u++) {
+            const T df = c[u] - q[j];
+            const T sq = df * df;
+            run[u] += (double)sq;
+          }
         }
       }
-      sum += sqrt(run);
+#pragma unroll
+      for (uint32_t u = 0; u < 8; u++)
+        if (k0 + u < L && i0 + 1000ull * (k0 + u) < n) sum += sqrt(run[u]);
     }
   }
   seg[item] = sum;
@@ -188,12 +188,14 @@ __global__ void k_avg_part(const double *seg, uint32_t G, uint32_t S, double *pa
   part[g] = t;
 }
 
-__global__ void k_avg_chunks(const double *part, uint32_t G, double *chunk) {
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= G / 256) return;
-  double t = 0;
-  for (uint32_t g = 256 * c; g < 256 * c + 256; g++) t += part[g];
-  chunk[c] = t;
+// one wave per chunk: 256 values to LDS, added in order (20 us as one thread's reads of global
+// memory, 100k points; now 3.5)
+__global__ __launch_bounds__(64) void k_avg_chunks(const double *part, double *chunk) {
+  __shared__ __align__(16) double buf[256];
+#pragma unroll
+  for (uint32_t u = 0; u < 4; u++) buf[threadIdx.x + 64 * u] = part[256u * blockIdx.x + threadIdx.x + 64 * u];
+  __syncthreads();
+  if (threadIdx.x == 0) chunk[blockIdx.x] = ordered_sum(buf, 256, 0.0);
 }
 
 __global__ void k_avg_total(const double *chunk, uint32_t C, double *total) {
@@ -205,34 +207,50 @@ __global__ void k_avg_total(const double *chunk, uint32_t C, double *total) {
 
 constexpr uint32_t NBUCKETS = 10000;
 
-// kernel.cu:450-523: sample s = blockIdx.x / KD_PARTS (point s * offset) against the first
-// 256 points of every 2048, +8 per hit in bucket floor(d / bw) for d < avg (self excluded).
-// The counts are integers, so the partition is free: each sample's 2048-point strides are
-// dealt to KD_PARTS blocks, and a thread loads KD_UNROLL strides before it bins any.  Built
-// per dimensionality D (the coordinates in registers, no per-dim predication); a pair whose
-// squared distance is at or above avg^2 (1 + 2^-40) has a rounded root >= avg and skips the
-// root and the division.
-constexpr uint32_t KD_PARTS = 2, KD_UNROLL = 4;
+// kernel.cu:450-523: sample s (point s * offset) against the first 256 points of every 2048, +8
+// per hit in bucket floor(d / bw) for d < avg (self excluded).  The counts are integers, so the
+// partition is free: groups of KS samples share each point they load, a group's 2048-point strides
+// are dealt to `parts` units, and up to 256 blocks of 1024 threads take units in turn (four strides
+// at a time, KD_UNROLL loads per thread in flight), so that the 10,000 counters are cleared and
+// added up once per block.  Built per dimensionality D (the coordinates in registers, no per-dim
+// predication).
+// d / bw comes from an FP32 root with one FP64 Newton step, within 2^-40: only where that leaves
+// the bucket, or d < avg, open (and for sums outside the FP32 range) are the root and the quotient
+// rounded as the reference's.  10M 2-D points 1.16 ms (a block per sample and half,
+// every root and quotient rounded) / 0.68, 2M 6-D 0.31 / 0.20, 100k 2-D 0.047 / 0.028.
+constexpr uint32_t KD_BLOCKS = 256;
 template <typename T, int D>
-__global__ __launch_bounds__(256) void k_kdist(const T *__restrict__ x, uint32_t n, uint32_t offset,
-                                               double avg, double bw, uint32_t *hist) {
+constexpr uint32_t kd_samples() { return D * sizeof(T) <= 32 ? 4 : (D * sizeof(T) <= 64 ? 2 : 1); }
+template <typename T, int D>
+__global__ __launch_bounds__(1024) void k_kdist(const T *__restrict__ x, uint32_t n, uint32_t offset,
+                                                uint32_t nsample, uint32_t parts, double avg, double bw,
+                                                uint32_t *hist) {
   __shared__ uint32_t lh[NBUCKETS];
-  for (uint32_t b = threadIdx.x; b < NBUCKETS; b += 256) lh[b] = 0;
+  for (uint32_t b = threadIdx.x; b < NBUCKETS; b += 1024) lh[b] = 0;
   __syncthreads();
-  const uint64_t tid = (uint64_t)(blockIdx.x / KD_PARTS) * offset;
-  const uint32_t part = blockIdx.x % KD_PARTS;
+  constexpr uint32_t KS = kd_samples<T, D>(), KD_UNROLL = KS > 2 ? 4 : 2;
   const double cut2 = avg * avg * (1.0 + 0x1p-40);
-  if (tid < n) {
-    T q[D];
+  const double invbw = 1.0 / bw;
+  const uint32_t col = threadIdx.x & 255u, row = threadIdx.x >> 8;
+  const uint32_t units = (nsample + KS - 1) / KS * parts;
+  for (uint32_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
+    const uint32_t s0 = unit / parts * KS, part = unit % parts;
+    T q[KS][D];
+    uint64_t tid[KS];
 #pragma unroll
-    for (int j = 0; j < D; j++) q[j] = x[(size_t)j * n + tid];
-    const uint64_t step = 2048ull * KD_PARTS;
-    for (uint64_t i0 = 2048ull * part; i0 < n; i0 += step * KD_UNROLL) {
+    for (uint32_t k = 0; k < KS; k++) {
+      const bool have = s0 + k < nsample && (uint64_t)(s0 + k) * offset < n;
+      tid[k] = have ? (uint64_t)(s0 + k) * offset : ~0ull;
+#pragma unroll
+      for (int j = 0; j < D; j++) q[k][j] = x[(size_t)j * n + (have ? tid[k] : 0)];
+    }
+    const uint64_t step = 2048ull * parts * 4;  // between a thread's strides
+    for (uint64_t i0 = 2048ull * (part + parts * row); i0 < n; i0 += step * KD_UNROLL) {
       T c[KD_UNROLL][D];
       bool ok[KD_UNROLL];
 #pragma unroll
       for (uint32_t u = 0; u < KD_UNROLL; u++) {
-        const uint64_t p = i0 + step * u + threadIdx.x;
+        const uint64_t p = i0 + step * u + col;
         ok[u] = p < n;
         const uint64_t pc = ok[u] ? p : (uint64_t)n - 1;
 #pragma unroll
@@ -240,25 +258,35 @@ __global__ __launch_bounds__(256) void k_kdist(const T *__restrict__ x, uint32_t
       }
 #pragma unroll
       for (uint32_t u = 0; u < KD_UNROLL; u++) {
-        const uint64_t p = i0 + step * u + threadIdx.x;
-        double run = 0;
+        const uint64_t p = i0 + step * u + col;
 #pragma unroll
-        for (int j = 0; j < D; j++) {
-          T df = c[u][j] - q[j];
-          T sq = df * df;
-          run += (double)sq;
-        }
-        if (!ok[u] || !(run < cut2) || p == tid) continue;
-        run = sqrt(run);
-        if (run < avg) {
-          uint32_t bucket = (uint32_t)(run / bw);
-          if (bucket < NBUCKETS) atomicAdd(&lh[bucket], 8u);
+        for (uint32_t k = 0; k < KS; k++) {
+          double run = 0;
+#pragma unroll
+          for (int j = 0; j < D; j++) {
+            T df = c[u][j] - q[k][j];
+            T sq = df * df;
+            run += (double)sq;
+          }
+          if (!ok[u] || !(run < cut2) || p == tid[k] || tid[k] == ~0ull) continue;
+          const float f = (float)run;
+          const double y = (double)__builtin_amdgcn_sqrtf(f);
+          const double t = __builtin_fma(__builtin_fma(-y, y, run), 0.5 * (double)__builtin_amdgcn_rcpf((float)y), y) * invbw;
+          uint32_t bucket = (uint32_t)t;
+          const double frac = t - (double)bucket;
+          if (!(f > 1e-30f && f < 1e30f && t < NBUCKETS - 0.01 && frac > 1e-6 && frac < 1.0 - 1e-6)) {
+            run = sqrt(run);
+            if (!(run < avg)) continue;
+            bucket = (uint32_t)(run / bw);
+            if (bucket >= NBUCKETS) continue;
+          }
+          atomicAdd(&lh[bucket], 8u);
         }
       }
     }
   }
   __syncthreads();
-  for (uint32_t b = threadIdx.x; b < NBUCKETS; b += 256)
+  for (uint32_t b = threadIdx.x; b < NBUCKETS; b += 1024)
     if (lh[b]) atomicAdd(&hist[b], lh[b]);
 }
 
@@ -266,7 +294,7 @@ __global__ __launch_bounds__(256) void k_kdist(const T *__restrict__ x, uint32_t
 
 template <typename T>
 void variance_rows(const T *pts, uint32_t n, uint32_t d, T *var, hipStream_t s) {
-  k_variance<T><<<d, 256, 0, s>>>(pts, n, d, var);
+  k_variance<T><<<d, VAR_THREADS, 0, s>>>(pts, n, d, var);
 }
 
 template <typename T>
@@ -320,7 +348,7 @@ void avg_dist_soa(const T *x, uint32_t n, uint32_t d, double *scratch, double *t
   const uint64_t items = (uint64_t)G * S;
   k_avg_seg<T><<<(uint32_t)((items + 255) / 256), 256, 0, s>>>(x, n, d, G, S, a.L, seg);
   k_avg_part<<<(G + 255) / 256, 256, 0, s>>>(seg, G, S, part);
-  k_avg_chunks<<<(G / 256 + 255) / 256, 256, 0, s>>>(part, G, chunk);
+  k_avg_chunks<<<G / 256, 64, 0, s>>>(part, chunk);
   k_avg_total<<<1, 64, 0, s>>>(chunk, G / 256, total);
 }
 
@@ -336,10 +364,15 @@ void kdist_hist_soa(const T *x, uint32_t n, uint32_t d, uint32_t offset, uint32_
                     double avg, double bw, uint32_t *hist, hipStream_t s) {
   fill_u32(hist, 0u, NBUCKETS, s);
   if (!nsample) return;
-  const uint32_t grid = nsample * KD_PARTS;
+  // strides per unit: at least the block's four, and enough units to even out 256 blocks
+  const uint32_t strides = (n + 2047) / 2048, parts = std::max(1u, std::min(strides / 4, 16u));
   switch (d) {
 #define KD_CASE(DD) \
-    case DD: k_kdist<T, DD><<<grid, 256, 0, s>>>(x, n, offset, avg, bw, hist); break;
+    case DD: { \
+      const uint32_t units = (nsample + kd_samples<T, DD>() - 1) / kd_samples<T, DD>() * parts; \
+      k_kdist<T, DD><<<std::min(units, KD_BLOCKS), 1024, 0, s>>>(x, n, offset, nsample, parts, avg, bw, hist); \
+      break; \
+    }
     KD_CASE(1) KD_CASE(2) KD_CASE(3) KD_CASE(4) KD_CASE(5) KD_CASE(6) KD_CASE(7) KD_CASE(8)
     KD_CASE(9) KD_CASE(10) KD_CASE(11) KD_CASE(12) KD_CASE(13) KD_CASE(14) KD_CASE(15) KD_CASE(16)
 #undef KD_CASE

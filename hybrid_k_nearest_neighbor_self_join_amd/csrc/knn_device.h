@@ -171,4 +171,31 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   return v;
 }
 
+// s + b[0] + b[1] + ... in that order (b in LDS, 16-byte aligned): one lane's chain of dependent
+// additions, with the next 32 values read while 32 are added.
+template <typename T>
+__device__ __forceinline__ T ordered_sum(const T *b, uint32_t cnt, T s) {
+  constexpr uint32_t U = 32;
+  uint32_t t = 0;
+  if (cnt >= U) {
+    T v[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) v[u] = b[u];
+    for (; t + 2 * U <= cnt; t += U) {
+      T w[U];
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) w[u] = b[t + U + u];
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) s += v[u];
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) v[u] = w[u];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) s += v[u];
+    t += U;
+  }
+  for (; t < cnt; t++) s += b[t];
+  return s;
+}
+
 }  // namespace knn

@@ -218,3 +218,31 @@ def test_both_range_kernels_match_oracle(oracle, monkeypatch, kernel, d, nd, k, 
     assert rc == 0
     assert np.array_equal(ids, i2)
     assert np.array_equal(bits(dist), bits(d2))
+
+
+@pytest.mark.parametrize("n,d", [(1001, 1), (8191, 2), (8193, 8), (66000, 9), (50001, 16)])
+@pytest.mark.parametrize("scale", [1.0, 1e-17, 1e17])
+def test_estimator_edges(oracle, n, d, scale):
+    # strides of the sample pass around a block's four, the sample groups of 4, 2 and 1, lattice
+    # distances on bucket edges, equal points, and squares outside the FP32 range of its fast root
+    rng = np.random.default_rng(n + d)
+    pts = (np.round(rng.random((n, d)) * 64) / 64 * scale).astype(np.float32)
+    pts[n // 2: n // 2 + 300] = pts[0]
+    eps, avg, cnt, bucket, hist = _lib.stage_estimate_eps(pts, 8, 0.025)
+    rc, info, h2 = oracle.estimate_eps(pts, 8, 0.025)
+    assert rc == 0
+    assert cnt == info.cnt and avg == info.avg
+    assert np.array_equal(hist, h2)
+    assert bucket == info.bucket and eps == info.eps
+
+
+@pytest.mark.parametrize("n,d", [(409601, 3), (409501, 2), (1700, 16), (99, 5), (3201, 4)])
+def test_sequential_variance_edges(oracle, n, d):
+    # sampled rows at, one past and below a staged chunk and the chain's 32 values in flight; equal
+    # spreads, so that the order of the dims needs the sequential sums
+    rng = np.random.default_rng(n)
+    pts = rng.random((n, d)).astype(np.float32)
+    perm, var = _lib.stage_reorder(pts)
+    p2, v2 = oracle.reorder(pts)
+    assert list(perm) == list(p2)
+    assert np.array_equal(bits(var), bits(v2))
