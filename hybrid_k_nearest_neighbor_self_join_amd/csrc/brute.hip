@@ -161,7 +161,10 @@ __global__ __launch_bounds__(1024) void k_brute_sample(BruteArgs a) {
   if (tid == 0) a.bound[qi] = (double)__uint_as_float(prefix < 0x7f800000u ? prefix + 1u : prefix);
 }
 
-template <typename T, int D>
+// U: rounds of points loaded together.  Several for a tail of few queries, whose waves wait for
+// memory; one for a whole join, whose waves are many and bound by issue (28,903 uniform 4-D points,
+// K=8: 1.25 ms, with four rounds 1.35).
+template <typename T, int D, uint32_t U>
 __global__ __launch_bounds__(64) void k_brute_partial(BruteArgs a) {
   extern __shared__ __align__(16) unsigned char br_lds[];
   const uint32_t lane = threadIdx.x;
@@ -195,7 +198,6 @@ __global__ __launch_bounds__(64) void k_brute_partial(BruteArgs a) {
   const uint64_t c0 = (uint64_t)chunk * a.chunk;
   const uint32_t p0 = (uint32_t)c0;
   const uint32_t p1 = c0 + a.chunk < a.n ? (uint32_t)(c0 + a.chunk) : a.n;
-  constexpr uint32_t U = D <= 4 ? 4 : (D <= 8 ? 2 : 1);  // rounds loaded together
   for (uint32_t base = p0; base < p1; base += 64 * U) {
     T c[U][D];
 #pragma unroll
@@ -280,7 +282,9 @@ void launch_brute(const BruteArgs &a, hipStream_t s) {
   const uint64_t blocks = (uint64_t)tiles * a.nchunks;
   if (a.nchunks > 1) fill_u32(a.partCount, 0u, a.nq, s);
   if (a.bound) k_brute_sample<T, D><<<a.nq, 1024, 0, s>>>(a);
-  k_brute_partial<T, D><<<(uint32_t)blocks, 64, br_lds_bytes(a.k1, a.qw), s>>>(a);
+  constexpr uint32_t U = D <= 4 ? 4 : (D <= 8 ? 2 : 1);
+  auto partial = a.bound ? k_brute_partial<T, D, U> : k_brute_partial<T, D, 1>;
+  partial<<<(uint32_t)blocks, 64, br_lds_bytes(a.k1, a.qw), s>>>(a);
   if (a.nchunks > 1) k_brute_merge<T, D><<<a.nq, 64, br_lds_bytes(a.k1, 1), s>>>(a);
 }
 
