@@ -113,7 +113,7 @@ def load_traffic(workload_key: str):
     """HBM bytes per launch of the range kernel measured with rocprofv3 PMC counters
     (FETCH_SIZE / WRITE_SIZE, scaled by the same counters' reading on a copy of known size),
     committed beside the profile summaries; None when no measurement of this workload exists."""
-    path = os.path.join(ROOT, "profiles", "k_select_traffic.json")
+    path = os.path.join(ROOT, "profiles", "k_direct_traffic.json")
     try:
         with open(path) as f:
             e = json.load(f).get(workload_key)
@@ -127,7 +127,7 @@ def load_counters(workload_key: str):
     measurement (SQ_INSTS_VALU, SQ_WAVES, SQ_BUSY_CYCLES, ...): VALU wave instructions per
     launch, the fraction of the VALU issue peak they use at the traced launch time, and VALU
     lane instructions per (query, candidate) pair; None when no measurement exists."""
-    path = os.path.join(ROOT, "profiles", "k_select_counters.json")
+    path = os.path.join(ROOT, "profiles", "k_direct_counters.json")
     try:
         with open(path) as f:
             return json.load(f).get(workload_key)
@@ -422,7 +422,7 @@ def main():
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": tr["bytes_per_launch"] if tr else None,
-            "kernel": "k_select",
+            "kernel": "k_direct",
             "algo_bytes_per_launch": g["algo_bytes"] / launches,
             "avg_launch_ms": g["kernel_ms"] / launches,
             "launches_per_step": g["kernel_launches"] / max(args.steps, 1),
