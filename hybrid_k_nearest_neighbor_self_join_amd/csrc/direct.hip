@@ -205,7 +205,7 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
     return a.sortedIds[p];
   };
   uint32_t Q;
-  const uint32_t NT = work_count(a, TAB ? 1u : 4u, Q);
+  const uint32_t NT = work_count(a, TAB ? 1u : 4u, ND >= 1 && ND <= 4, Q);
   WaveTally tally;
   for (;;) {
     const uint32_t t = next_tile(a.tileCounter, NT, a.tileRanges, lane);

@@ -374,14 +374,16 @@ __device__ __forceinline__ uint32_t tile_count(const JoinArgs &a) {
 // Work units of a wave = query kernel: the tiles (batched groups), or, without tiles, chunks of Q
 // consecutive active queries, Q small enough for every wave of the launch to take `per` of them
 // (a pass of few queries then still fills the chip) and at most 64.
-__device__ __forceinline__ uint32_t work_count(const JoinArgs &a, uint32_t per, uint32_t &Q) {
+// `even` (queries of up to 4 indexed dims): as many whole turns as that takes, and with few queries
+// one chunk per wave, since a chunk's set-up costs as much as such a query (26,849 uniform 3-D double
+// points, K=7, one query per chunk: 1.88 ms per join, now 1.62).  Queries of more dims are long and
+// uneven, and are dealt one by one (1M skewed 6-D points on 4 dims: 26.2 ms in even turns, 24.8 so).
+__device__ __forceinline__ uint32_t work_count(const JoinArgs &a, uint32_t per, bool even, uint32_t &Q) {
   Q = 64;
   if (a.tiles) return tile_count(a);
   const uint32_t A = *a.activeCount, W = gridDim.x;
-  // few queries: one chunk per wave, since a chunk's set-up costs as much as a short query (26,849
-  // uniform 3-D double points, K=7, one query per chunk: 1.88 ms per join, now 1.62)
-  if (A <= 8u * W) per = 1u;
-  Q = A / (W * per) + (A % (W * per) ? 1u : 0u);
+  if (even && A <= 8u * W) per = 1u;
+  Q = A / (W * per) + (even && A % (W * per) ? 1u : 0u);
   Q = Q < 1u ? 1u : (Q > 64u ? 64u : Q);
   return (A + Q - 1u) / Q;
 }

@@ -37,7 +37,7 @@ __global__ __launch_bounds__(64) void k_range_collect(JoinArgs a, G g0) {
   const T *__restrict__ x = reinterpret_cast<const T *>(a.x);
   const size_t n = a.n;
   uint32_t Q;
-  const uint32_t NT = work_count(a, 4u, Q);
+  const uint32_t NT = work_count(a, 4u, false, Q);
   constexpr int PR = D <= 8 ? 4 : 2;
   WaveTally tally;
   for (;;) {
