@@ -1320,12 +1320,14 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
 
   // ---- the join loop (main.cu:305-430)
   T curW = (T)0;
-  uint32_t curDims = nd;
+  double reach = 1.0;  // cells of radius up to which the index is kept
   auto build = [&](T e) -> double {
     const uint64_t small = std::min<uint64_t>(Pipeline<T>::kDenseMaxCells - 1, 16ull * n + (1u << 20));
     uint32_t gd = P.max_grid_dims();
     while (gd > nd && !P.grid_fits(hmn, hmx, gd, (T)((double)e / plain_grid_div(d, gd, K1)), small)) gd--;
-    const double pdiv = plain_grid_div(d, gd, K1);
+    // (the hybrid split judges the cells of the first index, which are eps0 wide)
+    const bool split = prm.hybrid_threads && curW == (T)0;
+    const double pdiv = split ? 1.0 : plain_grid_div(d, gd, K1);
     T w = (T)((double)e / pdiv);
     // a finer grid only while its dense start table stays small beside the points
     if (pdiv > 1.0 && !P.grid_fits(hmn, hmx, gd, w, small)) w = e;
@@ -1334,7 +1336,7 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
     P.build_index(hmn, hmx, gd, w);
     P.tBuild = nullptr;
     curW = w;
-    curDims = gd;
+    reach = split ? std::min(plain_max_reach(d, gd, K1), 2.0) : plain_max_reach(d, gd, K1);
     return tPh.elapsed();
   };
   P.radius = nullptr;  // every query searches the same radius, passed by value
@@ -1367,7 +1369,7 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
           throw Error(KNN_ERR_NO_PROGRESS, "eps + eps0/2 == eps: epsilon cannot grow");
         }
         eps = grown;
-        if ((double)eps > plain_max_reach(d, curDims, K1) * (double)curW) stats.ms_index += build(eps);
+        if ((double)eps > reach * (double)curW) stats.ms_index += build(eps);
         reindexes++;  // the reference's re-index count: eps growths
       } else {
         // The reference reruns the failed queries at the same eps (main.cu:330 is false);

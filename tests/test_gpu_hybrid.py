@@ -1,6 +1,8 @@
 """GPU tests of the hybrid CPU/GPU split (splitWork, main.cu:2733-2933): the queries of the
 sparse cells of the first grid are joined by host threads concurrently with the GPU's
 failed-query loop over the others; every row equals the oracle's."""
+import math
+
 import numpy as np
 import pytest
 
@@ -56,3 +58,32 @@ def test_hybrid_needs_the_beta_schedule():
     with pytest.raises(_lib.KnnError) as e:
         _lib.knnjoin_ex(pts, 8, mode=_lib.KNN_MODE_LEARNED, hybrid_threads=4)
     assert e.value.code == _lib.KNN_ERR_ARG
+
+
+def _sparse_cell_queries(pts, nd, k, eps0):
+    """Points whose cell of the grid of width eps0 over the first nd dims (variance order) holds
+    at most ceil((K+1) 2^nd / V_nd) points, in the index's arithmetic."""
+    f = pts.dtype.type
+    eps0 = f(eps0)
+    cell = np.zeros(len(pts), np.int64)
+    tot = 1
+    for j in range(nd):
+        lo, hi = pts[:, j].min() - eps0, pts[:, j].max() + eps0
+        nc = int(np.ceil((hi - lo) / eps0))
+        cell += np.minimum(((pts[:, j] - lo) / eps0).astype(np.int64), nc - 1) * tot
+        tot *= nc
+    _, at, cnt = np.unique(cell, return_inverse=True, return_counts=True)
+    ball = math.pi ** (nd / 2) / math.gamma(nd / 2 + 1)
+    return int(np.count_nonzero(cnt[at] <= math.ceil((k + 1) * (2 ** nd / ball))))
+
+
+@pytest.mark.parametrize("gen,n,d,nd,k", [("mixed", 60_000, 2, 2, 16), ("mixed", 60_000, 2, 2, 8),
+                                          ("mixed", 60_000, 2, 2, 32), ("skewed", 60_000, 4, 2, 32),
+                                          ("skewed", 40_000, 4, 4, 16)])
+def test_hybrid_host_share_is_the_sparse_cells_of_width_eps0(oracle, gen, n, d, nd, k):
+    # the split's threshold is the population of a cell whose side is the radius eps0: on the
+    # finer cells of the GPU passes nearly every query would count as sparse
+    pts = synthetic.mixed_box(n, seed=45) if gen == "mixed" else synthetic.skewed_cube(n, d, seed=45)
+    perm, _ = oracle.reorder(pts)
+    st = _check(oracle, pts, k, nd=nd, hybrid_threads=8)
+    assert st.hybrid_queries == _sparse_cell_queries(pts[:, perm], nd, k, st.eps0)
