@@ -2274,6 +2274,7 @@ struct BatchPlan {
   uint32_t tq = 64, grid = 2048, passes = 3;
   int reorder = 1;
   bool useGraph = true;
+  std::vector<uint32_t> routes;  // batch_routes at the capture
   template <typename U>
   U *alloc(size_t count) {
     void *p = nullptr;
@@ -2466,6 +2467,19 @@ static JoinArgs batch_args(const BatchPlan &B, const BatchGroup &G) {
   return a;
 }
 
+// What the launches of a pass take from the environment: a captured graph keeps the kernels and
+// operands it was captured with.
+static std::vector<uint32_t> batch_routes(const BatchPlan &B) {
+  std::vector<uint32_t> r{seg_cap_log2()};
+  for (const BatchGroup &G : B.groups) {
+    r.push_back((uint32_t)range_kernel(G.k1max));
+    r.push_back(overflow_by_collect(G.k1max) ? 1u : 0u);
+    r.push_back(lookup_rows(G.hsets[0].nd));
+    r.push_back(tile_ranges(G.d, true));
+  }
+  return r;
+}
+
 // Index of a group at the sets' current widths (classes: those of their lowest pending radius class): per-set grids, cell keys, radix sort, cell
 // table, cell-sorted coordinates, dense cell-start table.
 static void batch_index(BatchGroup &G, bool classes, hipStream_t s) {
@@ -2616,9 +2630,11 @@ static int run_batched(uint32_t nsets, const float *const *points, const uint32_
     if (st) *st = stats;
     return KNN_OK;
   }
+  std::vector<uint32_t> routes = batch_routes(B);
   if (B.tq != tq || B.grid != grid || B.passes != passes || B.reorder != (p.reorder ? 1 : 0) ||
-      B.useGraph != (p.use_graph != 0)) {
+      B.useGraph != (p.use_graph != 0) || B.routes != routes) {
     B.drop_graphs();
+    B.routes.swap(routes);
     B.tq = tq;
     B.grid = grid;
     B.passes = passes;

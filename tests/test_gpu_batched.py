@@ -177,3 +177,25 @@ def test_batched_set_boundaries(nsets, d, oracle):
             bi, bd = oracle.bruteforce(np.ascontiguousarray(p_[:, perm]), k, queries=q)
             assert np.array_equal(ids[i][q], bi), f"set {i}: n={len(p_)} k={k} graph={graph}"
             assert np.array_equal(bits(dists[i][q]), bits(bd)), f"set {i}"
+
+
+@pytest.mark.parametrize("knob,value", [("KNN_RANGE_KERNEL", "collect"), ("KNN_OVERFLOW_KERNEL", "heap"),
+                                        ("KNN_TILE_ROWS", "1"), ("KNN_SEG_CHUNK_LOG2", "6"),
+                                        ("KNN_TILE_RANGES", "8")])
+def test_batched_graphs_follow_the_kernel_switches(monkeypatch, knob, value):
+    # a switch that picks another kernel or operand: graphs captured without it are not replayed
+    rng = np.random.default_rng(31)
+    sets = [(np.concatenate([np.full((2000, 2), 0.5, np.float32), rng.random((1500, 2)).astype(np.float32)]), 16),
+            (rng.random((5000, 2)).astype(np.float32), 8), (rng.random((3000, 4)).astype(np.float32), 8)]
+    pts, ks = [s for s, _ in sets], [k for _, k in sets]
+    batched.knnjoin_batched(pts, ks)
+    assert batched.knnjoin_batched(pts, ks)[2].graph_replayed == 1
+    for replay in (0, 1):
+        with monkeypatch.context() as m:
+            m.setenv(knob, value)
+            ids, dists, st = batched.knnjoin_batched(pts, ks)
+        assert st.graph_replayed == replay
+        _check_against_single(sets, ids, dists)
+    ids, dists, st = batched.knnjoin_batched(pts, ks)
+    assert st.graph_replayed == 0
+    _check_against_single(sets, ids, dists)
