@@ -1,8 +1,9 @@
 """Batched joins of many independent point sets (knnjoin_batched / knnjoin_batch_autotune).
 
-Each set gets exactly the rows `knnjoin_ex` gives it alone; the library joins all sets of one
-dimensionality together (one index, one persistent range-kernel launch per radius pass) and
-replays a captured hipGraph of the whole join for calls with the same set shapes.
+Each set gets exactly the rows `knnjoin_ex` gives it alone; the library joins the sets of one
+dimensionality whose K takes the same range kernel together (one index, one persistent
+range-kernel launch per radius pass) and replays captured hipGraphs of the passes for calls with
+the same set shapes.
 
     ids, dists, stats = batched.knnjoin_batched([pts0, pts1, ...], [k0, k1, ...])
 """

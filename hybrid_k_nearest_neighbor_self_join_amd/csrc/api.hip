@@ -2239,7 +2239,12 @@ struct BatchGraph {
   hipGraphExec_t exec = nullptr;
 };
 
+// The sets of one dimensionality whose K+1 takes the same range kernel: one set of long rows does
+// not send the others to its kernel (6 sets of 200k points with K=16 and one of 600 with K=460,
+// ms_device with one group / two: 2-D 5.0 / 2.1, 4-D 8.8 / 5.9, 6-D 14.9 / 10.8; one of 2,200 with
+// K=2100: 19.3 / 16.1, 50.1 / 31.9, 98.6 / 45.3).
 struct BatchGroup {
+  RangeKernel kernel = RK_DIRECT;
   uint32_t d = 0, nsets = 0, N = 0, k1max = 0;
   uint64_t outElems = 0, bound = 0;
   int bits = 0;
@@ -2271,10 +2276,13 @@ struct BatchPlan {
   std::vector<void *> allocs;
   uint32_t *pin = nullptr;  // pinned, 2 words per group: overflowed and pending queries of a pass
   bool captured = false;
-  uint32_t tq = 64, grid = 2048, passes = 3;
+  uint32_t tq = 0, grid = 2048, passes = 3;  // tq 0: tile_queries' own choice
   int reorder = 1;
   bool useGraph = true;
   std::vector<uint32_t> routes;  // batch_routes at the capture
+  // queries per tile: whole chunks of 64 for the direct kernel, which looks all their rows up at
+  // once; 16-query tiles of one cell for the others
+  uint32_t tile_queries(const BatchGroup &G) const { return tq ? tq : (G.kernel == RK_DIRECT ? 64u : 16u); }
   template <typename U>
   U *alloc(size_t count) {
     void *p = nullptr;
@@ -2343,10 +2351,23 @@ static uint32_t g_tunedTq = 0, g_tunedGrid = 0;
 
 constexpr uint32_t kBatchMaxGrid = 8192;
 
+// What a plan is laid out for: the sets' shapes, their K and the range kernel each takes.
+static std::vector<uint64_t> batch_signature(uint32_t nsets, const uint32_t *n, const uint32_t *ndim,
+                                             const uint32_t *k, uint32_t ndParam) {
+  std::vector<uint64_t> sig;
+  sig.reserve((size_t)nsets * 2 + 1);
+  for (uint32_t i = 0; i < nsets; i++) {
+    sig.push_back(((uint64_t)range_kernel(k[i] + 1) << 32) | n[i]);
+    sig.push_back(((uint64_t)ndim[i] << 32) | k[i]);
+  }
+  sig.push_back(ndParam);
+  return sig;
+}
+
 static void batch_build(BatchPlan &B, uint32_t nsets, const uint32_t *n, const uint32_t *ndim,
                         const uint32_t *k, uint32_t ndParam, hipStream_t s) {
   B.free_all();
-  std::vector<int> groupOf(KNN_MAXDIM + 1, -1);
+  std::vector<int> groupOf(3 * (KNN_MAXDIM + 1), -1);
   for (uint32_t si = 0; si < nsets; si++) {
     const uint32_t d = ndim[si];
     if (d == 0 || d > KNN_MAXDIM) throw Error(KNN_ERR_ARG, "set dimensionality must be in 1..16");
@@ -2355,12 +2376,15 @@ static void batch_build(BatchPlan &B, uint32_t nsets, const uint32_t *n, const u
     if (n[si] != 0 && (uint64_t)n[si] < (uint64_t)k[si] + 1)
       throw Error(KNN_ERR_TOO_FEW, "a set has fewer than K+1 points");
     if (n[si] == 0) continue;
-    if (groupOf[d] < 0) {
-      groupOf[d] = (int)B.groups.size();
+    const RangeKernel rk = range_kernel(k[si] + 1);
+    int &gi = groupOf[3 * d + rk];
+    if (gi < 0) {
+      gi = (int)B.groups.size();
       B.groups.emplace_back();
       B.groups.back().d = d;
+      B.groups.back().kernel = rk;
     }
-    BatchGroup &G = B.groups[groupOf[d]];
+    BatchGroup &G = B.groups[gi];
     SetDesc sd{};
     sd.pStart = G.N;
     sd.n = n[si];
@@ -2423,7 +2447,7 @@ static void batch_build(BatchPlan &B, uint32_t nsets, const uint32_t *n, const u
     G.outIds = B.alloc<int32_t>(G.outElems);
     G.outDists = B.alloc<float>(G.outElems);
     const size_t heapBytes = (size_t)G.k1max * 64 * 12;
-    G.heap = heapBytes > 65536 ? B.alloc<unsigned char>(heapBytes * kBatchMaxGrid) : nullptr;
+    G.heap = heapBytes > 65536 && G.kernel != RK_COLLECT ? B.alloc<unsigned char>(heapBytes * kBatchMaxGrid) : nullptr;
     std::vector<uint32_t> so(N);
     for (uint32_t i = 0; i < G.nsets; i++)
       std::fill(so.begin() + G.hsets[i].pStart, so.begin() + G.hsets[i].pStart + G.hsets[i].n, i);
@@ -2472,7 +2496,6 @@ static JoinArgs batch_args(const BatchPlan &B, const BatchGroup &G) {
 static std::vector<uint32_t> batch_routes(const BatchPlan &B) {
   std::vector<uint32_t> r{seg_cap_log2()};
   for (const BatchGroup &G : B.groups) {
-    r.push_back((uint32_t)range_kernel(G.k1max));
     r.push_back(overflow_by_collect(G.k1max) ? 1u : 0u);
     r.push_back(lookup_rows(G.hsets[0].nd));
     r.push_back(tile_ranges(G.d, true));
@@ -2512,14 +2535,14 @@ static void batch_pass(const BatchPlan &B, BatchGroup &G, hipStream_t s) {
   scan_exclusive_u32(G.aflags, G.apos, N, G.scratch, s);
   compact_active(G.ids, G.aflags, G.apos, N, G.act, s);
   fill_u32(G.ctr, 0u, 8 + TILE_QUEUES, s);
-  const RangeKernel rk = range_kernel(G.k1max);
-  if (rk == RK_DIRECT) {
-    batch_chunks(G.sets, G.nsets, g0.nd, G.apos, N, B.grid, B.tq, G.chunkOff, G.tileOff + N + 1, G.ctr + 4, G.tiles,
+  const uint32_t tq = B.tile_queries(G);
+  if (G.kernel == RK_DIRECT) {
+    batch_chunks(G.sets, G.nsets, g0.nd, G.apos, N, B.grid, tq, G.chunkOff, G.tileOff + N + 1, G.ctr + 4, G.tiles,
                  s);
     range_direct<float>(a, g0, s);
   } else {
-    batch_tiles(G.cellStart, G.apos, G.cpos + N, N, B.tq, G.ntiles, G.tileOff, G.scratch, G.tiles, s);
-    if (rk == RK_COLLECT)
+    batch_tiles(G.cellStart, G.apos, G.cpos + N, N, tq, G.ntiles, G.tileOff, G.scratch, G.tiles, s);
+    if (G.kernel == RK_COLLECT)
       range_collect<float>(a, g0, s);
     else
       range_topk<float>(a, g0, s);
@@ -2528,7 +2551,7 @@ static void batch_pass(const BatchPlan &B, BatchGroup &G, hipStream_t s) {
                    G.setMinBin, s);
 }
 
-// The queries the range kernel of the last pass could not list, on the overflow kernel, and the
+// The queries the direct kernel of the last pass could not list, on the overflow kernel, and the
 // radius growth of those that failed there; G.ctr[3] = queries still pending.
 static void batch_overflow(const BatchPlan &B, BatchGroup &G, hipStream_t s) {
   const uint32_t N = G.N;
@@ -2538,7 +2561,7 @@ static void batch_overflow(const BatchPlan &B, BatchGroup &G, hipStream_t s) {
   batch_flags_u8(G.ids, G.overflow, N, G.aflags, s);
   scan_exclusive_u32(G.aflags, G.apos, N, G.scratch, s);
   compact_active(G.ids, G.aflags, G.apos, N, G.act, s);
-  batch_tiles(G.cellStart, G.apos, G.cpos + N, N, std::min(B.tq, 16u), G.ntiles, G.tileOff, G.scratch, G.tiles, s);
+  batch_tiles(G.cellStart, G.apos, G.cpos + N, N, std::min(B.tile_queries(G), 16u), G.ntiles, G.tileOff, G.scratch, G.tiles, s);
   fill_u32(G.ctr + 8, 0u, TILE_QUEUES, s);
   if (overflow_by_collect(G.k1max))
     range_collect<float>(a, g0, s);
@@ -2596,25 +2619,11 @@ static int run_batched(uint32_t nsets, const float *const *points, const uint32_
   hipStream_t s = lib_stream();
   knnjoin_batch_stats stats{};
   BatchPlan &B = g_batch;
-  std::vector<uint64_t> sig;
-  sig.reserve((size_t)nsets * 3 + 4);
-  for (uint32_t i = 0; i < nsets; i++) {
-    sig.push_back(n[i]);
-    sig.push_back(((uint64_t)ndim[i] << 32) | k[i]);
-  }
-  sig.push_back(p.num_indexed_dims);
+  const std::vector<uint64_t> sig = batch_signature(nsets, n, ndim, k, p.num_indexed_dims);
   uint32_t tq = p.tile_queries, grid = p.grid_blocks;
   if ((!tq || !grid) && sig == g_tunedSig) {
     if (!tq) tq = g_tunedTq;
     if (!grid) grid = g_tunedGrid;
-  }
-  // defaults: whole chunks of 64 queries for the direct kernel, which looks all their rows up at
-  // once; 16-query tiles of one cell for the collect kernel
-  if (!tq) {
-    uint32_t k1max = 0;
-    for (uint32_t i = 0; i < nsets; i++)
-      if (n[i]) k1max = std::max(k1max, k[i] + 1);
-    tq = range_kernel(k1max) == RK_DIRECT ? 64u : 16u;
   }
   if (!grid) grid = 4096;
   if (tq > 64) throw Error(KNN_ERR_ARG, "tile_queries must be <= 64");
@@ -2658,7 +2667,7 @@ static int run_batched(uint32_t nsets, const float *const *points, const uint32_
     for (BatchGroup &G : B.groups) {
       batch_capture(G.gStart, G.stream, [&]() { batch_start(B, G, G.stream); });
       batch_capture(G.gPass, G.stream, [&]() { batch_pass(B, G, G.stream); });
-      batch_capture(G.gOver, G.stream, [&]() { batch_overflow(B, G, G.stream); });
+      if (G.kernel == RK_DIRECT) batch_capture(G.gOver, G.stream, [&]() { batch_overflow(B, G, G.stream); });
     }
     B.captured = true;
   } else if (B.useGraph) {
@@ -2729,11 +2738,15 @@ static int run_batched(uint32_t nsets, const float *const *points, const uint32_
       HIP_CHECK(hipMemcpyAsync(outDists[si], G.outDists + sd.outOff, sizeof(float) * cnt, kout, G.stream));
     }
   for (BatchGroup &G : B.groups) HIP_CHECK(hipStreamSynchronize(G.stream));
-  stats.groups = (uint32_t)B.groups.size();
+  uint32_t dims = 0;
+  for (const BatchGroup &G : B.groups) {
+    dims |= 1u << G.d;
+    stats.tile_queries = std::max(stats.tile_queries, B.tile_queries(G));
+  }
+  stats.groups = (uint32_t)__builtin_popcount(dims);
   stats.graph_replayed = replay ? 1u : 0u;
   stats.passes_graph = B.passes;
   stats.passes_eager = eager;
-  stats.tile_queries = B.tq;
   stats.grid_blocks = B.grid;
   if (p.verbose)
     printf("[knn] batched: %u sets in %u groups, %llu points, device %.3f ms (%s), eager passes %u\n",
@@ -2796,13 +2809,7 @@ int knnjoin_batch_autotune(uint32_t nsets, const float *const *points, const uin
           bg = gr;
         }
       }
-    std::vector<uint64_t> sig;
-    for (uint32_t i = 0; i < nsets; i++) {
-      sig.push_back(n[i]);
-      sig.push_back(((uint64_t)ndim[i] << 32) | k[i]);
-    }
-    sig.push_back(p.num_indexed_dims);
-    g_tunedSig = sig;
+    g_tunedSig = batch_signature(nsets, n, ndim, k, p.num_indexed_dims);
     g_tunedTq = bt;
     g_tunedGrid = bg;
     if (best_tq) *best_tq = bt;

@@ -1,8 +1,8 @@
 // batched.hip -- many independent point sets joined together (float32).
 //
 // No counterpart in the reference, which joins one set per process (main.cu:109-510).  The
-// sets of one dimensionality form a group; the group's points are concatenated and every
-// stage runs once per group over all of them:
+// sets of one dimensionality and range kernel form a group; the group's points are concatenated
+// and every stage runs once per group over all of them:
 //   per-set variance reorder (main.cu:2521-2615, same FP32 sums as a single-set join),
 //   per-set min/max, per-set grid (own width, own key range [keyBase, keyBase + cells)),
 //   one radix sort / cell table / dense start table for the whole group,

@@ -249,8 +249,9 @@ int knnjoin_mlp_train(float *weights, const float *X, const float *Y, uint32_t n
 /* ---------------------------------------------------------------------------------------
  * Batched joins: many independent point sets (float32), each joined as knnjoin_ex would
  * join it alone (same rows, same distance bits), processed together: one index and one
- * persistent range-kernel launch per radius pass for all sets of a dimensionality, the passes
- * captured in hipGraphs and replayed for later calls with the same set shapes.
+ * persistent range-kernel launch per radius pass for the sets of a dimensionality whose K
+ * takes the same range kernel, the passes captured in hipGraphs and replayed for
+ * later calls with the same set shapes.
  * No counterpart in the reference (one set per process, main.cu:109-510); for callers with
  * many small sets, where per-set launches and host round trips dominate.
  * ------------------------------------------------------------------------------------- */
@@ -260,7 +261,7 @@ typedef struct {
   int32_t device_ptrs;       /* 1 = set points and outputs are device pointers */
   int32_t use_graph;         /* 1 = capture the passes in hipGraphs, replay for equal shapes */
   uint32_t graph_passes;     /* radius passes run from graphs (0 = 8); later passes run eagerly */
-  uint32_t tile_queries;     /* queries per tile, <= 64 (0 = autotuned value, or 64; 16 with K+1 > 448) */
+  uint32_t tile_queries;     /* queries per tile, <= 64 (0 = autotuned value, or 64; 16 for sets with K+1 > 448) */
   uint32_t grid_blocks;      /* persistent range-kernel blocks, <= 8192 (0 = autotuned or 4096) */
   int32_t verbose;
 } knnjoin_batch_params;

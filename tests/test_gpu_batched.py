@@ -199,3 +199,23 @@ def test_batched_graphs_follow_the_kernel_switches(monkeypatch, knob, value):
     ids, dists, st = batched.knnjoin_batched(pts, ks)
     assert st.graph_replayed == 0
     _check_against_single(sets, ids, dists)
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 6])
+def test_batched_long_rows_leave_the_other_sets_alone(d):
+    # K+1 of 449 and more takes the collect kernel, above 2048 the heap kernel: the sets with
+    # small K examine the same candidates with such sets beside them as without
+    rng = np.random.default_rng(40 + d)
+    mk = lambda n: rng.random((n, d)).astype(np.float32)  # noqa: E731
+    small = [(mk(4000), 8), (mk(900), 16), (mk(2500), 40)]
+    long = [(mk(1500), 600), (mk(2300), 2100)]
+
+    def cand(sets):
+        ids, dists, st = batched.knnjoin_batched([p for p, _ in sets], [k for _, k in sets])
+        assert st.groups == 1 and st.tile_queries == (64 if sets[0][1] < 448 else 16)
+        _check_against_single(sets, ids, dists)
+        return st.candidates
+
+    apart = cand(small) + cand(long[:1]) + cand(long[1:])
+    assert cand(small + long) == apart
+    assert cand([small[0], long[1], small[1], long[0], small[2]]) == apart
