@@ -1985,7 +1985,7 @@ int knnjoin_outlier_scores(const int32_t *ids, const float *dists, uint32_t n, u
     uint32_t *k0 = w + 4 * (size_t)n, *v0 = w + 5 * (size_t)n, *k1t = w + 6 * (size_t)n, *v1t = w + 7 * (size_t)n;
     uint32_t *scr = w + 8 * (size_t)n;
     uint32_t *bins = scr + ((sw + 3) & ~(size_t)3);
-    outlier_scores(dIds, dD, n, k1, ds, dr, dg, gr, k0, v0, k1t, v1t, scr, pl, bins, pinned(), s);
+    HIP_CHECK(outlier_scores(dIds, dD, n, k1, ds, dr, dg, gr, k0, v0, k1t, v1t, scr, pl, bins, pinned(), s));
     LAUNCH_CHECK();
     const hipMemcpyKind kout = device_ptrs ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
     HIP_CHECK(hipMemcpyAsync(dist_sum, ds, sizeof(float) * n, kout, s));

@@ -270,16 +270,17 @@ void batch_chunks(const SetDesc *sets, uint32_t nsets, uint32_t nd, const uint32
 // main.cu:952-1067 over an N x k1 table: FP32 row sums of the distances (entry order) and
 // their rank (descending), in-degree of every point and its rank (ascending); equal values
 // ranked by point id.  keys/vals/keysTmp/valsTmp: n words each; scratch: radix_scratch_words(n).
-// bins: p.words words (16-byte aligned); pinnedWord: host, read after a wait when p.shift is set.
+// bins: p.words words (16-byte aligned); pinnedWord: host, read after a wait when p.shift is set;
+// returns the status of that copy and wait.
 struct OutlierPlan {
   uint32_t shift, slabRows;  // in-degrees by bins of 2^shift ids, slabRows rows at a time (shift 0: by atomics)
   size_t words;
 };
 OutlierPlan outlier_plan(uint32_t n, uint32_t k1);
-void outlier_scores(const int32_t *ids, const float *dists, uint32_t n, uint32_t k1, float *distSum,
-                    uint32_t *distRank, uint32_t *indeg, uint32_t *indegRank, uint32_t *keys,
-                    uint32_t *vals, uint32_t *keysTmp, uint32_t *valsTmp, uint32_t *scratch,
-                    const OutlierPlan &p, uint32_t *bins, uint32_t *pinnedWord, hipStream_t s);
+hipError_t outlier_scores(const int32_t *ids, const float *dists, uint32_t n, uint32_t k1, float *distSum,
+                          uint32_t *distRank, uint32_t *indeg, uint32_t *indegRank, uint32_t *keys,
+                          uint32_t *vals, uint32_t *keysTmp, uint32_t *valsTmp, uint32_t *scratch,
+                          const OutlierPlan &p, uint32_t *bins, uint32_t *pinnedWord, hipStream_t s);
 
 // ------------------------------------------------------------- brute force (brute.hip)
 // Exact top-(K+1) of a query list against every point, no index (the reference's

@@ -221,11 +221,11 @@ OutlierPlan outlier_plan(uint32_t n, uint32_t k1) {
   return p;
 }
 
-void outlier_scores(const int32_t *ids, const float *dists, uint32_t n, uint32_t k1, float *distSum,
-                    uint32_t *distRank, uint32_t *indeg, uint32_t *indegRank, uint32_t *keys,
-                    uint32_t *vals, uint32_t *keysTmp, uint32_t *valsTmp, uint32_t *scratch,
-                    const OutlierPlan &p, uint32_t *bins, uint32_t *pinnedWord, hipStream_t s) {
-  if (!n) return;
+hipError_t outlier_scores(const int32_t *ids, const float *dists, uint32_t n, uint32_t k1, float *distSum,
+                          uint32_t *distRank, uint32_t *indeg, uint32_t *indegRank, uint32_t *keys,
+                          uint32_t *vals, uint32_t *keysTmp, uint32_t *valsTmp, uint32_t *scratch,
+                          const OutlierPlan &p, uint32_t *bins, uint32_t *pinnedWord, hipStream_t s) {
+  if (!n) return hipSuccess;
   const uint32_t g = (n + 255) / 256;
   int degBits = 32;
   if (p.shift) {
@@ -242,7 +242,8 @@ void outlier_scores(const int32_t *ids, const float *dists, uint32_t n, uint32_t
       k_deg_scatter<<<(m + 1024 * DEG_ITEMS - 1) / (1024 * DEG_ITEMS), 1024, 0, s>>>(sl, m, n, p.shift, cursor, binned);
       k_deg_count<<<nb, 1024, sizeof(uint32_t) << p.shift, s>>>(binned, start, n, p.shift, r0 != 0, indeg, maxDeg);
     }
-    (void)hipMemcpyAsync(pinnedWord, maxDeg, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
+    const hipError_t e = hipMemcpyAsync(pinnedWord, maxDeg, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
+    if (e != hipSuccess) return e;
   } else {
     fill_u32(indeg, 0u, n, s);
     const uint64_t m = (uint64_t)n * k1;
@@ -252,12 +253,15 @@ void outlier_scores(const int32_t *ids, const float *dists, uint32_t n, uint32_t
   radix_sort_pairs_u32(keys, vals, keysTmp, valsTmp, n, 32, scratch, s);
   k_scatter_rank<<<g, 256, 0, s>>>(vals, n, distRank);
   k_indeg_keys<<<g, 256, 0, s>>>(indeg, n, keys, vals);
-  if (p.shift && hipStreamSynchronize(s) == hipSuccess) {
+  if (p.shift) {
+    const hipError_t e = hipStreamSynchronize(s);
+    if (e != hipSuccess) return e;
     degBits = 1;  // the keys' digits: one 8-bit pass instead of four for most tables
     while (degBits < 32 && (*pinnedWord >> degBits)) degBits++;
   }
   radix_sort_pairs_u32(keys, vals, keysTmp, valsTmp, n, degBits, scratch, s);
   k_scatter_rank<<<g, 256, 0, s>>>(vals, n, indegRank);
+  return hipSuccess;
 }
 
 }  // namespace knn
