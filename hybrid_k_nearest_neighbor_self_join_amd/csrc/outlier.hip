@@ -21,13 +21,23 @@ namespace {
 // orders the sums descending (non-negative floats: larger value, larger bits).
 // A block takes 256 rows: OUT_E entries of each at a time come in as one coalesced stream and go
 // through LDS (odd row stride) to the thread that sums the row.
+// COUNT: also counts the in-degrees of the block's entries, by atomics.
 constexpr uint32_t OUT_E = 16;
-__global__ __launch_bounds__(256) void k_outlier_rows(const float *__restrict__ dists, uint32_t n, uint32_t k1,
-                                                      float *distSum, uint32_t *key, uint32_t *val) {
+template <bool COUNT>
+__global__ __launch_bounds__(256) void k_outlier_rows(const int32_t *__restrict__ ids, const float *__restrict__ dists,
+                                                      uint32_t n, uint32_t k1, float *distSum, uint32_t *key,
+                                                      uint32_t *val, uint32_t *indeg) {
   __shared__ float tile[256 * (OUT_E + 1)];
   const uint32_t r0 = blockIdx.x * 256u, tid = threadIdx.x;
   const uint32_t rows = n - r0 < 256u ? n - r0 : 256u;
   const uint32_t i = r0 + tid;
+  if (COUNT) {
+    const int32_t *own = ids + (size_t)r0 * k1;
+    for (uint32_t t = tid; t < rows * k1; t += 256) {
+      const int32_t id = own[t];
+      if (id >= 0 && (uint32_t)id < n) atomicAdd(&indeg[id], 1u);
+    }
+  }
   const float *src = dists + (size_t)r0 * k1;
   float s = 0.0f;
   for (uint32_t e0 = 0; e0 < k1; e0 += OUT_E) {
@@ -54,7 +64,11 @@ __global__ __launch_bounds__(256) void k_outlier_rows(const float *__restrict__ 
 // In-degrees.  Counters in global memory take about 28 atomic additions per ns whatever their
 // spread (the XCDs' L2s do not share them): 0.6 ms for 17M entries.  With enough entries the ids
 // are first dealt into at most DEG_BINS bins of consecutive ids, 16 bits each, and a block per bin
-// counts its ids in LDS: the scores of 1M points with 17 entries 0.93 -> 0.37 ms.
+// counts its ids in LDS: the scores of 1M points with 17 entries 0.93 -> 0.37 ms.  With fewer, rows of
+// up to 32 are counted by the kernel that sums them (9M points with 4 entries 2.45 -> 2.37 ms, 100k
+// with 9 0.307 -> 0.305, 1,000 with 17 0.141 -> 0.137); longer ones by k_deg_atomic, over more
+// blocks than they have rows for (1,000 points with 64 entries: 0.160 with the sums, 0.148 so).
+constexpr uint32_t ROW_COUNT_K1 = 32;
 __global__ void k_deg_atomic(const int32_t *__restrict__ ids, uint64_t m, uint32_t n, uint32_t *indeg) {
   for (uint64_t t = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; t < m; t += (uint64_t)gridDim.x * blockDim.x) {
     const int32_t id = ids[t];
@@ -207,7 +221,7 @@ __global__ void k_scatter_rank(const uint32_t *val, uint32_t n, uint32_t *rank) 
 // The largest number of entries dealt at once: 64 MB of 16-bit ids.
 constexpr uint64_t DEG_SLAB = 1ull << 25;
 // Bins of 2^shift ids, at least 1024 so that small tables keep few bins and at most 16384 (64 KB
-// of LDS); from 4M entries on, where the counters' atomics take 0.14 ms (below, the three extra
+// of LDS); from 4M entries on, where the counters' atomics take 0.14 ms (below, the four extra
 // launches cost what they save: 100k points with 9 entries 0.30 ms either way), and to 8M points.
 OutlierPlan outlier_plan(uint32_t n, uint32_t k1) {
   OutlierPlan p{};
@@ -247,9 +261,10 @@ hipError_t outlier_scores(const int32_t *ids, const float *dists, uint32_t n, ui
   } else {
     fill_u32(indeg, 0u, n, s);
     const uint64_t m = (uint64_t)n * k1;
-    k_deg_atomic<<<(uint32_t)std::min<uint64_t>((m + 255) / 256, 8192u), 256, 0, s>>>(ids, m, n, indeg);
+    if (k1 > ROW_COUNT_K1) k_deg_atomic<<<(uint32_t)std::min<uint64_t>((m + 255) / 256, 8192u), 256, 0, s>>>(ids, m, n, indeg);
   }
-  k_outlier_rows<<<g, 256, 0, s>>>(dists, n, k1, distSum, keys, vals);
+  auto rows = !p.shift && k1 <= ROW_COUNT_K1 ? k_outlier_rows<true> : k_outlier_rows<false>;
+  rows<<<g, 256, 0, s>>>(ids, dists, n, k1, distSum, keys, vals, indeg);
   radix_sort_pairs_u32(keys, vals, keysTmp, valsTmp, n, 32, scratch, s);
   k_scatter_rank<<<g, 256, 0, s>>>(vals, n, distRank);
   k_indeg_keys<<<g, 256, 0, s>>>(indeg, n, keys, vals);

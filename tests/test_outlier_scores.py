@@ -88,3 +88,24 @@ def test_gpu_indegrees_by_bins(oracle, n, k1):
     assert np.array_equal(got[0].view(np.uint32), want[0].view(np.uint32))
     for g, w in zip(got[1:], want[1:]):
         assert np.array_equal(g, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k1", [(1, 1), (255, 32), (256, 33), (257, 1), (1000, 32), (3001, 33), (5000, 31)])
+def test_gpu_indegrees_of_few_entries(n, k1):
+    # rows of up to 32 entries are counted with their sums, longer ones by a kernel of their own;
+    # absent entries (-1) count nowhere
+    rng = np.random.default_rng(1000 * n + k1)
+    ids = rng.integers(0, n, (n, k1)).astype(np.int32)
+    ids[::4, k1 // 2] = 0
+    d = np.round(rng.uniform(0, 2, (n, k1)), 2).astype(np.float32)
+    want = np_outlier(ids, d)
+    gone = ids[::3, k1 - 1].copy()
+    ids[::3, k1 - 1] = -1
+    deg = want[2] - np.bincount(gone, minlength=n).astype(np.uint32)
+    rank = np.empty(n, np.uint32)
+    rank[np.lexsort((np.arange(n), deg))] = np.arange(n)
+    got = _lib.outlier_scores(ids, d)
+    assert np.array_equal(got[0].view(np.uint32), want[0].view(np.uint32))
+    for g, w in zip(got[1:], (want[1], deg, rank)):
+        assert np.array_equal(g, w)
