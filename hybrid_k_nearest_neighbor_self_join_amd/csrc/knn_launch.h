@@ -163,8 +163,13 @@ void range_direct(const JoinArgs &a, const typename GridOf<T>::type &g, hipStrea
 constexpr uint32_t DR_NB = 256;   // buckets of the key, 4 per lane
 constexpr uint32_t DR_RMAX = 10;  // rows of a query's block kept per chunk (<= 2 indexed dims)
 // Built for three list sizes: H rounds of 64 list items are ranked in registers, up to K+1 =
-// direct_k1(H).
-constexpr uint32_t direct_k1(int h) { return h == 3 ? 40u : (h == 4 ? 224u : 448u); }
+// direct_k1(H).  The largest keeps 16 of its 512 places free: a list is cut at the edge of one of
+// 256 buckets, so that a few items past K+1 stay.  ms per join, direct / collect kernel, at K+1 =
+// 456, 496, 504 and 511: 300k mixed 2-D plain 9.1 / 25.1, 10.4 / 26.0, 10.5 / 28.0, 19.9 / 29.0;
+// 150k uniform 4-D plain 5.7 / 16.5, 7.9 / 18.5, 9.2 / 20.1, 21.9 / 20.4; 50k skewed 6-D learned
+// 10.1 / 12.6, 10.7 / 13.3, 16.6 / 16.4, 20.5 / 16.5 (overflows at 496: at most 8 queries, at 504
+// thousands).
+constexpr uint32_t direct_k1(int h) { return h == 3 ? 40u : (h == 4 ? 224u : 496u); }
 constexpr uint32_t DR_MAX_K1 = direct_k1(8);
 // Collect kernel (wave = query, one pass over its block into an LDS top-(K+1) collector): for
 // queries with many candidates per neighbour.  K+1 <= BRUTE_MAX_K1.

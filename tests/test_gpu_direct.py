@@ -5,7 +5,7 @@ fast path's range.  Rows are compared with FP64 brute force (ids, and FP32 dista
 import numpy as np
 import pytest
 
-from hybrid_k_nearest_neighbor_self_join_amd import _lib, learned_radius, synthetic
+from hybrid_k_nearest_neighbor_self_join_amd import _lib, batched, learned_radius, synthetic
 
 pytestmark = pytest.mark.gpu
 
@@ -103,3 +103,15 @@ def test_grid_dims(oracle, monkeypatch, d, nd, k, dtype, mode, data):
     assert np.array_equal(i0, i1) and np.array_equal(d0, d1)
     if mode == "plain":
         assert (s0.iterations, s0.reindexes, s0.eps0, s0.eps_final) == (s1.iterations, s1.reindexes, s1.eps0, s1.eps_final)
+
+
+@pytest.mark.parametrize("d,gen", [(2, "mixed"), (2, "uniform"), (4, "uniform"), (6, "skewed")])
+@pytest.mark.parametrize("k", [455, 479, 495, 496])
+def test_longest_lists(oracle, d, gen, k):
+    # K+1 up to 496: the direct kernel; 497: the collect kernel.  A batched join reports the tile
+    # size of the kernel it takes
+    n = 8009
+    pts = {"mixed": synthetic.mixed_box, "uniform": lambda n, seed: synthetic.unit_cube(n, d, seed=seed),
+           "skewed": lambda n, seed: synthetic.skewed_cube(n, d, seed=seed)}[gen](n, seed=k)
+    _check(oracle, pts, k, beta=0.025)
+    assert batched.knnjoin_batched([pts], [k])[2].tile_queries == (64 if k < 496 else 16)
