@@ -214,8 +214,10 @@ __global__ __launch_bounds__(64) void k_brute_partial(BruteArgs a) {
       for (uint32_t t = 0; t < BR_QW; t++) {
         if (t >= qw) continue;
         if (std::is_same<T, float>::value) {
-          const bool near = valid && br_dist_sq<D, T>(c[u], qc[t]) <= fb[t];
-          if (__ballot(near) == 0) continue;
+          // (& and not &&, whose branch per query costs a whole join of 300k 2-D points, K=8, 30.8 ms
+          // against 27.3)
+          const bool near = valid & (br_dist_sq<D, T>(c[u], qc[t]) <= fb[t]);
+          if (__builtin_amdgcn_ballot_w64(near) == 0) continue;
           col[t].offer(near, br_key<D, T>(c[u], qc[t]), p, lane);
           fb[t] = (T)(col[t].tk * (1.0 + 0x1p-16) + 0x1p-140);  // +inf until k1 entries are held
         } else {
