@@ -321,21 +321,31 @@ __device__ __forceinline__ bool row_chord_lane(const G &g, const uint32_t *cur, 
 // and, once that is empty, from the other ranges in turn.  Wave-uniform.
 static_assert(TILE_QUEUES == 8, "tile ranges are split by a shift of 3");
 // Next tile index of the workgroup, NT when every range is empty.  ranges: 1 or TILE_QUEUES.
-// No state is kept between calls: a workgroup whose ranges are empty re-reads their heads (at
-// most TILE_QUEUES atomics per call once its own range is empty).
+// No state is kept between calls: a workgroup whose own range is empty reads the other heads at
+// once (lane = range; a head only grows, so an old value costs a failing atomic and loses no tile)
+// and goes to the next one that still shows tiles.  A failing atomic on every head instead cost
+// each pass of a join about 0.3 ms, whatever its queries: 4096 waves times eight atomics on eight
+// words (ms per join, plain: 20k skewed 3-D points on 2 dims K=1, 23 passes, 11.6 / 4.5, 500k
+// skewed 4-D K=16 13.5 / 7.3, 2M uniform 6-D K=32 23.4 / 22.6).  One loop for all of it: a separate
+// first attempt spills 8 more registers of the 2-D kernel.
 __device__ __forceinline__ uint32_t next_tile(uint32_t *heads, uint32_t NT, uint32_t ranges, uint32_t lane) {
   const uint32_t sh = ranges == TILE_QUEUES ? 3u : 0u;
   const uint32_t mask = (1u << sh) - 1u;
-  for (uint32_t j = 0; j <= mask; j++) {
-    const uint32_t r = (blockIdx.x + j) & mask;
-    const uint32_t b = (uint32_t)(((uint64_t)NT * r) >> sh);
-    const uint32_t e = (uint32_t)(((uint64_t)NT * (r + 1)) >> sh);
+  auto begin = [&](uint32_t r) { return (uint32_t)(((uint64_t)NT * r) >> sh); };
+  uint32_t j = 0;  // ranges tried or seen empty
+  for (;;) {
+    const uint32_t r = (blockIdx.x + j) & mask, b = begin(r), e = begin(r + 1);
     uint32_t t = 0;
     if (lane == 0) t = atomicAdd(&heads[r], 1u);
-    t = (uint32_t)__shfl((int)t, 0, 64);
+    t = (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
     if (t < e - b) return b + t;
+    const uint32_t q = (blockIdx.x + lane) & mask;
+    bool left = lane > j && lane <= mask;
+    if (left) left = __hip_atomic_load(&heads[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < begin(q + 1) - begin(q);
+    const uint64_t m = __builtin_amdgcn_ballot_w64(left);
+    if (!m) return NT;
+    j = (uint32_t)__builtin_ctzll(m);
   }
-  return NT;
 }
 
 // The grid, K+1 and row addressing of one tile: the kernel's own for a single set; the

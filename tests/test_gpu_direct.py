@@ -115,3 +115,17 @@ def test_longest_lists(oracle, d, gen, k):
            "skewed": lambda n, seed: synthetic.skewed_cube(n, d, seed=seed)}[gen](n, seed=k)
     _check(oracle, pts, k, beta=0.025)
     assert batched.knnjoin_batched([pts], [k])[2].tile_queries == (64 if k < 496 else 16)
+
+
+@pytest.mark.parametrize("kern", ["direct", "collect"])
+@pytest.mark.parametrize("n", [7, 65, 500, 9001])
+def test_tile_ranges(oracle, monkeypatch, kern, n):
+    # one queue over all tiles or one range per XCD, with fewer tiles than ranges and with many:
+    # every tile is taken once whichever range it lies in
+    monkeypatch.setenv("KNN_RANGE_KERNEL", kern)
+    pts = synthetic.skewed_cube(n, 3, seed=n)
+    cand = set()
+    for ranges in ("1", "8"):
+        monkeypatch.setenv("KNN_TILE_RANGES", ranges)
+        cand.add(_check(oracle, pts, min(5, n - 1), beta=0.05).candidates)
+    assert len(cand) == 1
