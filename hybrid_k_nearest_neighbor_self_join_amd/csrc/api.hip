@@ -1122,6 +1122,10 @@ static double env_knob(const char *name, double lo, double hi) {
 // uniform K=8 0.89 / 0.98, 1M mixed K=8 5.4 / 5.9).  Above 2 indexed dims cells of eps until eps
 // has grown by half, against a re-index at every growth: 3M skewed 4-D K=16 27.8 / 24.3, 500k
 // skewed 6-D K=32 31.0 / 26.1, finer cells multiply the rows (500k 6-D at eps / 1.5: 28.7).
+// Above 6 a re-index at every growth: a radius of 1.5 cells meets 5 cells per dim, not 3, and the
+// block counts and lookups visit all their rows (until eps has grown by half / at every growth: 8-D
+// uniform 20k K=1 6.5 / 3.3, skewed 100k K=2 37.7 / 20.3, 60k K=32 23.8 / 12.7; 7-D skewed 100k K=16
+// 12.8 / 12.0; 12-D on 8 dims uniform 60k K=32 10.7 / 10.7).
 // Projected grids of up to 2 indexed dims, eps / 1.5: 500k skewed 4-D K=16 22.7 / 18.7.
 static double plain_grid_div(uint32_t d, uint32_t nd, uint32_t k1) {
   const double e = env_knob("KNN_PLAIN_GRID_DIV", 1.0, 8.0);
@@ -1132,7 +1136,7 @@ static double plain_grid_div(uint32_t d, uint32_t nd, uint32_t k1) {
 static double plain_max_reach(uint32_t d, uint32_t nd, uint32_t k1) {
   const double e = env_knob("KNN_PLAIN_MAX_REACH", 1.0, 8.0);
   if (e > 0.0) return e;
-  if (nd > 2) return 1.5;
+  if (nd > 2) return nd > 6 ? 1.0 : 1.5;
   return nd < d ? 2.0 : (k1 >= 12 ? 5.0 : 2.0);
 }
 
