@@ -129,3 +129,16 @@ def test_tile_ranges(oracle, monkeypatch, kern, n):
         monkeypatch.setenv("KNN_TILE_RANGES", ranges)
         cand.add(_check(oracle, pts, min(5, n - 1), beta=0.05).candidates)
     assert len(cand) == 1
+
+
+@pytest.mark.parametrize("div", ["1", "2", "2.5", "4.5", "5", "6"])
+def test_rows_looked_up_together(oracle, monkeypatch, div):
+    # blocks of 2 div to 2 div + 2 rows (a chunk's table holds 10: at 4.5 some and at 5 most blocks
+    # have more, and are streamed), looked up one or two at a time
+    monkeypatch.setenv("KNN_PLAIN_GRID_DIV", div)
+    monkeypatch.setenv("KNN_PLAIN_MAX_REACH", div)
+    pts = synthetic.mixed_box(9001, seed=int(10 * float(div)))
+    st = [_check(oracle, pts, 20, beta=0.025)]
+    monkeypatch.setenv("KNN_TILE_ROWS", "1")
+    st.append(_check(oracle, pts, 20, beta=0.025))
+    assert st[0].candidates == st[1].candidates and st[0].iterations == st[1].iterations

@@ -40,3 +40,21 @@ def test_small_bitmap_chunks_give_the_same_rows(oracle, monkeypatch, d, nd, gen,
     bi, bd = oracle.bruteforce(np.ascontiguousarray(pts[:, perm]), k, queries=q)
     assert np.array_equal(ref[0][q], bi)
     assert np.array_equal(bits(ref[1][q]), bits(bd))
+
+
+@pytest.mark.parametrize("d,nd,gen,k", [(3, 1, "uniform", 16), (4, 2, "uniform", 16), (6, 4, "skewed", 16), (7, 5, "skewed", 8)])
+@pytest.mark.parametrize("log2", ["6", "8"])
+def test_small_bitmap_chunks_of_slab_segments(oracle, monkeypatch, d, nd, gen, k, log2):
+    # a grid of the indexed dims alone (KNN_GRID_DIMS=0), whose cells are cut to the query's slab: a
+    # segment per cell
+    pts = _points(d, gen, 30_000, seed=d * 37 + nd)
+    monkeypatch.setenv("KNN_GRID_DIMS", "0")
+    ref = _lib.knnjoin_ex(pts, k, num_indexed_dims=nd, beta=0.025, brute_fallback=0)
+    monkeypatch.setenv("KNN_SEG_CHUNK_LOG2", log2)
+    ids, dist, st = _lib.knnjoin_ex(pts, k, num_indexed_dims=nd, beta=0.025, brute_fallback=0)
+    assert np.array_equal(ids, ref[0]) and np.array_equal(bits(dist), bits(ref[1]))
+    assert st.candidates == ref[2].candidates
+    q = np.random.default_rng(d + nd).choice(len(pts), 200, replace=False)
+    perm, _ = oracle.reorder(pts)
+    bi, bd = oracle.bruteforce(np.ascontiguousarray(pts[:, perm]), k, queries=q)
+    assert np.array_equal(ids[q], bi) and np.array_equal(bits(dist[q]), bits(bd))

@@ -76,3 +76,29 @@ def test_slab_order_double(oracle, d, nd):
     assert rc == 0
     assert np.array_equal(ids, i2)
     assert np.array_equal(dist.view(np.uint64), d2.view(np.uint64))
+
+
+@pytest.mark.parametrize("d,nd,gen,kern", [
+    (3, 1, "uniform", "direct"), (4, 2, "skewed", "direct"), (4, 2, "lattice", "direct"), (5, 3, "lattice", "direct"),
+    (6, 4, "uniform", "direct"), (7, 5, "skewed", "direct"), (8, 6, "uniform", "direct"), (8, 6, "skewed", "collect"),
+])
+@pytest.mark.parametrize("mode", [_lib.KNN_MODE_BETA, _lib.KNN_MODE_LEARNED])
+def test_slab_cut_alone(oracle, monkeypatch, d, nd, gen, kern, mode):
+    # KNN_GRID_DIMS=0 keeps the grid of the indexed dims on both sides, so that the slab cut is the
+    # only difference: the same rows, from fewer candidates
+    pts = _points(d, gen, 30_000, seed=d * 13 + nd)
+    loaded = learned_radius.register_default_models()
+    if not learned_radius.has_model(loaded, d, nd):
+        _lib.set_radius_model(nd, learned_radius.init_weights(d * 10 + nd) * 0.1, 0.3, ndim=d)
+    monkeypatch.setenv("KNN_GRID_DIMS", "0")
+    monkeypatch.setenv("KNN_RANGE_KERNEL", kern)
+    kw = dict(num_indexed_dims=nd, mode=mode, brute_fallback=0)
+    on = _lib.knnjoin_ex(pts, 16, **kw)
+    monkeypatch.setenv("KNN_SLAB", "0")
+    off = _lib.knnjoin_ex(pts, 16, **kw)
+    assert np.array_equal(on[0], off[0]) and np.array_equal(bits(on[1]), bits(off[1]))
+    assert on[2].candidates < off[2].candidates
+    q = np.random.default_rng(d + nd).choice(len(pts), 200, replace=False)
+    perm, _ = oracle.reorder(pts)
+    bi, bd = oracle.bruteforce(np.ascontiguousarray(pts[:, perm]), 16, queries=q)
+    assert np.array_equal(on[0][q], bi) and np.array_equal(bits(on[1][q]), bits(bd))
