@@ -287,7 +287,7 @@ struct Timer {
 // Pinned host words for the values the host reads back during a join (cell, active, failure
 // and overflow counts, accounting counters, radius histograms): allocated once, so that those
 // copies are asynchronous and one stream wait per pass collects them all.
-enum PinWord { PW_NCELL = 0, PW_KFAIL = 1, PW_OVF = 2, PW_ACTIVE = 3, PW_SPAN = 4, PW_CTR = 8, PW_HIST = 64, PW_MAXR = 128 };
+enum PinWord { PW_NCELL = 0, PW_KFAIL = 1, PW_OVF = 2, PW_ACTIVE = 3, PW_CTR = 8, PW_HIST = 64, PW_MAXR = 128 };
 static uint32_t *g_pin = nullptr;
 static uint32_t *pinned() {
   if (!g_pin) HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&g_pin), 4096, hipHostMallocDefault));
@@ -497,7 +497,7 @@ struct Pipeline {
   void make_active(const uint8_t *activeFailed, uint32_t *&act, uint8_t *failed, unsigned long long *cellAcc);
   // tiles of at most 64 of them per cell for the heap kernel, which scans the union of a tile's
   // blocks; the tile count ends in *ntilesDev
-  void make_tiles(uint4 *&tiles, const uint32_t *&ntilesDev);
+  void make_tiles(uint2 *&tiles, const uint32_t *&ntilesDev);
   unsigned long long accBytes = 0;  // accumulated pre-check accounting bytes
   const T *radius = nullptr;  // per-query radii (learned schedule), null = radiusAll
   T radiusAll = (T)0;         // one radius for every query (plain schedule); 0 = the grid's eps
@@ -731,11 +731,11 @@ void Pipeline<T>::make_active(const uint8_t *activeFailed, uint32_t *&act, uint8
 }
 
 template <typename T>
-void Pipeline<T>::make_tiles(uint4 *&tiles, const uint32_t *&ntilesDev) {
+void Pipeline<T>::make_tiles(uint2 *&tiles, const uint32_t *&ntilesDev) {
   const uint32_t *pos = buf<uint32_t>(S_POS, n + 1);
   uint32_t *ntiles = buf<uint32_t>(S_NTILES, (size_t)n + 2);
   uint32_t *tileOff = buf<uint32_t>(S_TILEOFF, (size_t)n + 3);
-  tiles = buf<uint4>(S_TILES, n);
+  tiles = buf<uint2>(S_TILES, n);
   uint32_t *nc = buf<uint32_t>(S_TILEMETA, 16);  // (the build's own device count is overwritten by now)
   fill_u32(nc, ncell, 1, s);
   batch_tiles(cellStart, pos, nc, n, 64u, ntiles, tileOff, scratch, tiles, s);
@@ -790,7 +790,7 @@ PassResult Pipeline<T>::pass(const uint8_t *activeFailed, uint32_t nq, uint8_t *
   a.overflowCount = overflowCount;
   PassResult r{};
   auto heap = [&]() {
-    uint4 *tiles;
+    uint2 *tiles;
     make_tiles(tiles, a.ntilesDev);
     a.tiles = tiles;
     a.ntiles = kHeapGrid;
@@ -2263,7 +2263,7 @@ struct BatchGroup {
            *ctr = nullptr;
   uint64_t *cellKeys = nullptr;
   unsigned long long *cand = nullptr;
-  uint4 *tiles = nullptr;
+  uint2 *tiles = nullptr;
   uint8_t *failed = nullptr, *overflow = nullptr, *bin = nullptr;
   uint32_t *setMinBin = nullptr, *setClass = nullptr, *chunkOff = nullptr;
   SetDesc *sets = nullptr;
@@ -2436,7 +2436,7 @@ static void batch_build(BatchPlan &B, uint32_t nsets, const uint32_t *n, const u
     G.act = B.alloc<uint32_t>((size_t)N + 1);
     G.ntiles = B.alloc<uint32_t>((size_t)N + 2);
     G.tileOff = B.alloc<uint32_t>((size_t)N + 3);
-    G.tiles = B.alloc<uint4>((size_t)N + 1);
+    G.tiles = B.alloc<uint2>((size_t)N + 1);
     G.scratch = B.alloc<uint32_t>(sw);
     G.status = B.alloc<uint32_t>(4);
     G.ctr = B.alloc<uint32_t>(8 + TILE_QUEUES);  // [8..]: the tile queue heads

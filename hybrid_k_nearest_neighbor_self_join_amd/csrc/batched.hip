@@ -481,14 +481,14 @@ __global__ void k_b_tile_counts(const uint32_t *cellStart, const uint32_t *pos, 
 }
 
 __global__ void k_b_write_tiles(const uint32_t *cellStart, const uint32_t *pos, const uint32_t *tileOff,
-                                const uint32_t *ncell, uint32_t N, uint32_t tq, uint4 *tiles) {
+                                const uint32_t *ncell, uint32_t N, uint32_t tq, uint2 *tiles) {
   const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= N || c >= *ncell) return;
   const uint32_t a0 = pos[cellStart[c]], a1 = pos[cellStart[c + 1]];
   uint32_t t = tileOff[c];
   for (uint32_t a = a0; a < a1; a += tq, t++) {
     const uint32_t m = (a1 - a < tq) ? a1 - a : tq;
-    tiles[t] = make_uint4(0u, a, m, m);
+    tiles[t] = make_uint2(a, m);
   }
 }
 
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(256) void k_b_chunk_offsets(const SetDesc *sets, ui
 // tiles[t] = chunk t: thread per chunk, its set by binary search (at most N chunks: every chunk
 // holds a query)
 __global__ void k_b_chunks(const SetDesc *sets, uint32_t nsets, const uint32_t *__restrict__ pos,
-                           const uint32_t *__restrict__ chunkOff, const uint32_t *qIn, uint4 *tiles) {
+                           const uint32_t *__restrict__ chunkOff, const uint32_t *qIn, uint2 *tiles) {
   const uint32_t q = *qIn, n = chunkOff[nsets];
   for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
     uint32_t l = 0, h = nsets;  // chunkOff[l] <= t < chunkOff[h]
@@ -547,7 +547,7 @@ __global__ void k_b_chunks(const SetDesc *sets, uint32_t nsets, const uint32_t *
     }
     const uint32_t a0 = pos[sets[l].pStart] + (t - chunkOff[l]) * q, a1 = pos[sets[l].pStart + sets[l].n];
     const uint32_t m = a1 - a0 < q ? a1 - a0 : q;
-    tiles[t] = make_uint4(0u, a0, m, m);
+    tiles[t] = make_uint2(a0, m);
   }
 }
 
@@ -604,14 +604,14 @@ void batch_flags_u8(const uint32_t *sortedIds, const uint8_t *f, uint32_t N, uin
   if (N) k_b_flags_u8<<<nblk(N), BLK, 0, s>>>(sortedIds, f, N, flags);
 }
 void batch_tiles(const uint32_t *cellStart, const uint32_t *pos, const uint32_t *ncell, uint32_t N,
-                 uint32_t tq, uint32_t *ntiles, uint32_t *tileOff, uint32_t *scratch, uint4 *tiles,
+                 uint32_t tq, uint32_t *ntiles, uint32_t *tileOff, uint32_t *scratch, uint2 *tiles,
                  hipStream_t s) {
   k_b_tile_counts<<<nblk((size_t)N + 1), BLK, 0, s>>>(cellStart, pos, ncell, N, tq, ntiles);
   scan_exclusive_u32(ntiles, tileOff, N + 1, scratch, s);
   if (N) k_b_write_tiles<<<nblk(N), BLK, 0, s>>>(cellStart, pos, tileOff, ncell, N, tq, tiles);
 }
 void batch_chunks(const SetDesc *sets, uint32_t nsets, uint32_t nd, const uint32_t *pos, uint32_t N, uint32_t waves, uint32_t cap,
-                  uint32_t *chunkOff, uint32_t *ntiles, uint32_t *q, uint4 *tiles, hipStream_t s) {
+                  uint32_t *chunkOff, uint32_t *ntiles, uint32_t *q, uint2 *tiles, hipStream_t s) {
   // chunks per wave: a query's time grows with its indexed dims and with it the cost of an uneven
   // end (6-D group of a 48-set mix: 12.2 ms with 1, 9.3 with 4, 8.1 with 8;
   // 2-D chunks look up the rows of 64 queries at a time, so that smaller ones waste lanes)

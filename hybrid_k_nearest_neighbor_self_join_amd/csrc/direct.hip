@@ -210,8 +210,8 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
   for (;;) {
     const uint32_t t = next_tile(a.tileCounter, NT, a.tileRanges, lane);
     if (t >= NT) break;
-    const uint4 tl = work_tile(a, t, Q);
-    const uint32_t nq = tl.z;
+    const uint2 tl = work_tile(a, t, Q);
+    const uint32_t nq = tl.y;
     const uint32_t qL = tile_query(a, tl, lane < nq ? lane : 0u);
     TileCtx<G> C;
     if constexpr (SETS) {

@@ -315,7 +315,6 @@ __global__ void k_row_sums_direct(const T *__restrict__ dists, uint32_t n, uint3
   rowSum[r] = s;
 }
 
-// the chunk sums in order by one thread; sixteen loads in flight ahead of the adds
 // one block: the chunks' sums in order, SUM_CHUNK at a time through LDS (2442 chunks: 45 us reading
 // global memory 16 at a time, now 18)
 __global__ __launch_bounds__(256) void k_sum_final(const double *partial, uint32_t m, double *out) {

@@ -90,12 +90,9 @@ template <typename T>
 void gather_rows(const T *in, const uint32_t *ids, uint32_t n, uint32_t d, const DimPerm &perm, T *xs,
                  hipStream_t s);
 
-// Dense cell-start table (totalCells + 1 entries): denseStart[id] = first sorted position of
-// linear cell id (number of points in cells < id).  counts are scattered from the compacted
-// cell table, then scanned in place.
-
-// Active flags per sorted position with the own-block pre-check: queries whose own cell
-// block holds fewer than k1 points get failed[q] = 1 and flag 0.  activeBits (pack_bits of the
+// Active flags per sorted position with the own-block pre-check on the dense cell-start table
+// (totalCells + 1 entries, dense[id] = points in cells < id): queries whose own cell block holds
+// fewer than k1 points get failed[q] = 1 and flag 0.  activeBits (pack_bits of the
 // per-id active bytes) null = all active.  cellOf/cellMax (optional) collect per-cell
 // candidate counts for accounting.
 void pack_bits(const uint8_t *src, uint32_t n, uint64_t *bits, hipStream_t s);
@@ -127,9 +124,8 @@ struct JoinArgs {
   uint32_t ncell;
   const uint32_t *denseStart;  // dense cell-start table, or null (binary search of cellKeys)
   const uint32_t *act;   // active query ids, grouped by cell
-  // tile = up to 64 active queries in at most two runs of act: {start of the second run, start
-  // of the first, query count, length of the first run (= count for a single run)}
-  const uint4 *tiles;
+  // tile = up to 64 consecutive active queries: {start in act, query count}
+  const uint2 *tiles;
   uint32_t ntiles;       // tile count; with ntilesDev: the persistent grid size (blocks)
   uint32_t n, d, k1;
   const void *radius;    // per-query search radius (T); null = radiusAll for all
@@ -264,11 +260,11 @@ void batch_flags_u8(const uint32_t *sortedIds, const uint8_t *f, uint32_t N, uin
 // tiles of <= tq active queries per cell: ntiles/tileOff hold N + 2 words, tileOff[N + 1] =
 // tile count
 void batch_tiles(const uint32_t *cellStart, const uint32_t *pos, const uint32_t *ncell, uint32_t N,
-                 uint32_t tq, uint32_t *ntiles, uint32_t *tileOff, uint32_t *scratch, uint4 *tiles,
+                 uint32_t tq, uint32_t *ntiles, uint32_t *tileOff, uint32_t *scratch, uint2 *tiles,
                  hipStream_t s);
 // direct-kernel tiles: chunks of consecutive active queries of one set
 void batch_chunks(const SetDesc *sets, uint32_t nsets, uint32_t nd, const uint32_t *pos, uint32_t N, uint32_t waves, uint32_t cap,
-                  uint32_t *chunkOff, uint32_t *ntiles, uint32_t *q, uint4 *tiles, hipStream_t s);
+                  uint32_t *chunkOff, uint32_t *ntiles, uint32_t *q, uint2 *tiles, hipStream_t s);
 
 
 // ------------------------------------------------------------- outlier scores (outlier.hip)

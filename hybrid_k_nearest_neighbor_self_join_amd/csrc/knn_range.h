@@ -6,7 +6,7 @@
 // Within one row of a block (indexed dims 1.. fixed) the cells of dim 0 are adjacent linear
 // ids, i.e. one contiguous range of cell-sorted points.
 //
-// ND is the number of indexed dims when known at compile time (1..4), or 0 for the grid's
+// ND is the number of indexed dims when known at compile time (1..6), or 0 for the grid's
 // runtime value (up to KNN_MAX_INDEXED).  Every loop over indexed dims runs over a constant
 // bound (ND, or KNN_MAX_INDEXED with an exit at the runtime count) and is fully unrolled, so
 // the per-dim arrays live in registers rather than in private scratch memory.
@@ -129,20 +129,19 @@ struct Lane {
   T F;        // filter bound on the T sum
 };
 
-// Query i < tl.z of a tile: the first run act[tl.y ..) holds tl.w of them, the second run
-// act[tl.x ..) the rest.
-__device__ __forceinline__ uint32_t tile_query(const JoinArgs &a, const uint4 &tl, uint32_t i) {
-  return a.act[i < tl.w ? tl.y + i : tl.x + (i - tl.w)];
+// Query i < tl.y of a tile.
+__device__ __forceinline__ uint32_t tile_query(const JoinArgs &a, const uint2 &tl, uint32_t i) {
+  return a.act[tl.x + i];
 }
 
 // Lane = query of the tile: its coordinates, radius r (its own, or the pass's one radius) and
 // Tq = r^2 (1 - 2^-20); lo/hi = the wave's union of the lanes' cell ranges per indexed dim.
 template <typename T, int D, int ND, typename G>
-__device__ __forceinline__ void tile_setup(const JoinArgs &a, const G &g, const uint4 &tl, uint32_t lane,
+__device__ __forceinline__ void tile_setup(const JoinArgs &a, const G &g, const uint2 &tl, uint32_t lane,
                                            Lane<T, D> &L, uint32_t *lo, uint32_t *hi) {
   const T *__restrict__ x = reinterpret_cast<const T *>(a.x);
   const size_t n = a.n;
-  L.active = lane < tl.z;
+  L.active = lane < tl.y;
   L.q = tile_query(a, tl, L.active ? lane : 0u);
 #pragma unroll
   for (int j = 0; j < D; j++) {
@@ -234,21 +233,6 @@ __device__ __forceinline__ void for_each_row(const JoinArgs &a, const G &g, cons
       pEnd = (uint32_t)__builtin_amdgcn_readfirstlane((int)pEnd);
       if (pEnd > pBeg) f(pBeg, pEnd);
     }
-  } while (next_row<ND>(cur, lo, hi, nd));
-}
-
-// for_each_row without the point ranges: f(rowBase, l0, h0) for each row kept by narrow
-// (uniform across the wave when lo/hi are).
-template <int ND, typename G, typename R, typename F>
-__device__ __forceinline__ void for_each_row_span(const G &g, const uint32_t *lo, const uint32_t *hi,
-                                                  R &&narrow, F &&f) {
-  uint32_t cur[nd_cap<ND>()];
-  const uint32_t nd = nd_of<ND>(g);
-#pragma unroll
-  for (uint32_t j = 0; j < nd_cap<ND>(); j++) cur[j] = lo[j < nd ? j : 0];
-  do {
-    uint32_t l0 = lo[0], h0 = hi[0];
-    if (narrow(cur, l0, h0)) f(row_base<ND>(g, cur), l0, h0);
   } while (next_row<ND>(cur, lo, hi, nd));
 }
 
@@ -359,7 +343,7 @@ struct TileCtx {
   __device__ __forceinline__ size_t row(uint32_t q) const { return (size_t)((int64_t)q * k1 + rowAdj); }
 };
 template <typename G>
-__device__ __forceinline__ TileCtx<G> tile_ctx(const JoinArgs &a, const G &g, const uint4 &tl) {
+__device__ __forceinline__ TileCtx<G> tile_ctx(const JoinArgs &a, const G &g, const uint2 &tl) {
   TileCtx<G> c;
   c.g = g;
   c.k1 = a.k1;
@@ -397,10 +381,10 @@ __device__ __forceinline__ uint32_t work_count(const JoinArgs &a, uint32_t per, 
   Q = Q < 1u ? 1u : (Q > 64u ? 64u : Q);
   return (A + Q - 1u) / Q;
 }
-__device__ __forceinline__ uint4 work_tile(const JoinArgs &a, uint32_t t, uint32_t Q) {
+__device__ __forceinline__ uint2 work_tile(const JoinArgs &a, uint32_t t, uint32_t Q) {
   if (a.tiles) return a.tiles[t];
   const uint32_t q0 = t * Q, left = *a.activeCount - q0, nq = left < Q ? left : Q;
-  return make_uint4(q0, q0, nq, nq);
+  return make_uint2(q0, nq);
 }
 
 // Per-wave counters of a persistent kernel (wave-uniform), added to the global counters once
@@ -411,15 +395,15 @@ struct WaveTally {
 };
 
 template <typename T>
-__device__ __forceinline__ void tile_accounting(WaveTally &w, const uint4 &tl, bool ok, bool failedLane,
+__device__ __forceinline__ void tile_accounting(WaveTally &w, const uint2 &tl, bool ok, bool failedLane,
                                                 uint64_t tileCand, uint32_t K1) {
   const uint64_t fm = __ballot(failedLane);
   const uint64_t om = __ballot(ok);
   w.fails += (uint32_t)__popcll(fm);
   // compulsory HBM bytes of the tile's queries: ids in / failure flags out and the finished
   // rows (the query cells' candidate blocks are counted by the pre-filter)
-  w.bytes += (unsigned long long)tl.z * 8ull + (unsigned long long)__popcll(om) * K1 * (4ull + sizeof(T));
-  w.cand += (unsigned long long)tileCand * tl.z;
+  w.bytes += (unsigned long long)tl.y * 8ull + (unsigned long long)__popcll(om) * K1 * (4ull + sizeof(T));
+  w.cand += (unsigned long long)tileCand * tl.y;
 }
 
 __device__ __forceinline__ void flush_tally(const JoinArgs &a, const WaveTally &w, uint32_t lane) {

@@ -377,7 +377,8 @@ __global__ void k_max_radius_d(const double *radius, const uint8_t *failed, uint
   if (q < n && failed[q]) atomicMax(out, (unsigned long long)__double_as_longlong(radius[q]));
 }
 
-// gather rows of a (n x w) float matrix: out[b] = in[idx[b]]
+// ---------------------------------------------------------------- training kernels
+// thread = sample: activations and output of the forward pass
 __global__ void k_mlp_fwd(const float *__restrict__ Wg, const float *__restrict__ X, uint32_t B,
                           float *H1, float *H2, float *out) {
   __shared__ float W[MLP_NW];

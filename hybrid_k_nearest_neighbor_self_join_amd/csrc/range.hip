@@ -43,7 +43,7 @@ __global__ __launch_bounds__(64) void k_range_collect(JoinArgs a, G g0) {
   for (;;) {
     const uint32_t t = next_tile(a.tileCounter, NT, a.tileRanges, lane);
     if (t >= NT) break;
-    const uint4 tl = work_tile(a, t, Q);
+    const uint2 tl = work_tile(a, t, Q);
     const TileCtx<G> C = tile_ctx<G>(a, g0, tl);
     const G &g = C.g;
     const uint32_t nd = nd_of<ND>(g);
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(64) void k_range_collect(JoinArgs a, G g0) {
     const T eps = (T)g.eps;
     uint32_t nok = 0;
     unsigned long long cand = 0;
-    for (uint32_t i = 0; i < tl.z; i++) {
+    for (uint32_t i = 0; i < tl.y; i++) {
       const uint32_t q = (uint32_t)__builtin_amdgcn_readfirstlane((int)tile_query(a, tl, i));
       T qc[D];
       double qd[D];
@@ -142,8 +142,8 @@ __global__ __launch_bounds__(64) void k_range_collect(JoinArgs a, G g0) {
       nok += ok ? 1u : 0u;
       br_sync();  // the collector's LDS is reused by the next query
     }
-    tally.fails += tl.z - nok;
-    tally.bytes += (unsigned long long)tl.z * 8ull + (unsigned long long)nok * K1 * (4ull + sizeof(T));
+    tally.fails += tl.y - nok;
+    tally.bytes += (unsigned long long)tl.y * 8ull + (unsigned long long)nok * K1 * (4ull + sizeof(T));
     tally.cand += cand;
   }
   flush_tally(a, tally, lane);
@@ -237,7 +237,7 @@ __global__ __launch_bounds__(64) void k_range_heap(JoinArgs a, G g0) {
   for (;;) {
     const uint32_t t = next_tile(a.tileCounter, NT, a.tileRanges, lane);
     if (t >= NT) break;
-    const uint4 tl = a.tiles[t];
+    const uint2 tl = a.tiles[t];
     const TileCtx<G> C = tile_ctx<G>(a, g0, tl);
     const G &g = C.g;
     const uint32_t K1 = C.k1;
