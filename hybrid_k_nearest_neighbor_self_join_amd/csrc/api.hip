@@ -66,6 +66,7 @@ struct Arena {
   static size_t round(size_t b) { return ((b ? b : 16) + 255) & ~size_t(255); }
   // bytes of free scratch
   size_t room() const { return cap - used; }
+  size_t held(Slot s) const { return p[s] ? sz[s] : 0; }
   // scratch bytes that slot s would take to hold `bytes` (0 when its region holds them)
   size_t extra(Slot s, size_t bytes) const { return sz[s] >= bytes && p[s] ? 0 : round(bytes); }
   void *get(Slot s, size_t bytes) {
@@ -393,16 +394,7 @@ struct Pipeline {
     // dense cell-start table: O(1) row lookups when the grid is small enough (its counts are
     // scattered for the cells below the device-side cell count, so no host round trip here)
     denseStart = nullptr;
-    // with the no-allocation scratch: only when the table, its scan scratch and the pass
-    // buffers still to come (active list, tiles, block tables, flags) fit
-    bool denseFits = totalCells + 1 <= kDenseMaxCells;
-    if (denseFits && g_arena) {
-      const size_t tcb = (size_t)totalCells + 1;
-      const size_t more = g_arena->extra(S_DENSE, tcb * 4) +
-                          g_arena->extra(S_SCRATCH, (scan_scratch_words((uint32_t)tcb) + 1024) * 4);
-      denseFits = more + 48ull * n + (64u << 10) <= g_arena->room();
-    }
-    if (denseFits) {
+    if (dense_fits(totalCells)) {
       const uint32_t tc = (uint32_t)totalCells;
       const size_t need = scan_scratch_words(tc + 1) + 1024;
       if (need > scratchWords) {
@@ -441,11 +433,14 @@ struct Pipeline {
   // Dims of the range passes' grids: the join's indexed dims define its schedule and its radius
   // features, while a grid may be over more of the data's dims (any grid gives the same rows and
   // the same failures at a radius).
-  // Up to 6 dims, as a join that indexes them all (ms per join, the indexed dims' grid against
-  // one over all dims): 1M skewed 6-D points on 4 indexed dims K=32, learned 62.3 / 46.5, 3M
-  // uniform 4-D on 2 K=16 29.6 / 8.8; plain, 500k uniform 6-D on 4 K=16 8.3 / 5.7, 500k skewed
-  // 4-D on 2 K=16 18.2 / 11.9, 200k uniform 6-D on 2 K=8 5.8 / 2.9, 500k mixed 3-D on 1 K=8 28.3 /
-  // 20.0.  A grid falls back to fewer dims where its cells outgrow the points.  The no-allocation
+  // Up to 6 dims, as a join that indexes them all (ms per join, K=16, the indexed dims' grid /
+  // one over all dims): 500k points learned, skewed 6-D on 4 18.6 / 11.9, uniform 14.7 / 5.7,
+  // uniform 4-D on 2 8.6 / 2.0; plain, uniform 6-D on 4 6.9 / 4.1, on 2 29.5 / 4.2, skewed 4-D on 2
+  // 13.7 / 6.3, uniform 3-D on 1 2.7 / 1.5.  In 6-D small sets lose by it, skewed ones up to 100k
+  // points and uniform ones up to 20k: learned skewed on 4 50k 2.3 / 2.9, 100k 4.05 / 4.6, 200k 7.1 /
+  // 6.6; plain 20k 3.06 / 3.53, 100k 6.9 / 5.9; uniform learned 50k 1.7 / 1.3, plain 20k 1.10 / 1.25.
+  // No line by N parts them (where it lies depends on the data), and up to 5 dims none loses over 5 %.
+  // A grid falls back to fewer dims where its cells outgrow the points.  The no-allocation
   // scratch and the hybrid split keep the indexed dims' grid.  KNN_GRID_DIMS=0..6 overrides the 6.
   static bool indexed_dims_only() {
     const char *v = std::getenv("KNN_SLAB");
@@ -457,16 +452,38 @@ struct Pipeline {
     const uint32_t top = ev ? (uint32_t)std::atoi(ev) : 6u;
     return g_arena || !moreDims || indexed_dims_only() ? nd : std::max(nd, std::min(d, std::min(top, 6u)));
   }
-  bool grid_fits(const T *mn, const T *mx, uint32_t gd, T w, uint64_t cells) const {
+  // cells of the grid of width w over the first gd dims, 2^64 - 1 when there is no such grid
+  uint64_t grid_cells(const T *mn, const T *mx, uint32_t gd, T w) const {
     typename GridOf<T>::type gt;
     uint64_t tc = 0;
     try {
-      if (!(w > (T)0)) return false;
+      if (!(w > (T)0)) return ~0ull;
       grid_dims<T>(mn, mx, gd, w, gt, tc);
     } catch (const Error &) {
-      return false;
+      return ~0ull;
     }
-    return tc <= cells;
+    return tc;
+  }
+  bool grid_fits(const T *mn, const T *mx, uint32_t gd, T w, uint64_t cells) const {
+    return grid_cells(mn, mx, gd, w) <= cells;
+  }
+  // whether a grid of so many cells gets a dense start table; with the no-allocation scratch only
+  // when the table and its scan scratch fit beside what is not laid out yet of the index's buffers
+  // and of the 48 bytes per point that the passes may take (active list, tiles, flags, ...): a table
+  // that fitted once fits again at a later, coarser build
+  bool dense_fits(uint64_t cells) const {
+    if (cells >= kDenseMaxCells) return false;
+    if (!g_arena) return true;
+    const size_t u32s = 4 * ((size_t)n + 1);
+    size_t more = g_arena->extra(S_DENSE, 4 * ((size_t)cells + 1)) +
+                  g_arena->extra(S_SCRATCH, (scan_scratch_words((uint32_t)cells + 1) + 1024) * 4) +
+                  g_arena->extra(S_CELLKEYS, 8ull * n) + g_arena->extra(S_XS, sizeof(T) * n * d);
+    for (Slot sl : {S_SIDS, S_IDS_TMP, S_KEYS, S_KEYS_TMP, S_CELLOF}) more += g_arena->extra(sl, 4ull * n);
+    for (Slot sl : {S_FLAGS, S_POS, S_CELLSTART}) more += g_arena->extra(sl, u32s);
+    size_t pass = 48ull * n;
+    for (Slot sl : {S_ACT, S_CELLMAX, S_ABITS, S_OVERFLOW, S_NTILES, S_TILEOFF, S_TILES, S_BLIST})
+      pass -= std::min(pass, g_arena->held(sl));
+    return more + pass + (64u << 10) <= g_arena->room();
   }
   const uint32_t *ncellDev = nullptr;  // device copy of ncell (the scan total of the build)
   Slot xsSlot = S_XS;                   // the slot holding the current cell-sorted copy
@@ -1333,8 +1350,9 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
     const bool split = prm.hybrid_threads && curW == (T)0;
     const double pdiv = split ? 1.0 : plain_grid_div(d, gd, K1);
     T w = (T)((double)e / pdiv);
-    // a finer grid only while its dense start table stays small beside the points
-    if (pdiv > 1.0 && !P.grid_fits(hmn, hmx, gd, w, small)) w = e;
+    // a finer grid only while its dense start table stays small beside the points and fits
+    const uint64_t fineCells = pdiv > 1.0 ? P.grid_cells(hmn, hmx, gd, w) : 0;
+    if (fineCells > small || !P.dense_fits(fineCells)) w = e;
     P.tBuild = &tPh;
     tPh.start();
     P.build_index(hmn, hmx, gd, w);
@@ -1437,6 +1455,11 @@ static void run_plain(Pipeline<T> &P, const knnjoin_params &prm, double beta, kn
 //   2-D  K=64 10M mixed:  R/3, 8 16.3;  R/4, 8 16.1;  R/3, 10 14.3;  R/4, 10 14.8;  R/5, 10 14.6
 //        K=16 10M mixed:  R/3, 8 12.0;  R/3, 10 12.0;  R/5, 10 12.4;  R/4, 8 17.6
 //        K=100 1.3M / K=128 3M mixed:  R/4, 10 6.03 / 9.89;  R/5, 10 5.81 / 8.95;  R/4, 12 6.57 / 10.1
+//        R/3 / R/4 / R/5, 10 bins:  10M mixed K=39 12.7 / 12.0 / 12.6, K=48 13.1 / 13.3 / 13.1, K=64
+//        14.1 / 14.4 / 14.2;  3M mixed K=32 4.6 / 4.5 / 4.9, K=48 5.2 / 4.9 / 4.9, K=64 6.0 / 5.6 / 5.4;
+//        3M uniform K=32 3.25 / 3.23 / 3.12, K=64 4.0 / 3.8 / 3.7;  100k mixed K=32 1.39 / 1.42 / 1.42,
+//        K=64 2.22 / 2.26 / 2.22:  the finer cells gain from K+1 = 40 to 50 on, at K=64 most of all
+//        below 10M points
 //   4-D  5M skewed K=32 / 3M uniform K=16 / 1M on 2 indexed dims, skewed K=32, with failures
 //        growing x2^(1/4):  R/1.5, 5 21.6 / 8.7 / 9.5;  x2^(1/2):  R/1.5, 5 19.2 / 7.9 / 7.6;
 //        R/1.75, 6 19.3 / 8.0 / 7.6;  R/2, 8 18.4 / 8.3 / 9.0
@@ -2507,8 +2530,9 @@ static std::vector<uint32_t> batch_routes(const BatchPlan &B) {
   return r;
 }
 
-// Index of a group at the sets' current widths (classes: those of their lowest pending radius class): per-set grids, cell keys, radix sort, cell
-// table, cell-sorted coordinates, dense cell-start table.
+// Index of a group at the sets' current widths (classes: those of their lowest pending radius
+// class): per-set grids, cell keys, radix sort, cell table, cell-sorted coordinates, dense cell-start
+// table.
 static void batch_index(BatchGroup &G, bool classes, hipStream_t s) {
   const uint32_t N = G.N;
   batch_grids(G.sets, G.nsets, G.mnmx, G.width, G.bound, G.status, classes ? G.setMinBin : nullptr, G.setClass, s);

@@ -92,3 +92,18 @@ def test_noalloc_rejects_inputs_beyond_its_scratch():
     rc = _lib.lib().knnjoin_ex_noalloc(_lib.p(small), _lib.KNN_FLOAT32, 5000, 2, 8, ctypes.byref(prm),
                                        _lib.p(ids), _lib.p(d), None)
     assert rc == _lib.KNN_ERR_ARG
+
+
+@pytest.mark.parametrize("n,k,same_grids", [(1_600_000, 12, True), (1_700_000, 16, True), (1_800_000, 16, False)])
+def test_noalloc_keeps_the_dense_cell_table(n, k, same_grids):
+    # near the scratch's limit the plain schedule's grids must leave room for their dense start table,
+    # at the first build and at the later ones: without it no query is ruled out by its block's count,
+    # and its candidates are read in vain.  (At the third size the first grid has wider cells.)
+    pts = synthetic.mixed_box(n, seed=n + k)
+    rc0, i0, d0, s0 = _join("knnjoin_ex", pts, k, _lib.KNN_MODE_BETA)
+    rc1, i1, d1, s1 = _join("knnjoin_ex_noalloc", pts, k, _lib.KNN_MODE_BETA)
+    assert rc0 == 0 and rc1 == 0, _lib.lib().knnjoin_last_error()
+    assert np.array_equal(i0, i1) and np.array_equal(d0.view(np.uint32), d1.view(np.uint32))
+    assert s0.iterations == s1.iterations
+    if same_grids:
+        assert s0.candidates == s1.candidates
