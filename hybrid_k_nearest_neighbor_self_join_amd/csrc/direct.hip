@@ -207,9 +207,11 @@ __global__ __launch_bounds__(64, waves_per_simd(H)) void k_direct(JoinArgs a, G 
   uint32_t Q;
   const uint32_t NT = work_count(a, TAB ? 1u : 4u, ND >= 1 && ND <= 4, Q);
   WaveTally tally;
+  bool first = true;
   for (;;) {
-    const uint32_t t = next_tile(a.tileCounter, NT, a.tileRanges, lane);
+    const uint32_t t = next_tile(a.tileCounter, NT, a.tileRanges, lane, first);
     if (t >= NT) break;
+    first = false;
     const uint2 tl = work_tile(a, t, Q);
     const uint32_t nq = tl.y;
     const uint32_t qL = tile_query(a, tl, lane < nq ? lane : 0u);

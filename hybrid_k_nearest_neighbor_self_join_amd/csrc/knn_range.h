@@ -305,27 +305,40 @@ __device__ __forceinline__ bool row_chord_lane(const G &g, const uint32_t *cur, 
 // and, once that is empty, from the other ranges in turn.  Wave-uniform.
 static_assert(TILE_QUEUES == 8, "tile ranges are split by a shift of 3");
 // Next tile index of the workgroup, NT when every range is empty.  ranges: 1 or TILE_QUEUES.
-// No state is kept between calls: a workgroup whose own range is empty reads the other heads at
-// once (lane = range; a head only grows, so an old value costs a failing atomic and loses no tile)
-// and goes to the next one that still shows tiles.  A failing atomic on every head instead cost
-// each pass of a join about 0.3 ms, whatever its queries: 4096 waves times eight atomics on eight
-// words (ms per join, plain: 20k skewed 3-D points on 2 dims K=1, 23 passes, 11.6 / 4.5, 500k
-// skewed 4-D K=16 13.5 / 7.3, 2M uniform 6-D K=32 23.4 / 22.6).  One loop for all of it: a separate
+// A workgroup's first tile (`first`) is its own by its index within the range, and the heads count
+// the tiles after those: atomics on one word come back at a few per ns, so that a pass of as many
+// tiles as workgroups (or fewer) spent 30 us and more on 4096 first and 4096 failing additions,
+// whatever its queries, more than the 2816 waves of the kernel before it.  ms per join with a
+// first tile from the queue / so: 100k uniform 2-D K=8 plain 0.78 / 0.69, 100k mixed K=16 plain 2.93 /
+// 2.42, 20k skewed 3-D on 2 dims K=1 4.6 / 3.1, 500k skewed 4-D K=16 plain 6.2 / 4.9, 10M mixed 2-D K=64
+// learned 14.17 / 14.01, plain 19.1 / 18.5; 4249 passes over 100k points of a power law, K=64,
+// range kernel 486 / 304 (the kernel before: 339).
+// Otherwise no state is kept between calls: a workgroup whose own range is empty reads the other
+// heads at once (lane = range; a head only grows, so an old value costs a failing atomic and loses no
+// tile) and goes to the next one that still shows tiles: eight failing atomics per wave had cost each
+// pass about 0.3 ms (500k skewed 4-D K=16 plain 13.5 / 7.3).  One loop for all of it: a separate
 // first attempt spills 8 more registers of the 2-D kernel.
-__device__ __forceinline__ uint32_t next_tile(uint32_t *heads, uint32_t NT, uint32_t ranges, uint32_t lane) {
+__device__ __forceinline__ uint32_t next_tile(uint32_t *heads, uint32_t NT, uint32_t ranges, uint32_t lane,
+                                              bool first) {
   const uint32_t sh = ranges == TILE_QUEUES ? 3u : 0u;
   const uint32_t mask = (1u << sh) - 1u;
   auto begin = [&](uint32_t r) { return (uint32_t)(((uint64_t)NT * r) >> sh); };
+  auto share = [&](uint32_t r) { return (gridDim.x + mask - r) >> sh; };  // workgroups of range r
   uint32_t j = 0;  // ranges tried or seen empty
   for (;;) {
     const uint32_t r = (blockIdx.x + j) & mask, b = begin(r), e = begin(r + 1);
-    uint32_t t = 0;
-    if (lane == 0) t = atomicAdd(&heads[r], 1u);
-    t = (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
+    const uint32_t s = share(r);
+    uint32_t t = blockIdx.x >> sh;
+    if (!first) {
+      t = 0;
+      if (lane == 0 && s < e - b) t = atomicAdd(&heads[r], 1u);
+      t = s + (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
+    }
     if (t < e - b) return b + t;
-    const uint32_t q = (blockIdx.x + lane) & mask;
-    bool left = lane > j && lane <= mask;
-    if (left) left = __hip_atomic_load(&heads[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < begin(q + 1) - begin(q);
+    first = false;
+    const uint32_t q = (blockIdx.x + lane) & mask, sq = share(q), nq = begin(q + 1) - begin(q);
+    bool left = lane > j && lane <= mask && sq < nq;
+    if (left) left = sq + __hip_atomic_load(&heads[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < nq;
     const uint64_t m = __builtin_amdgcn_ballot_w64(left);
     if (!m) return NT;
     j = (uint32_t)__builtin_ctzll(m);

@@ -40,9 +40,11 @@ __global__ __launch_bounds__(64) void k_range_collect(JoinArgs a, G g0) {
   const uint32_t NT = work_count(a, 4u, false, Q);
   constexpr int PR = D <= 8 ? 4 : 2;
   WaveTally tally;
+  bool first = true;
   for (;;) {
-    const uint32_t t = next_tile(a.tileCounter, NT, a.tileRanges, lane);
+    const uint32_t t = next_tile(a.tileCounter, NT, a.tileRanges, lane, first);
     if (t >= NT) break;
+    first = false;
     const uint2 tl = work_tile(a, t, Q);
     const TileCtx<G> C = tile_ctx<G>(a, g0, tl);
     const G &g = C.g;
@@ -234,9 +236,11 @@ __global__ __launch_bounds__(64) void k_range_heap(JoinArgs a, G g0) {
   const uint32_t NT = tile_count(a);
 
   WaveTally tally;
+  bool first = true;
   for (;;) {
-    const uint32_t t = next_tile(a.tileCounter, NT, a.tileRanges, lane);
+    const uint32_t t = next_tile(a.tileCounter, NT, a.tileRanges, lane, first);
     if (t >= NT) break;
+    first = false;
     const uint2 tl = a.tiles[t];
     const TileCtx<G> C = tile_ctx<G>(a, g0, tl);
     const G &g = C.g;

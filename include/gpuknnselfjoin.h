@@ -267,7 +267,8 @@ typedef struct {
 } knnjoin_batch_params;
 
 typedef struct {
-  double ms_device;          /* time of the join's passes on the device, HIP events */
+  double ms_device;          /* span of the join's passes, from the first launch to the last wait (the
+                                groups run on streams of their own, the host waits between passes) */
   double ms_setup;           /* host time before the launch: plan build, capture, input copies */
   uint32_t groups;           /* distinct dimensionalities */
   uint32_t graph_replayed;   /* 1 = existing graphs were replayed */

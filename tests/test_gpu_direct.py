@@ -142,3 +142,26 @@ def test_rows_looked_up_together(oracle, monkeypatch, div):
     monkeypatch.setenv("KNN_TILE_ROWS", "1")
     st.append(_check(oracle, pts, 20, beta=0.025))
     assert st[0].candidates == st[1].candidates and st[0].iterations == st[1].iterations
+
+
+@pytest.mark.parametrize("ranges", ["1", "8"])
+@pytest.mark.parametrize("grid", [1, 5, 9, 100, 4096])
+def test_first_tiles(monkeypatch, ranges, grid):
+    # every workgroup has a first tile of its own and takes the rest from the queues: fewer workgroups
+    # than ranges, uneven shares of them, more workgroups than tiles
+    monkeypatch.setenv("KNN_TILE_RANGES", ranges)
+    sets = [synthetic.skewed_cube(n, d, seed=n) for n, d in ((3, 2), (700, 2), (1, 3), (2500, 3), (65, 6))]
+    ks = [2, 9, 0, 12, 5]
+    for kern in ("direct", "collect"):
+        monkeypatch.setenv("KNN_RANGE_KERNEL", kern)
+        ids, dists, st = batched.knnjoin_batched(sets, ks, grid_blocks=grid, tile_queries=16)
+        for p, k, i, d in zip(sets, ks, ids, dists):
+            ri, rd, _ = _lib.knnjoin_ex(p, k, brute_fallback=0)
+            assert np.array_equal(i, ri) and np.array_equal(d.view(np.uint32), rd.view(np.uint32))
+
+
+@pytest.mark.parametrize("ranges", ["1", "8"])
+@pytest.mark.parametrize("n", [2101, 3000])
+def test_first_tiles_of_the_heap_kernel(oracle, monkeypatch, ranges, n):
+    monkeypatch.setenv("KNN_TILE_RANGES", ranges)
+    _check(oracle, synthetic.skewed_cube(n, 3, seed=n), 2100, beta=0.05)
