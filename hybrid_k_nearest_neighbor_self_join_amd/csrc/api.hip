@@ -698,11 +698,11 @@ static uint32_t feature_reps(uint64_t cells) {
 
 // Tile ranges of a range-kernel launch: one per XCD for single sets of 3 or more data dims,
 // one queue for 2-D sets and batched groups.  Measured on one MI355X, each pair in one process
-// (ms per join, one queue against one range per XCD): 10M mixed 2-D points K=64, plain 35.0 /
-// 35.9, learned 21.3 / 21.5; 5M points, K=32, plain unless marked: 4-D uniform 26.7 / 25.9,
-// skewed 49.3 / 52.2; 4-D on 2 indexed dims uniform 92.1 / 79.8, skewed (learned) 189 / 187;
-// 6-D on 4 indexed dims uniform 233 / 221, skewed (learned) 532 / 552; 6-D (collect kernel)
-// uniform 132 / 106, skewed 189 / 177; the 256-set batched join 144 / 164.
+// (ms per join, one queue against one range per XCD): 10M mixed 2-D points K=64, plain 18.5 /
+// 19.1, learned 13.9 / 14.3; 3M uniform 3-D K=16 plain 4.31 / 4.33; K=32, 5M 4-D uniform plain 13.7 /
+// 11.8, skewed learned 22.6 / 17.2 (100k skewed K=16 plain 3.5 / 3.8); 2M 6-D uniform plain 35.2 / 22.3,
+// skewed learned 41.7 / 30.8; 1M skewed 6-D on 4 indexed dims learned 24.0 / 22.3; 300k uniform 8-D K=16
+// plain 18.2 / 18.5; 48 batched sets of 2 to 6 dims 12.2 / 13.7.
 // KNN_TILE_RANGES=1|8 overrides the choice for tuning.
 static uint32_t tile_ranges(uint32_t d, bool batched) {
   const char *v = std::getenv("KNN_TILE_RANGES");  // read per launch: tuning runs switch it in-process

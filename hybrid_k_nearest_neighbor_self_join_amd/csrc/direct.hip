@@ -32,14 +32,15 @@
 // A query whose list does not fit (thousands of equal keys) goes to the overflow kernel
 // (range.hip).
 //
-// What bounds it: VALU issue in 2-D (75 % of the issue slots at 4 waves per SIMD; about 270 vector
-// instructions per query at K = 64, of which the selection is 150).  One query per wave needs no
+// What bounds it: VALU issue in 2-D (72 % of the issue slots at 4 waves per SIMD; about 350 vector
+// instructions per query at K = 64, failed searches included, of which the selection is about 150).  One query per wave needs no
 // tile of queries around a shared union of blocks, so few queries left in a pass still fill the
 // chip, and each candidate is loaded only for queries whose ball may hold it.  Against the kernel
 // before it (a tile-wide histogram pass, then a second pass over each query's sub-block; the
 // collect kernel with 5 or more indexed dims), range-kernel ms per join on one MI355X, same rows:
-// 10M mixed 2-D K=64 learned 11.4 / 8.0, plain 21.6 / 11.4; 5M skewed 4-D K=32 learned 30.4 /
-// 12.5; 2M uniform 6-D K=32 plain 38.9 / 28.5; 1M skewed 6-D on 4 dims K=32 learned 108 / 58.
+// 10M mixed 2-D K=64 learned 11.4 / 7.9, plain 21.5 / 10.9; 5M skewed 4-D K=32 learned 30.1 /
+// 10.8; 2M uniform 6-D K=32 plain 38.7 / 20.4; 1M skewed 6-D on 4 dims K=32 learned 107 / 16.9 (there
+// on a grid over all 6 dims).
 // 128 registers (4 waves per SIMD): 96 (5 waves) spills and loses 25 % in 2-D.
 #include "knn_range.h"
 
@@ -86,7 +87,8 @@ constexpr int waves_per_simd(int h) { return h <= 4 ? 4 : 2; }
 // Windows of 64 candidates that a chunk's row tables cover, and those kept in registers: the last
 // two of the 8 at H = 4 live in LDS (1 KB, within the 10 KB of 16 waves per CU).  All 8 in
 // registers spill 18 of the 128: range-kernel ms, 10M mixed 2-D K=64 learned 8.9 / 8.1 and plain
-// 13.5 / 11.6, 3M K=128 learned 6.8 / 6.4, 3M K=200 plain 9.1 / 8.7.
+// 13.5 / 11.6, 3M mixed K=128 learned 6.8 / 6.4 (6.3 now), 3M uniform K=200 plain 9.1 /
+// 8.7.
 constexpr uint32_t windows(int h) { return h >= 4 ? 8 : 4; }
 constexpr uint32_t reg_windows(int h) { return h == 4 ? 6 : windows(h); }
 // LDS: DR_NB bucket counters and 64 dummies, H * 64 sorted (key, id) slots and four sentinels, a
